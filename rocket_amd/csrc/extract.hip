@@ -192,6 +192,7 @@ __global__ __launch_bounds__(256) void fastnoise_kernel(const uint8_t *in_all, i
         cp[0] = csum[0][tid] + csum[2][tid];
         cp[1] = csum[1][tid] + csum[3][tid];
     }
+    if (!rowpart_all) return;
     // row r, column parity p: four threads (quad c = 0..3) sum 8 columns each
     const int r = tid >> 3, p = (tid >> 2) & 1, c = tid & 3;
     double rs = 0.0;
@@ -207,19 +208,40 @@ __global__ __launch_bounds__(256) void fastnoise_kernel(const uint8_t *in_all, i
 // aligned inputs): lane l of a wave holds the 4 pixels of columns
 // x0 + 4 (l - 1) + [0, 4) of one row, x0 = 248 * segment; lanes 0 and 63 are
 // the halo (their pixels feed lanes 1 and 62 and are not written).  A wave
-// walks down a band of 64 rows keeping three gray rows, one U row and three
-// V rows in registers: at step t it loads gray row t (one 12-byte load per
+// walks down a band of rows keeping three gray rows, two U rows and three
+// V rows in registers: at step t it converts gray row t (one 12-byte load per
 // lane for RGB8), forms U and V of row t - 1 and the output of row t - 2.
 // Horizontal neighbours come from the adjacent lanes through DPP moves, so
 // nothing goes through LDS.  The same arithmetic per pixel as
-// fastnoise_kernel (fastnoisefilter.cu:150-204).  Zero-mean partial sums:
-// per column and row parity over the band (FP64, bands of 64 rows), per row
-// and column parity over each 64-column group of 16 lanes (FP32 sums of the
-// group's 32 pixels of a parity, stored as FP64).
+// fastnoise_kernel (fastnoisefilter.cu:150-204).
+//
+// What bounds it: a step is one row's load latency if the row is asked for
+// when it is needed, and a small image has few waves to hide that behind.  So
+// the bytes of row t + kFnAhead are asked for at step t (the row rings are
+// registers: the loop is unrolled over their common period, so no row is
+// moved), and the band is chosen by the image's size (fn_band).  With one
+// load at a time and 64-row bands one gray 512x512 image took 63 us, 16 RGB8
+// of 1024x1024 92 us and 32 of 2048x1536 197 us; now 12, 40 and 185 us (the
+// last 3.8 TB/s of 22 MB a frame).
+//
+// Zero-mean partial sums: per column and row parity over the band (FP64);
+// per row and column parity over each 64-column group of 16 lanes (FP32 sums
+// of the group's 32 pixels of a parity, stored as FP64) where the caller
+// wants them (rowpart_all non-null).
 // grid (8 * per) x 256 threads: a workgroup = 4 waves = 4 bands of one
 // segment; units (image, segment, band group) are dealt in order to the
 // XCDs as in fastnoise_kernel.
-constexpr int kFnSeg = 248, kFnBand = 64;
+constexpr int kFnSeg = 248, kFnAhead = 3, kFnPeriod = 6;
+
+// Rows of a band: a function of the image alone, so that an image's partial
+// sums (one per band and column) are the same alone and in a batch.  A band
+// reads 4 halo rows: short bands are for images with too few waves without
+// them (512x512: 96 waves at 16 rows), long ones spare halo rows and partial
+// sums where a few frames fill the chip.
+int fn_band(int h, int w) {
+    const int64_t n = (int64_t)h * w;
+    return n <= (int64_t(1) << 19) ? 8 : n <= (int64_t(1) << 21) ? 16 : 32;
+}
 
 __device__ __forceinline__ float dpp_from_left(float v) {   // lane i <- lane i - 1 (0 for lane 0)
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
@@ -236,22 +258,51 @@ __device__ __forceinline__ float dpp_row_sum16(float v) {
     return v;
 }
 
-// Gray values of 4 consecutive pixels starting at pixel `px` (a multiple of
-// 4) of an image at `in`.  8-bit images may start at any byte: the pixels'
-// bytes are read as the aligned dwords that hold them (each holds at least
-// one of the wanted bytes, so no read leaves the pages of the image) and
-// realigned with v_alignbyte; `off` = (address of `in`) & 3, the same for
-// every group since 3 * px and px are multiples of 4.
+// The bytes of 4 consecutive pixels starting at pixel `px` (a multiple of
+// 4) of an image at `in`, and their gray values.  8-bit images may start at
+// any byte: the pixels' bytes are read as the aligned dwords that hold them
+// (each holds at least one of the wanted bytes, so no read leaves the pages
+// of the image) and realigned with v_alignbyte; `off` = (address of `in`) & 3,
+// the same for every group since 3 * px and px are multiples of 4.
+struct Raw4 {
+    uint32_t d[4];
+};
+
 template <int FMT>
-__device__ __forceinline__ void gray4(const uint8_t *in, int64_t px, int off, float g[4]) {
+__device__ __forceinline__ Raw4 raw4(const uint8_t *in, int64_t px, int off) {
+    Raw4 r = {};
     if constexpr (FMT == PRNU_INPUT_RGB8) {
+        typedef uint32_t u3a4 __attribute__((ext_vector_type(3), aligned(4)));
         const uint32_t *q = reinterpret_cast<const uint32_t *>(in + 3 * px - off);
-        uint32_t a = q[0], b = q[1], c = q[2];
+        const u3a4 v = *reinterpret_cast<const u3a4 *>(q);
+        r.d[0] = v.x;
+        r.d[1] = v.y;
+        r.d[2] = v.z;
+        if (off) r.d[3] = q[3];
+    } else if constexpr (FMT == PRNU_INPUT_GRAY8) {
+        const uint32_t *q = reinterpret_cast<const uint32_t *>(in + px - off);
+        r.d[0] = q[0];
+        if (off) r.d[1] = q[1];
+    } else {
+        // FP32 images are 4-byte aligned; a 16-byte load needs no more
+        typedef uint32_t u4a4 __attribute__((ext_vector_type(4), aligned(4)));
+        const u4a4 v = *reinterpret_cast<const u4a4 *>(reinterpret_cast<const float *>(in) + px);
+        r.d[0] = v.x;
+        r.d[1] = v.y;
+        r.d[2] = v.z;
+        r.d[3] = v.w;
+    }
+    return r;
+}
+
+template <int FMT>
+__device__ __forceinline__ void gray4(const Raw4 &r, int off, float g[4]) {
+    if constexpr (FMT == PRNU_INPUT_RGB8) {
+        uint32_t a = r.d[0], b = r.d[1], c = r.d[2];
         if (off) {
-            const uint32_t d = q[3];
             a = __builtin_amdgcn_alignbyte(b, a, off);
             b = __builtin_amdgcn_alignbyte(c, b, off);
-            c = __builtin_amdgcn_alignbyte(d, c, off);
+            c = __builtin_amdgcn_alignbyte(r.d[3], c, off);
         }
         const uint32_t by[12] = {a & 0xff, (a >> 8) & 0xff, (a >> 16) & 0xff, a >> 24,
                                  b & 0xff, (b >> 8) & 0xff, (b >> 16) & 0xff, b >> 24,
@@ -260,40 +311,35 @@ __device__ __forceinline__ void gray4(const uint8_t *in, int64_t px, int off, fl
         for (int k = 0; k < 4; ++k)
             g[k] = kWR * (float)by[3 * k + 2] + kWG * (float)by[3 * k + 1] + kWB * (float)by[3 * k];
     } else if constexpr (FMT == PRNU_INPUT_GRAY8) {
-        const uint32_t *q = reinterpret_cast<const uint32_t *>(in + px - off);
-        uint32_t a = q[0];
-        if (off) a = __builtin_amdgcn_alignbyte(q[1], a, off);
+        uint32_t a = r.d[0];
+        if (off) a = __builtin_amdgcn_alignbyte(r.d[1], a, off);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const float v = (float)((a >> (8 * k)) & 0xff);
             g[k] = kWR * v + kWG * v + kWB * v;
         }
     } else {
-        // FP32 images are 4-byte aligned; a 16-byte load needs no more
-        typedef float f4a4 __attribute__((ext_vector_type(4), aligned(4)));
-        const f4a4 v = *reinterpret_cast<const f4a4 *>(reinterpret_cast<const float *>(in) + px);
-        g[0] = v.x;
-        g[1] = v.y;
-        g[2] = v.z;
-        g[3] = v.w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) g[k] = __builtin_bit_cast(float, r.d[k]);
     }
 }
 
 template <int FMT>
 __global__ __launch_bounds__(256) void fastnoise_rows_kernel(const uint8_t *in_all, int64_t in_stride, float *out_all,
-                                                             int64_t out_stride, int h, int w, double *colpart_all,
-                                                             int64_t cp_stride, double *rowpart_all, int64_t rp_stride,
-                                                             int nseg, int ngrp, int nunits) {
+                                                             int64_t out_stride, int h, int w, int band_rows,
+                                                             double *colpart_all, int64_t cp_stride,
+                                                             double *rowpart_all, int64_t rp_stride, int nseg, int ngrp,
+                                                             int nunits) {
     const int per = (nunits + 7) / 8;
     const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (t >= nunits) return;
     const int bz = t / (nseg * ngrp), rem = t - bz * (nseg * ngrp);
     const int seg = rem / ngrp, grp = rem - (rem / ngrp) * ngrp;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int band = grp * 4 + wave;
-    const int y0 = band * kFnBand;
+    const int y0 = band * band_rows;  // even
     if (y0 >= h) return;  // no barriers in this kernel: a wave may leave alone
-    const int y1 = min(h, y0 + kFnBand);
+    const int y1 = min(h, y0 + band_rows);
     const uint8_t *in = in_all + (int64_t)bz * in_stride;
     const int off = FMT == PRNU_INPUT_FLOAT32 ? 0 : (int)(reinterpret_cast<uintptr_t>(in) & 3);
     float *out = out_all + (int64_t)bz * out_stride;
@@ -301,14 +347,18 @@ __global__ __launch_bounds__(256) void fastnoise_rows_kernel(const uint8_t *in_a
     const bool inx = xl >= 0 && xl < w;             // all 4 pixels (w is a multiple of 4)
     const bool own = inx && lane >= 1 && lane <= 62;
     const bool first_col = xl == 0, last_col = xl + 4 == w;
-    const bool zm = colpart_all != nullptr;
+    const bool zm = colpart_all != nullptr, zmr = rowpart_all != nullptr;
+    const int xc = min(max(xl, 0), w - 4);  // lanes outside the image load a column of it and use zeros
 
-    // gray rows t-2, t-1, t; U row t-2 (output row) and t-1; V rows t-3 .. t-1
-    float G0[4] = {}, G1[4] = {}, G2[4] = {};
-    float Ua[4] = {}, Ub[4] = {};
-    float V0[4] = {}, V1[4] = {}, V2[4] = {};
+    // rings over rows: bytes on their way, gray, U, V (indexes are constants
+    // after the unrolling below)
+    Raw4 raw[kFnAhead];
+    float G[3][4] = {}, U[2][4] = {}, V[3][4] = {};
     double ce[4] = {}, co[4] = {};  // column sums of even / odd rows
 
+    auto load = [&](int r) {  // a row outside the image: one inside it, used as zeros
+        return raw4<FMT>(in, (int64_t)min(max(r, 0), h - 1) * w + xc, off);
+    };
     auto dx4 = [&](const float g[4], float d[4]) {
         const float left = dpp_from_left(g[3]), right = dpp_from_right(g[0]);
         d[0] = first_col ? g[1] - g[0] : 0.5f * (g[1] - left);
@@ -316,67 +366,70 @@ __global__ __launch_bounds__(256) void fastnoise_rows_kernel(const uint8_t *in_a
         d[2] = 0.5f * (g[3] - g[1]);
         d[3] = last_col ? g[3] - g[2] : 0.5f * (right - g[2]);
     };
-    for (int r = y0 - 2; r <= y1 + 1; ++r) {
-        // shift the windows by one row
+    const int steps = y1 - y0 + 4;  // gray rows y0 - 2 .. y1 + 1
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            G0[k] = G1[k];
-            G1[k] = G2[k];
-            V0[k] = V1[k];
-            V1[k] = V2[k];
-            Ua[k] = Ub[k];
-        }
-        // gray row r
-        if (inx && r >= 0 && r < h) {
-            gray4<FMT>(in, (int64_t)r * w + xl, off, G2);
-        } else {
+    for (int k = 0; k < kFnAhead; ++k) raw[k] = load(y0 - 2 + k);
+    for (int s = 0; s < steps; s += kFnPeriod) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) G2[k] = 0.f;
-        }
-        // U, V of row r - 1 from gray rows r - 2, r - 1, r
-        // (every lane runs the DPP moves; lanes outside the image keep zeros)
-        const int ru = r - 1;
-        if (ru >= y0 - 1) {
-            const bool valid = inx && ru >= 0 && ru < h;
-            float dx[4];
-            dx4(G1, dx);
+        for (int k = 0; k < kFnPeriod; ++k) {
+            if (s + k >= steps) break;
+            const int r = y0 - 2 + s + k;
+            float(&G2)[4] = G[k % 3], (&G1)[4] = G[(k + 2) % 3], (&G0)[4] = G[(k + 1) % 3];
+            float(&V2)[4] = V[k % 3], (&V1)[4] = V[(k + 2) % 3], (&V0)[4] = V[(k + 1) % 3];
+            float(&Ub)[4] = U[k % 2], (&Ua)[4] = U[(k + 1) % 2];
+            // gray row r
+            const bool rin = inx && r >= 0 && r < h;
+            gray4<FMT>(raw[k % kFnAhead], off, G2);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const float dy = ru == 0 ? G2[k] - G1[k] : ru == h - 1 ? G1[k] - G0[k] : 0.5f * (G2[k] - G0[k]);
-                const float norm = __builtin_amdgcn_sqrtf(dx[k] * dx[k] + dy * dy);
-                const float scale = __builtin_amdgcn_rcpf(1.0f + norm);
-                Ub[k] = valid ? scale * dx[k] : 0.f;
-                V2[k] = valid ? scale * dy : 0.f;
-            }
-        }
-        // output row r - 2 from U row r - 2 and V rows r - 3 .. r - 1
-        const int ro = r - 2;
-        if (ro >= y0) {
-            float a[4];
-            dx4(Ua, a);  // the same one-sided / central rule on U
-            float o[4];
+            for (int e = 0; e < 4; ++e) G2[e] = rin ? G2[e] : 0.f;
+            if (s + k + kFnAhead < steps) raw[k % kFnAhead] = load(r + kFnAhead);
+            // U, V of row r - 1 from gray rows r - 2, r - 1, r
+            // (every lane runs the DPP moves; lanes outside the image keep zeros)
+            const int ru = r - 1;
+            if (ru >= y0 - 1) {
+                const bool valid = inx && ru >= 0 && ru < h;
+                float dx[4];
+                dx4(G1, dx);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const float b = ro == 0 ? V2[k] - V1[k] : ro == h - 1 ? V1[k] - V0[k] : 0.5f * (V2[k] - V0[k]);
-                o[k] = own ? a[k] + b : 0.f;
-            }
-            if (own) *reinterpret_cast<float4 *>(out + (int64_t)ro * w + xl) = make_float4(o[0], o[1], o[2], o[3]);
-            if (zm) {
-                if (ro & 1) {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) co[k] += (double)o[k];
-                } else {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) ce[k] += (double)o[k];
+                for (int e = 0; e < 4; ++e) {
+                    const float dy = ru == 0 ? G2[e] - G1[e] : ru == h - 1 ? G1[e] - G0[e] : 0.5f * (G2[e] - G0[e]);
+                    const float norm = __builtin_amdgcn_sqrtf(dx[e] * dx[e] + dy * dy);
+                    const float scale = __builtin_amdgcn_rcpf(1.0f + norm);
+                    Ub[e] = valid ? scale * dx[e] : 0.f;
+                    V2[e] = valid ? scale * dy : 0.f;
                 }
-                // columns xl + k have parity k & 1 (xl is a multiple of 4)
-                const float se = dpp_row_sum16(o[0] + o[2]);
-                const float so = dpp_row_sum16(o[1] + o[3]);
-                if ((lane & 15) == 15) {
-                    double *rp = rowpart_all + (int64_t)bz * rp_stride +
-                                 ((int64_t)(seg * 4 + (lane >> 4)) * h + ro) * 2;
-                    rp[0] = (double)se;
-                    rp[1] = (double)so;
+            }
+            // output row r - 2 from U row r - 2 and V rows r - 3 .. r - 1
+            const int ro = r - 2;
+            if (ro >= y0) {
+                float a[4];
+                dx4(Ua, a);  // the same one-sided / central rule on U
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float b = ro == 0 ? V2[e] - V1[e] : ro == h - 1 ? V1[e] - V0[e] : 0.5f * (V2[e] - V0[e]);
+                    o[e] = own ? a[e] + b : 0.f;
+                }
+                if (own) *reinterpret_cast<float4 *>(out + (int64_t)ro * w + xl) = make_float4(o[0], o[1], o[2], o[3]);
+                if (zm) {
+                    if (k & 1) {  // ro has the parity of k: y0 and s are even
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) co[e] += (double)o[e];
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) ce[e] += (double)o[e];
+                    }
+                }
+                if (zmr) {
+                    // columns xl + e have parity e & 1 (xl is a multiple of 4)
+                    const float se = dpp_row_sum16(o[0] + o[2]);
+                    const float so = dpp_row_sum16(o[1] + o[3]);
+                    if ((lane & 15) == 15) {
+                        double *rp = rowpart_all + (int64_t)bz * rp_stride +
+                                     ((int64_t)(seg * 4 + (lane >> 4)) * h + ro) * 2;
+                        rp[0] = (double)se;
+                        rp[1] = (double)so;
+                    }
                 }
             }
         }
@@ -395,7 +448,7 @@ __global__ __launch_bounds__(256) void fastnoise_rows_kernel(const uint8_t *in_a
 // row of column sums per tile row, rowpart one column of row sums per tile
 // column.
 constexpr int kZmTileRows = kFnTY, kZmTileCols = kFnTX;             // fastnoise_kernel, zm_partials_kernel
-int zm_tiles_y_rows(int h) { return (h + kFnBand - 1) / kFnBand; }  // fastnoise_rows_kernel
+int zm_tiles_y_rows(int h, int w) { return (h + fn_band(h, w) - 1) / fn_band(h, w); }  // fastnoise_rows_kernel
 int zm_tiles_x_rows(int w) { return 4 * ((w + kFnSeg - 1) / kFnSeg); }
 
 // -------------------------------------------------------------- zero-mean
@@ -491,6 +544,39 @@ __global__ __launch_bounds__(256) void zm_lattice_kernel(double *colsum_all, int
     }
 }
 
+// Column means alone, cz[pi][x] = colsum[pi][x] / rows of parity pi (FP32),
+// for the Wiener rows of even widths, which need no row means
+// (wiener_rows_fwd_kernel).  Thread (g, c) of a 4 x 64 block sums tiles g,
+// g + 4, ... of column c, the four sums are added in order.  (With the row
+// means and the sub-lattice means the general form takes two kernels: 40 us
+// for 32 frames of 2048x1536 against 11.)
+// grid (ceil(w/64), B)
+__global__ __launch_bounds__(256) void zm_colmean_kernel(const double *colpart_all, int64_t cp_stride, int h, int w,
+                                                         int tiles_y, float *cz_all) {
+    __shared__ double2 sh[4][64];
+    const double2 *cp = reinterpret_cast<const double2 *>(colpart_all + (int64_t)blockIdx.y * cp_stride);
+    const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int x = blockIdx.x * 64 + c;
+    double2 s = make_double2(0.0, 0.0);
+    if (x < w) {
+#pragma unroll 4
+        for (int t = g; t < tiles_y; t += 4) {
+            const double2 v = cp[(int64_t)t * w + x];
+            s.x += v.x;
+            s.y += v.y;
+        }
+    }
+    sh[g][c] = s;
+    __syncthreads();
+    if (g == 0 && x < w) {
+        const double se = (sh[0][c].x + sh[1][c].x) + (sh[2][c].x + sh[3][c].x);
+        const double so = (sh[0][c].y + sh[1][c].y) + (sh[2][c].y + sh[3][c].y);
+        float *cz = cz_all + (int64_t)blockIdx.y * 2 * w;
+        cz[x] = (float)(se / (double)((h + 1) >> 1));
+        cz[w + x] = (float)(so / (double)(h >> 1));
+    }
+}
+
 // out = x - colmean[pi][x] - rowmean[pj][y] + g[pi][pj]: columns-then-rows
 // zero-mean of zeromeantotalfilter.cu in closed form.
 __device__ __forceinline__ float zm_value(float x, int y, int xx, int h, int w, const double *colmean,
@@ -527,11 +613,21 @@ __global__ __launch_bounds__(256) void zm_apply_kernel(float *img_all, int64_t i
 // Rows 2r and 2r+1 of image b: (optional zero-mean) -> sums of squares
 // (FP64) -> forward FFT (w) -> half spectra into A (h x (w/2+1)).
 // grid (ceil(h/2), B).
-// Zero-mean (cz non-null): x - cz[row parity][j] - rz[j & 1][row] in FP32,
-// the column terms cz = colmean - g and row means rz of zm_lattice_kernel /
-// zm_reduce_kernel (within an ulp of the FP64 closed form zm_value).
+// Zero-mean, odd widths (cz and rz non-null): x - cz[row parity][j] -
+// rz[j & 1][row] in FP32, the column terms cz = colmean - g and row means rz
+// of zm_lattice_kernel / zm_reduce_kernel (within an ulp of the FP64 closed
+// form zm_value).
+// ZM_EVEN (even widths): x - cz[row parity][j] with the column means alone.
+// What the row means and g would still take away is one constant on the
+// row's even columns and one on its odd columns, which lie in bins 0 and w/2
+// alone; the zero-mean row has no even-column sum and no odd-column sum, so
+// both bins are zero: they are written as zeros, and the row's sum of squares
+// loses Se^2 / (w/2) + So^2 / (w/2), Se and So the row's even- and odd-column
+// sums from the same two bins.  No row sums are taken before the transform
+// (32 frames of 2048x1536: 304 -> 275 us, two loads and two subtractions less
+// per value pair).
 // PAD2048: rows of 2048 by fft_block_2048_r8 (LDS kFft2048PadLds values).
-template <int MAXN, bool PAD2048 = false>
+template <int MAXN, bool PAD2048 = false, bool ZM_EVEN = false>
 __global__ __launch_bounds__(kFftThreads) void wiener_rows_fwd_kernel(FftDesc d, const float *img_all,
                                                                       int64_t img_stride, int h, float2 *A_all,
                                                                       int64_t plane, double *rowsq_all,
@@ -543,19 +639,22 @@ __global__ __launch_bounds__(kFftThreads) void wiener_rows_fwd_kernel(FftDesc d,
     const bool two = i1 < h;
     const int w = d.n, wh = w / 2 + 1;
     const float *img = img_all + (int64_t)b * img_stride;
-    const bool zm = cz_all != nullptr;
+    const bool zm = ZM_EVEN || cz_all != nullptr;
     // rows i0 (even) and i1 (odd): column terms of parities 0 and 1
     const float *cz0 = zm ? cz_all + (int64_t)b * 2 * w : nullptr;
     const float *cz1 = zm ? cz0 + w : nullptr;
-    const float *rz = zm ? rz_all + (int64_t)b * 2 * h : nullptr;
-    const float ra0 = zm ? rz[i0] : 0.f, ra1 = zm ? rz[h + i0] : 0.f;   // row i0, even / odd columns
-    const float rb0 = zm && two ? rz[i1] : 0.f, rb1 = zm && two ? rz[h + i1] : 0.f;
+    const float *rz = !ZM_EVEN && zm ? rz_all + (int64_t)b * 2 * h : nullptr;
+    const float ra0 = rz ? rz[i0] : 0.f, ra1 = rz ? rz[h + i0] : 0.f;   // row i0, even / odd columns
+    const float rb0 = rz && two ? rz[i1] : 0.f, rb1 = rz && two ? rz[h + i1] : 0.f;
     double sq0 = 0.0, sq1 = 0.0;
     const float *r0 = img + (int64_t)i0 * w;
     const float *r1 = img + (int64_t)(two ? i1 : i0) * w;
     auto get = [&](int j) {
             float va = r0[j], vb = two ? r1[j] : 0.f;
-            if (zm) {
+            if (ZM_EVEN) {
+                va -= cz0[j];
+                vb = two ? vb - cz1[j] : 0.f;
+            } else if (zm) {
                 const bool odd = j & 1;
                 va = (va - cz0[j]) - (odd ? ra1 : ra0);
                 vb = two ? (vb - cz1[j]) - (odd ? rb1 : rb0) : 0.f;
@@ -572,8 +671,11 @@ __global__ __launch_bounds__(kFftThreads) void wiener_rows_fwd_kernel(FftDesc d,
     float2 *a0 = A_all + (int64_t)b * plane + (int64_t)i0 * lda;  // rows lda values apart
     for (int k = threadIdx.x; k < wh; k += kFftThreads) {
         const float2 zk = buf[k], zm_ = buf[k == 0 ? 0 : w - k];
-        a0[k] = make_float2(0.5f * (zk.x + zm_.x), 0.5f * (zk.y - zm_.y));
-        if (two) a0[lda + k] = make_float2(0.5f * (zk.y + zm_.y), -0.5f * (zk.x - zm_.x));
+        float2 fa = make_float2(0.5f * (zk.x + zm_.x), 0.5f * (zk.y - zm_.y));
+        float2 fb = make_float2(0.5f * (zk.y + zm_.y), -0.5f * (zk.x - zm_.x));
+        if (ZM_EVEN && (k == 0 || 2 * k == w)) fa = fb = make_float2(0.f, 0.f);
+        a0[k] = fa;
+        if (two) a0[lda + k] = fb;
     }
     // both row sums in one fixed-order block reduction
     sq0 = wave_sum_d(sq0);
@@ -584,8 +686,16 @@ __global__ __launch_bounds__(kFftThreads) void wiener_rows_fwd_kernel(FftDesc d,
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        rowsq_all[(int64_t)b * h + i0] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-        if (two) rowsq_all[(int64_t)b * h + i1] = (sh[4] + sh[5]) + (sh[6] + sh[7]);
+        double s0 = (sh[0] + sh[1]) + (sh[2] + sh[3]), s1 = (sh[4] + sh[5]) + (sh[6] + sh[7]);
+        if (ZM_EVEN) {
+            // Z_0 = Se + So, Z_{w/2} = Se - So (row i0 the real, i1 the imaginary parts):
+            // Se^2 + So^2 = (Z_0^2 + Z_{w/2}^2) / 2
+            const float2 z0 = buf[0], zh = buf[w / 2];
+            s0 -= ((double)z0.x * z0.x + (double)zh.x * zh.x) / (double)w;
+            s1 -= ((double)z0.y * z0.y + (double)zh.y * zh.y) / (double)w;
+        }
+        rowsq_all[(int64_t)b * h + i0] = s0;
+        if (two) rowsq_all[(int64_t)b * h + i1] = s1;
     }
 }
 
@@ -1081,11 +1191,11 @@ size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 // Zero-mean partial-sum tiles the workspace holds: enough for either FastNoise kernel.
 int zm_tiles_x_max(int w) { return std::max((w + kZmTileCols - 1) / kZmTileCols, zm_tiles_x_rows(w)); }
-int zm_tiles_y_max(int h) { return std::max((h + kZmTileRows - 1) / kZmTileRows, zm_tiles_y_rows(h)); }
+int zm_tiles_y_max(int h, int w) { return std::max((h + kZmTileRows - 1) / kZmTileRows, zm_tiles_y_rows(h, w)); }
 
 size_t per_image_bytes(int h, int w) {
     const int64_t n = (int64_t)h * w;
-    const int tx = zm_tiles_x_max(w), ty = zm_tiles_y_max(h);
+    const int tx = zm_tiles_x_max(w), ty = zm_tiles_y_max(h, w);
     return (strips_for(h) ? 16 : 24) * (size_t)n + 8 * (size_t)(h + 1 + 2 * w * ty + 2 * h * tx + 2 * w + 2 * h + 4) +
            4 * (size_t)(2 * w + 2 * h) + 13 * 256;
 }
@@ -1098,7 +1208,7 @@ int get_ws(Context *c, int nb, ExtractWs &e) {
     // the tiles of the zm_partials_kernel layout; launch_fastnoise reports its own
     e.tiles_x = (w + kZmTileCols - 1) / kZmTileCols;
     e.tiles_y = (h + kZmTileRows - 1) / kZmTileRows;
-    e.cp_stride = 2 * (int64_t)w * zm_tiles_y_max(h);
+    e.cp_stride = 2 * (int64_t)w * zm_tiles_y_max(h, w);
     e.rp_stride = 2 * (int64_t)h * zm_tiles_x_max(w);
     const size_t sz[] = {align256(sizeof(float2) * n * nb),
                          strips_for(h) ? 0 : align256(sizeof(float2) * n * nb),
@@ -1152,16 +1262,16 @@ int launch_fastnoise_fmt(const void *in, int64_t in_stride, float *out, int64_t 
                          double *colpart, int64_t cp_stride, double *rowpart, int64_t rp_stride, int *tiles_x,
                          int *tiles_y, hipStream_t st) {
     if (fastnoise_rows_ok(out, out_stride, h, w, nb)) {
-        const int nseg = (w + kFnSeg - 1) / kFnSeg, ngrp = (zm_tiles_y_rows(h) + 3) / 4;
+        const int nseg = (w + kFnSeg - 1) / kFnSeg, ngrp = (zm_tiles_y_rows(h, w) + 3) / 4;
         const int64_t nunits = (int64_t)nseg * ngrp * nb;
         PRNU_REQUIRE(nunits < (int64_t(1) << 30), "fastnoise: %lld units", (long long)nunits);
         const int per = (int)((nunits + 7) / 8);
         hipLaunchKernelGGL(fastnoise_rows_kernel<FMT>, dim3((unsigned)(8 * per)), dim3(256), 0, st,
-                           static_cast<const uint8_t *>(in), in_stride, out, out_stride, h, w, colpart, cp_stride,
-                           rowpart, rp_stride, nseg, ngrp, (int)nunits);
+                           static_cast<const uint8_t *>(in), in_stride, out, out_stride, h, w, fn_band(h, w), colpart,
+                           cp_stride, rowpart, rp_stride, nseg, ngrp, (int)nunits);
         PRNU_CHECK_LAUNCH();
         *tiles_x = zm_tiles_x_rows(w);
-        *tiles_y = zm_tiles_y_rows(h);
+        *tiles_y = zm_tiles_y_rows(h, w);
         return PRNU_OK;
     }
     const int ntx = (w + kFnTX - 1) / kFnTX, nty = (h + kFnTY - 1) / kFnTY;
@@ -1224,6 +1334,11 @@ int launch_cols_fft(const FftDesc &dh, float2 *A, int64_t plane, int ld, int nco
     return PRNU_OK;
 }
 
+// Sizes whose zero-mean takes the ZM_EVEN form of wiener_rows_fwd_kernel.
+// (With one row or column of a parity the zero-mean image is nothing but
+// rounding: those keep the general form and its results.)
+bool zm_even_form(int h, int w) { return w % 2 == 0 && w >= 4 && h >= 3; }
+
 // Row pitch of the chain's half-spectrum plane A: 128-byte rows (a multiple
 // of 16 complex values) where the strip kernels read or write A in 64-byte
 // row pieces (1024 and 1536 rows), so that no piece straddles two lines;
@@ -1252,13 +1367,23 @@ int launch_wiener(Context *c, ExtractWs &e, int nb, const float *img, int64_t im
     // (the two-wave 2048-point form measured slower here, 331 -> 365 us per
     // 32 frames of 2048x1536: four loads per value and FP64 sums at 4 waves
     // per SIMD; it pays in rows_c2r_kernel)
-    if (w == 2048)
-        hipLaunchKernelGGL((wiener_rows_fwd_kernel<kFftSmallN, true>), dim3(pairs, nb), dim3(kFftThreads),
-                           sizeof(float2) * kFft2048PadLds, st, dw, img, img_stride, h, e.A, n, e.rowsq,
-                           zm ? e.cz : nullptr, zm ? e.rz : nullptr, lda);
-    else
-        PRNU_LAUNCH_ROW(wiener_rows_fwd_kernel, w, dim3(pairs, nb), st, dw, img, img_stride, h, e.A, n, e.rowsq,
-                        zm ? e.cz : nullptr, zm ? e.rz : nullptr, lda);
+    const bool zm_even = zm && zm_even_form(h, w);
+#define PRNU_WIENER_ROWS(M, PAD, ZE)                                                                                \
+    hipLaunchKernelGGL((wiener_rows_fwd_kernel<M, PAD, ZE>), dim3(pairs, nb), dim3(kFftThreads),                    \
+                       PAD ? sizeof(float2) * kFft2048PadLds : fft_row_smem(w), st, dw, img, img_stride, h, e.A, n, \
+                       e.rowsq, zm ? e.cz : nullptr, zm ? e.rz : nullptr, lda)
+    if (zm_even) {
+        if (w == 2048) PRNU_WIENER_ROWS(kFftSmallN, true, true);
+        else if (w <= kFftSmallN) PRNU_WIENER_ROWS(kFftSmallN, false, true);
+        else if (w <= kFftMidN) PRNU_WIENER_ROWS(kFftMidN, false, true);
+        else PRNU_WIENER_ROWS(kFftMaxN, false, true);
+    } else {
+        if (w == 2048) PRNU_WIENER_ROWS(kFftSmallN, true, false);
+        else if (w <= kFftSmallN) PRNU_WIENER_ROWS(kFftSmallN, false, false);
+        else if (w <= kFftMidN) PRNU_WIENER_ROWS(kFftMidN, false, false);
+        else PRNU_WIENER_ROWS(kFftMaxN, false, false);
+    }
+#undef PRNU_WIENER_ROWS
     PRNU_CHECK_LAUNCH();
     hipLaunchKernelGGL(wiener_var_kernel, dim3(nb), dim3(256), 0, st, e.rowsq, h, n, e.var);
     PRNU_CHECK_LAUNCH();
@@ -1395,9 +1520,16 @@ int run_preprocess_batch(Context *c, int fmt, const void *in, size_t in_bytes, i
         uint8_t *dst = static_cast<uint8_t *>(out) + (size_t)b0 * out_stride;
         // gray + FastNoise into S (FP32 images n apart), zero-mean sums on the side
         float *noise = e.S;
-        PRNU_TRY(launch_fastnoise(fmt, src, in_stride, noise, n, c->h, c->w, nb, e.colpart, e.cp_stride, e.rowpart,
-                                  e.rp_stride, &e.tiles_x, &e.tiles_y, st));
-        PRNU_TRY(launch_zm_means(c, e, nb, st));
+        const bool even = zm_even_form(c->h, c->w);  // column means are all the Wiener rows need
+        PRNU_TRY(launch_fastnoise(fmt, src, in_stride, noise, n, c->h, c->w, nb, e.colpart, e.cp_stride,
+                                  even ? nullptr : e.rowpart, e.rp_stride, &e.tiles_x, &e.tiles_y, st));
+        if (even) {
+            hipLaunchKernelGGL(zm_colmean_kernel, dim3((c->w + 63) / 64, nb), dim3(256), 0, st, e.colpart,
+                               e.cp_stride, c->h, c->w, e.tiles_y, e.cz);
+            PRNU_CHECK_LAUNCH();
+        } else {
+            PRNU_TRY(launch_zm_means(c, e, nb, st));
+        }
         if (c->mode == PRNU_MODE_NCC) {
             PRNU_TRY(launch_wiener(c, e, nb, noise, n, reinterpret_cast<float *>(dst), out_stride / 4, true, st));
         } else {
