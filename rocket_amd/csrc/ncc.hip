@@ -4,13 +4,15 @@
 //
 // Gram design.  G = P P^T over K = h*w is tiny-M, huge-K, so the triangle of
 // 256x256 tiles is split along K into S slabs.  One 512-thread workgroup
-// computes one (tile, slab) partial in FP32 MFMA accumulators and writes it
-// out; a second kernel sums the S partials of each element in FP64 in a fixed
-// order (deterministic) and applies the NCC epilogue.  Workgroup ids are
-// remapped so that the T tiles of one K slab land on the same XCD (workgroups
-// are dealt round-robin over the 8 XCDs), which lets those T workgroups share
+// computes one work item of a slab (gram_items.hpp: up to four 128 x 128 units
+// of the triangle) in FP32 MFMA accumulators and writes it out; a second
+// kernel sums the S partials of each element in FP64 in a fixed order
+// (deterministic) and applies the NCC epilogue.  Workgroup ids are
+// remapped so that the items of one K slab land on the same XCD (workgroups
+// are dealt round-robin over the 8 XCDs), which lets those workgroups share
 // the slab through that XCD's L2 instead of each pulling it from HBM.
 #include "prnu_internal.hpp"
+#include "gram_items.hpp"
 
 #include <algorithm>
 #include <mutex>
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(kThreads) void pair_ncc_final_kernel(const double *
 }
 
 // --------------------------------------------------------------- Gram
-constexpr int kTile = 256;         // patterns per tile side
+constexpr int kTile = kGramTile;   // patterns per tile side
 constexpr int kKT = 32;            // K per LDS stage
 constexpr int kGramThreads = 512;  // 8 waves: 2 (rows) x 4 (cols), wave tile 128 x 64
 constexpr int kRows = 2 * kTile;   // A rows then B rows in LDS
@@ -215,20 +217,11 @@ struct GramArgs {
     int64_t kchunk;
     int M;
     int nt;  // tiles per side
-    int T;   // tiles in the upper triangle, nt*(nt+1)/2
+    int T;   // work items per slab (variant 1: tiles in the upper triangle)
+    int ks;  // slabs the last of them takes at once (slab_split)
     int S;   // K slabs
-    int xcd_remap;  // 1: the T tiles of a slab run on one XCD
+    int xcd_remap;  // 1: the T items of a slab run on one XCD
 };
-
-// Linear index over the upper triangle (row-major, I <= J) -> (I, J).
-__device__ inline int2 tri_tile(int t, int nt) {
-    int I = 0;
-    while (t >= nt - I) {
-        t -= nt - I;
-        ++I;
-    }
-    return make_int2(I, I + t);
-}
 
 __device__ inline uint16_t bf16_bits(float v) { return __builtin_bit_cast(uint16_t, (__bf16)v); }
 __device__ inline float bf16_val(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
@@ -246,16 +239,20 @@ struct RowSet {
     const float *p[8];  // always a readable pattern row (absent rows alias a present one)
     bool valid[8];
 };
+// K range of each LDS quarter of 128 rows (rows r_lo + 64*it: quarter it / 2).
+struct KSet {
+    int64_t beg[4], end[4];
+};
 
-// Main K loop of one (tile, slab) workgroup.  Double-buffered LDS, one
-// barrier per stage: loads for stage s+1 are issued before the MFMAs of
+// Main K loop of one work item: `nst` stages, of which this wave multiplies
+// the first `own`.  Double-buffered LDS, one barrier per stage: loads for stage s+1 are issued before the MFMAs of
 // stage s and written to the other buffer after them.
 // FAST: every row 16-byte aligned and K % 4 == 0, so a float4 at a multiple
 // of 4 is wholly inside or wholly outside [k_begin, k_end); its address is
 // clamped into the row and out-of-slab values are zeroed when stored.
 template <int PREC, bool FAST>
-__device__ __forceinline__ void gram_mainloop(uint32_t *lds, const RowSet &rs, int nrows, int bbase, int wrow0,
-                                              int wcol0, int64_t k_begin, int64_t k_end, int64_t K,
+__device__ __forceinline__ void gram_mainloop(uint32_t *lds, const RowSet &rs, int nrows, int wrow0, int wcol0,
+                                              const KSet &ks, int64_t nst, int64_t own, int64_t K,
                                               floatx4 (&acc)[8][4]) {
     constexpr bool kSplit = PREC == PRNU_PREC_SPLIT_BF16;
     constexpr int kBuf = kRows * 32;  // uint32 per stage buffer (64 KiB)
@@ -265,11 +262,11 @@ __device__ __forceinline__ void gram_mainloop(uint32_t *lds, const RowSet &rs, i
     const int c4 = (tid & 7) * 4;
     float4 st[8];
 
-    auto load = [&](int64_t k0) {
+    auto load = [&](int64_t s) {
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
             if (FAST) {
-                const int64_t kk = k0 + c4;
+                const int64_t kk = ks.beg[it >> 1] + s * kKT + c4;
                 const int64_t kc = kk < K ? kk : K - 4;
                 // global (not flat) loads: flat loads also count on lgkmcnt and
                 // would make every LDS wait of the compute phase wait for them
@@ -280,20 +277,20 @@ __device__ __forceinline__ void gram_mainloop(uint32_t *lds, const RowSet &rs, i
                 float e[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int64_t kk = k0 + c4 + q;
-                    e[q] = (rs.valid[it] && kk < k_end) ? rs.p[it][kk] : 0.f;
+                    const int64_t kk = ks.beg[it >> 1] + s * kKT + c4 + q;
+                    e[q] = (rs.valid[it] && kk < ks.end[it >> 1]) ? rs.p[it][kk] : 0.f;
                 }
                 st[it] = make_float4(e[0], e[1], e[2], e[3]);
             }
         }
     };
 
-    auto store = [&](uint32_t *buf, int64_t k0) {
-        const bool kin = k0 + c4 < k_end;
+    auto store = [&](uint32_t *buf, int64_t s) {
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
             const int r = r_lo + 64 * it;
             if (r < nrows) {
+                const bool kin = ks.beg[it >> 1] + s * kKT + c4 < ks.end[it >> 1];
                 float4 v = st[it];
                 if (FAST && !(rs.valid[it] && kin)) v = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (kSplit) {
@@ -326,7 +323,7 @@ __device__ __forceinline__ void gram_mainloop(uint32_t *lds, const RowSet &rs, i
             bf16x8 bh[4], bl[4];
 #pragma unroll
             for (int cb = 0; cb < 4; ++cb) {
-                const int off = bf_off(bbase + wcol0 + cb * 16 + frow, chunk);
+                const int off = bf_off(wcol0 + cb * 16 + frow, chunk);
                 bh[cb] = *reinterpret_cast<const bf16x8 *>(hi + off);
                 bl[cb] = *reinterpret_cast<const bf16x8 *>(lo + off);
             }
@@ -350,7 +347,7 @@ __device__ __forceinline__ void gram_mainloop(uint32_t *lds, const RowSet &rs, i
                 float4 bf[4];
 #pragma unroll
                 for (int cb = 0; cb < 4; ++cb)
-                    bf[cb] = *reinterpret_cast<const float4 *>(f + f_off(bbase + wcol0 + cb * 16 + frow, chunk));
+                    bf[cb] = *reinterpret_cast<const float4 *>(f + f_off(wcol0 + cb * 16 + frow, chunk));
 #pragma unroll
                 for (int rb = 0; rb < 8; ++rb) {
                     const float4 af = *reinterpret_cast<const float4 *>(f + f_off(wrow0 + rb * 16 + frow, chunk));
@@ -366,16 +363,14 @@ __device__ __forceinline__ void gram_mainloop(uint32_t *lds, const RowSet &rs, i
         }
     };
 
-    const int64_t nst = (k_end - k_begin + kKT - 1) / kKT;
-    load(k_begin);
-    store(lds, k_begin);
+    load(0);
+    store(lds, 0);
     __syncthreads();
     for (int64_t s = 0; s < nst; ++s) {
         const bool next = s + 1 < nst;
-        const int64_t kn = k_begin + (s + 1) * kKT;
-        if (next) load(kn);
-        compute(lds + (s & 1) * kBuf);
-        if (next) store(lds + ((s + 1) & 1) * kBuf, kn);
+        if (next) load(s + 1);
+        if (s < own) compute(lds + (s & 1) * kBuf);
+        if (next) store(lds + ((s + 1) & 1) * kBuf, s + 1);
         __syncthreads();
     }
 }
@@ -384,40 +379,43 @@ template <int PREC>
 __global__ __launch_bounds__(kGramThreads, 1) void gram_tile_kernel(GramArgs a) {
     __shared__ __attribute__((aligned(16))) uint32_t lds[2 * kRows * 32];  // 2 x 64 KiB stage buffers
 
-    // ---- workgroup -> (tile, slab).  Workgroups are dealt round-robin to the
-    // 8 XCDs (bid mod 8); with xcd_remap the T tiles of slab s all have
-    // bid = s mod 8 (mod 8) and run back to back on one XCD.
-    const int bid = blockIdx.x;
-    int t, s;
-    if (a.xcd_remap) {
-        const int local = bid >> 3;
-        t = local % a.T;
-        s = (local / a.T) * 8 + (bid & 7);
-    } else {
-        t = bid % a.T;
-        s = bid / a.T;
-    }
-    if (s >= a.S) return;
-    const int2 tile = tri_tile(t, a.nt);
-    const bool diag = tile.x == tile.y;
-    const int nrows = diag ? kTile : kRows;
-    const int64_t k_begin = (int64_t)s * a.kchunk;
-    const int64_t k_end = min(a.K, k_begin + a.kchunk);
-
+    int u, s;
+    if (!ItemIndex(a.T, a.ks, a.S).at(blockIdx.x, a.xcd_remap, u, s)) return;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wrow0 = (wave >> 2) * 128;  // A rows of this wave
-    const int wcol0 = (wave & 3) * 64;    // B rows of this wave
-    const int bbase = diag ? 0 : kTile;   // B rows start in LDS
+    ItemWaves w = item_waves(u, a.M, __builtin_amdgcn_readfirstlane(tid >> 6));
+    // wave-uniform: keep it in scalar registers
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        w.q[k] = __builtin_amdgcn_readfirstlane(w.q[k]);
+        w.kq[k] = __builtin_amdgcn_readfirstlane(w.kq[k]);
+    }
+    w.nq = __builtin_amdgcn_readfirstlane(w.nq);
+    w.kw = __builtin_amdgcn_readfirstlane(w.kw);
+    w.out_tile = __builtin_amdgcn_readfirstlane(w.out_tile);
+    w.out_off = __builtin_amdgcn_readfirstlane(w.out_off);
+    const int wrow0 = __builtin_amdgcn_readfirstlane(w.a_off >> 6) << 6;
+    const int wcol0 = __builtin_amdgcn_readfirstlane(w.b_off >> 6) << 6;
+    const int nrows = 128 * w.nq;
+    KSet ks;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        ks.beg[k] = (int64_t)(s + w.kq[k]) * a.kchunk;
+        ks.end[k] = min(a.K, ks.beg[k] + a.kchunk);
+    }
+    auto stages = [&](int sl) {
+        const int64_t beg = (int64_t)sl * a.kchunk;
+        return max(int64_t(0), (min(a.K, beg + a.kchunk) - beg + kKT - 1) / kKT);
+    };
+    const int64_t nst = stages(s), own = w.out_tile < 0 ? 0 : stages(s + w.kw);
 
     RowSet rs;
-    const float *any_row = a.ptrs[min(tile.x * kTile, a.M - 1)];
+    const float *any_row = a.ptrs[min(w.q[0], a.M - 1)];
     int aligned = (a.K & 3) == 0;
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
         const int r = (tid >> 3) + 64 * it;
-        const int g = (r < kTile) ? tile.x * kTile + r : tile.y * kTile + (r - kTile);
+        const int g = w.q[it >> 1] + (r & 127);
         const bool v = r < nrows && g < a.M;
         rs.valid[it] = v;
         rs.p[it] = v ? a.ptrs[g] : any_row;
@@ -432,21 +430,26 @@ __global__ __launch_bounds__(kGramThreads, 1) void gram_tile_kernel(GramArgs a) 
         for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     if (aligned)
-        gram_mainloop<PREC, true>(lds, rs, nrows, bbase, wrow0, wcol0, k_begin, k_end, a.K, acc);
+        gram_mainloop<PREC, true>(lds, rs, nrows, wrow0, wcol0, ks, nst, own, a.K, acc);
     else
-        gram_mainloop<PREC, false>(lds, rs, nrows, bbase, wrow0, wcol0, k_begin, k_end, a.K, acc);
+        gram_mainloop<PREC, false>(lds, rs, nrows, wrow0, wcol0, ks, nst, own, a.K, acc);
 
-    // ---- epilogue: FP32 partial tile, row = A index, col = B index
-    float *out = a.partials + ((int64_t)t * a.S + s) * (kTile * kTile);
+    // ---- epilogue: FP32 partial block, row = A index, col = B index; 16 x 16
+    // sub-blocks past the set's end or below its diagonal are not read
+    if (own == 0) return;
+    float *out = a.partials + ((int64_t)w.out_tile * a.S + s + w.kw) * (kTile * kTile) + w.out_off;
+    const int i0 = row_pattern(w, wrow0), j0 = row_pattern(w, wcol0);
     const int ocol = lane & 15;
     const int orow = (lane >> 4) * 4;
 #pragma unroll
     for (int rb = 0; rb < 8; ++rb)
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
+        for (int cb = 0; cb < 4; ++cb) {
+            const int i = i0 + rb * 16, j = j0 + cb * 16;
+            if (i >= a.M || j >= a.M || i > j + 15) continue;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                out[(wrow0 + rb * 16 + orow + r) * kTile + wcol0 + cb * 16 + ocol] = acc[rb][cb][r];
+            for (int r = 0; r < 4; ++r) out[(rb * 16 + orow + r) * kTile + cb * 16 + ocol] = acc[rb][cb][r];
+        }
 }
 
 // Variant 1 of the split-BF16 tile kernel: 4 waves (one per SIMD, so each
@@ -626,30 +629,6 @@ __global__ __launch_bounds__(kG4Threads, 1) void gram_tile4_kernel(GramArgs a) {
                 out[(wrow0 + rb * 16 + orow + r) * kTile + wcol0 + cb * 16 + ocol] = acc[rb][cb][r];
 }
 
-// Sum the S partials of each element in FP64 (fixed order) and apply the NCC
-// epilogue of normalizedcrosscorrelation.cu:121-123.  grid (256, T), block 256.
-__global__ __launch_bounds__(kThreads) void gram_reduce_kernel(const float *__restrict__ partials, int S,
-                                                               int nt, int M,
-                                                               const double *__restrict__ sum,
-                                                               const double *__restrict__ sumsq,
-                                                               double *__restrict__ out) {
-    const int t = blockIdx.y;
-    const int e = blockIdx.x * kThreads + threadIdx.x;
-    const int2 tile = tri_tile(t, nt);
-    const int i = tile.x * kTile + (e >> 8);
-    const int j = tile.y * kTile + (e & 255);
-    if (i >= M || j >= M) return;
-    if (tile.x == tile.y && i > j) return;
-    const float *p = partials + (int64_t)t * S * (kTile * kTile) + e;
-    double g = 0.0;
-    for (int q = 0; q < S; ++q) g += (double)p[(int64_t)q * (kTile * kTile)];
-    const double di = sqrt(sumsq[i] - sum[i] * sum[i]);
-    const double dj = sqrt(sumsq[j] - sum[j] * sum[j]);
-    const double v = g / (di * dj);
-    out[(int64_t)i * M + j] = v;
-    out[(int64_t)j * M + i] = v;
-}
-
 }  // namespace
 
 // ================================================================ launchers
@@ -734,32 +713,38 @@ int launch_pair_ncc(const float *x, const float *y, int64_t n, double *d_out, Wo
 namespace {
 
 struct GramPlan {
-    int nt, T;
+    int nt, T, ks, tiles;  // items per slab, the slabs of the last (slab_split), partial tiles per slab
     int64_t S, kchunk;
     int xcd_remap;
     int variant;
 };
 
-// K split of the Gram: `slabs` per tile (0: about 5 workgroups per CU, >= 16
-// stages per slab), partials capped at 2 GiB.
+// K split of the Gram: `slabs` per tile (0: the slab length choose_kcb finds
+// cheapest, no longer than about 5 workgroups per CU of whole tiles give at 16
+// stages and more, for the FP32 sums' precision), partials capped at 2 GiB.
 GramPlan plan_gram(const Context *c, int count, int precision) {
     GramPlan p;
     const int64_t K = c->pixels();
+    p.variant = precision == PRNU_PREC_SPLIT_BF16 ? c->gram_cfg[precision].variant : 0;
     p.nt = (count + kTile - 1) / kTile;
-    p.T = p.nt * (p.nt + 1) / 2;
+    p.tiles = p.nt * (p.nt + 1) / 2;
+    p.T = p.variant == 1 ? p.tiles : tri_items_per_slab(count);  // gram_tile4_kernel runs whole tiles
+    p.ks = p.variant == 1 ? 1 : slab_split(count);
     const int64_t stages = (K + kKT - 1) / kKT;
-    int64_t S = c->gram_cfg[precision].slabs;
-    if (S <= 0) {
-        S = std::max<int64_t>(1, (256 * 5 + p.T - 1) / p.T);
-        S = std::min<int64_t>(S, std::max<int64_t>(1, stages / 16));
-    }
-    S = std::min<int64_t>(S, stages);
     const int64_t tile_bytes = (int64_t)kTile * kTile * sizeof(float);
-    S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * p.T)));
-    p.kchunk = ((stages + S - 1) / S) * kKT;
+    if (c->gram_cfg[precision].slabs > 0) {
+        int64_t S = std::min<int64_t>(c->gram_cfg[precision].slabs, stages);
+        S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * p.tiles)));
+        p.kchunk = ((stages + S - 1) / S) * kKT;
+    } else {
+        int64_t S = std::max<int64_t>(1, (256 * 5 + p.tiles - 1) / p.tiles);
+        S = std::min<int64_t>(S, std::max<int64_t>(1, stages / 16));
+        S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * p.tiles)));
+        p.kchunk = kKT * choose_kcb(&p.T, &p.ks, &p.tiles, &stages, 1, device_cus(c->device), size_t(2) << 30,
+                                    (stages + S - 1) / S);
+    }
     p.S = (K + p.kchunk - 1) / p.kchunk;
     p.xcd_remap = c->gram_cfg[precision].xcd_remap;
-    p.variant = precision == PRNU_PREC_SPLIT_BF16 ? c->gram_cfg[precision].variant : 0;
     return p;
 }
 
@@ -773,10 +758,10 @@ int launch_gram_tiles(Context *c, const GramPlan &p, const float *const *d_ptrs,
     a.M = count;
     a.nt = p.nt;
     a.T = p.T;
+    a.ks = p.ks;
     a.S = (int)p.S;
     a.xcd_remap = p.xcd_remap;
-    const int64_t S8 = p.xcd_remap ? (p.S + 7) / 8 * 8 : p.S;
-    const dim3 grid((unsigned)(p.T * S8));
+    const dim3 grid((unsigned)ItemIndex(p.T, p.ks, (int)p.S).ids(p.xcd_remap));
     if (precision == PRNU_PREC_SPLIT_BF16 && p.variant == 1)
         hipLaunchKernelGGL(gram_tile4_kernel, grid, dim3(kG4Threads), 0, st, a);
     else if (precision == PRNU_PREC_SPLIT_BF16)
@@ -807,16 +792,13 @@ int launch_gram_ncc(Context *c, const float *const *d_ptrs, int count, int preci
                               nullptr, nullptr, nullptr, stride, d_ncc, count, c->gram_cfg[precision].slabs, st, c);
     }
     const GramPlan p = plan_gram(c, count, precision);
-    const size_t part_bytes = (size_t)kTile * kTile * sizeof(float) * p.T * p.S;
+    const size_t part_bytes = (size_t)kTile * kTile * sizeof(float) * p.tiles * p.S;
     PRNU_TRY(c->ws_gram.ensure(part_bytes));
     float *partials = static_cast<float *>(c->ws_gram.ptr);
     time_begin(c, st);
     PRNU_TRY(launch_gram_tiles(c, p, d_ptrs, count, precision, partials, st));
     time_end(c, st);
-    hipLaunchKernelGGL(gram_reduce_kernel, dim3(kTile * kTile / kThreads, p.T), dim3(kThreads), 0, st, partials,
-                       (int)p.S, p.nt, count, d_sum, d_sumsq, d_ncc);
-    PRNU_CHECK_LAUNCH();
-    return PRNU_OK;
+    return launch_tri_reduce(partials, (int)p.S, p.nt, count, d_sum, d_sumsq, nullptr, d_ncc, (int64_t)count, st);
 }
 
 int gram_resolved_config(Context *c, int count, int precision, prnu_gram_config *out) {
@@ -850,7 +832,7 @@ int autotune_gram(Context *c, const float *const *d_ptrs, int count, int precisi
         for (int xcd = 1; xcd >= 0 && status == PRNU_OK; --xcd) {
             c->gram_cfg[precision] = prnu_gram_config{(int32_t)S, xcd, var};
             const GramPlan p = plan_gram(c, count, precision);
-            const size_t part_bytes = (size_t)kTile * kTile * sizeof(float) * p.T * p.S;
+            const size_t part_bytes = (size_t)kTile * kTile * sizeof(float) * p.tiles * p.S;
             status = c->ws_gram.ensure(part_bytes);
             if (status != PRNU_OK) break;
             float *partials = static_cast<float *>(c->ws_gram.ptr);

@@ -17,6 +17,7 @@
 // split is done once at insert time instead of in every tile that reads the
 // value, and the per-pattern FP64 statistics are taken in the same pass.
 #include "prnu_internal.hpp"
+#include "gram_items.hpp"
 
 #include <cstring>
 
@@ -51,7 +52,7 @@ constexpr int kBlk8 = 128;      // values per block (FP8)
 constexpr int kBlk16 = 64;      // values per block (FP16)
 constexpr float kE4M3Max = 448.0f;
 constexpr int kBlkBytes = 128;  // bytes per block
-constexpr int kTileS = 256;
+constexpr int kTileS = kGramTile;
 constexpr int kRowsS = 2 * kTileS;
 constexpr int kThrS = 512;
 constexpr int kMaxPlanGroups = 4096;
@@ -270,141 +271,147 @@ struct StoreGramArgs {
     int64_t kcb;         // blocks per slab
     int first, count;
     int nt, T, S;        // T: work items per slab
+    int ks;              // slabs the last of them takes at once (slab_split)
     int xcd_remap;
 };
-
-__device__ inline int2 tri_tile_s(int t, int nt) {
-    int I = 0;
-    while (t >= nt - I) {
-        t -= nt - I;
-        ++I;
-    }
-    return make_int2(I, I + t);
-}
 
 // 16-byte chunk c of LDS row r (128-byte rows), XOR-swizzled by row.
 __device__ __forceinline__ int s_off(int row, int chunk) { return row * kBlkBytes + ((chunk ^ (row & 7)) << 4); }
 
 constexpr int kBufS = kRowsS * kBlkBytes;  // 64 KiB per LDS stage
-
-// Work items.  The LDS stage holds four quarters of 128 pattern rows; a
-// wave multiplies the 128 rows of one quarter by 64 rows of another (a
-// 128 x 64 block of the output), and waves 2k, 2k+1 together cover the
-// 128 x 128 sub-tile of one quarter pair (unit k of the item).  The triangle
-// of Q = ceil(count / 128) quarters has Q (Q + 1) / 2 units (quarter pairs
-// qa <= qb); an item holds at most 4 units over at most 4 quarters, so a
-// slab needs at least ceil(Q (Q + 1) / 8) items.  With m = floor(Q / 2)
-// full 256-row tiles, per slab:
-//  - m (m - 1) / 2 off-diagonal tiles (I, J): quarters 2I, 2I+1, 2J, 2J+1,
-//    all four units of the pair;
-//  - Q even: ceil(6 m / 8) diagonal packs.  A diagonal tile needs 3 units,
-//    the 6 wave blocks (wr, wc) = (0,0) (0,1) (0,2) (0,3) (1,2) (1,3); the
-//    6m such blocks are numbered e = 6 d + l and pack p gives block 8p + w
-//    to wave w.  Eight consecutive blocks span at most two diagonal tiles
-//    d0 = 8p / 6 and d0 + 1, whose quarters fill the LDS.
-//  - Q odd (last quarter L = 2m alone in tile m): m "edge" items d with
-//    quarters 2d, 2d+1, L and units (2d,2d) (2d,2d+1) (2d,L) (2d+1,L), then
-//    ceil((m + 1) / 4) items of the remaining one-quarter units
-//    (2j+1, 2j+1), j < m, and (L, L), four per item.
-// Both reach the bound: m(m-1)/2 + ceil(6m/8) = ceil(Q(Q+1)/8) for even Q,
-// m(m-1)/2 + m + ceil((m+1)/4) = ceil(Q(Q+1)/8) for odd Q.  The output of
-// unit (qa, qb) is the sub-tile at rows 128 (qa & 1), columns 128 (qb & 1)
-// of partial tile (qa / 2, qb / 2).
-struct ItemWaves {
-    int q[4];             // first pattern (relative to the range) of LDS rows [128 k, 128 k + 128)
-    int nq;               // quarters loaded: LDS rows [0, 128 nq)
-    int a_off, b_off;     // this wave's first A row / first B row in LDS
-    int out_tile;         // triangle index of the tile this wave writes, -1: idle wave
-    int out_off;          // offset of the wave's 128 x 64 block inside that tile
-};
-
-__device__ __forceinline__ int tri_index(int I, int J, int nt) { return I * nt - I * (I - 1) / 2 + (J - I); }
-
-__device__ __forceinline__ void item_tiles(ItemWaves &r, int x, int y) {
-    r.q[0] = x * kTileS;
-    r.q[1] = x * kTileS + 128;
-    r.q[2] = y * kTileS;
-    r.q[3] = y * kTileS + 128;
+// FP16 items work in half blocks (32 values, 64-byte rows) through a ring of
+// five 32 KiB stages, four of them on their way (gram_item_fp16).
+constexpr int kRing16 = 5;
+constexpr int kHalfRow = kBlkBytes / 2;
+constexpr int kBuf16 = kRowsS * kHalfRow;
+template <int FMT, int VAR>
+constexpr int item_lds() {
+    return FMT == PRNU_PREC_FP16 && VAR != 1 ? kRing16 * kBuf16 : 2 * kBufS;
 }
 
-// Item u of a slab of the triangle of `count` patterns (nt = ceil(count /
-// 256) partial tiles), for wave `wave`.
-__device__ __forceinline__ ItemWaves item_waves(int u, int count, int wave) {
-    ItemWaves r;
-    const int Q = (count + 127) >> 7, m = Q >> 1, nt = (count + kTileS - 1) / kTileS;
-    const int wr = wave >> 2, wc = wave & 3;
-    const int toff = m * (m - 1) / 2;
-    if (u < toff) {
-        int I = 0, t = u;
-        while (t >= m - 1 - I) {
-            t -= m - 1 - I;
-            ++I;
-        }
-        const int J = I + 1 + t;
-        item_tiles(r, I, J);
-        r.nq = 4;
-        r.a_off = wr * 128;
-        r.b_off = kTileS + wc * 64;
-        r.out_tile = tri_index(I, J, nt);
-        r.out_off = wr * 128 * kTileS + wc * 64;
-        return r;
-    }
-    const int p = u - toff;
-    r.out_tile = -1;
-    r.a_off = r.b_off = r.out_off = 0;
-    if (!(Q & 1)) {
-        const int d0 = (8 * p) / 6;
-        const int dl = min(m - 1, (8 * p + 7) / 6);
-        item_tiles(r, d0, dl > d0 ? d0 + 1 : d0);
-        r.nq = dl > d0 ? 4 : 2;
-        const int e = 8 * p + wave;
-        if (e >= 6 * m) return r;
-        const int d = e / 6, l = e - 6 * (e / 6);
-        const int bwr = l < 4 ? 0 : 1;
-        const int bwc = l < 4 ? l : l - 2;
-        const int base = (d - d0) * kTileS;
-        r.a_off = base + bwr * 128;
-        r.b_off = base + bwc * 64;
-        r.out_tile = tri_index(d, d, nt);
-        r.out_off = bwr * 128 * kTileS + bwc * 64;
-        return r;
-    }
-    const int k = wave >> 1, h = wave & 1;
-    if (p < m) {  // edge item of tile d = p: quarters 2d, 2d+1, L
-        const int d = p;
-        r.q[0] = d * kTileS;
-        r.q[1] = d * kTileS + 128;
-        r.q[2] = r.q[3] = m * kTileS;
-        r.nq = 3;
-        const int sa = k == 3 ? 1 : 0;           // A quarter: 2d for units 0..2, 2d+1 for unit 3
-        const int sb = k == 0 ? 0 : k == 1 ? 1 : 2;
-        r.a_off = sa * 128;
-        r.b_off = sb * 128 + h * 64;
-        r.out_tile = tri_index(d, k < 2 ? d : m, nt);
-        r.out_off = sa * 128 * kTileS + (k == 1 ? 128 : 0) + h * 64;
-        return r;
-    }
-    // one-quarter units 4j' .. 4j'+3 of the list (2j+1, 2j+1) j < m, then (L, L)
-    const int j0 = 4 * (p - m);
+// A wave's FP32 partial block to `out` (row stride 256), without the 16 x 16
+// sub-blocks outside [0, rows) x [0, cols) of it or (tri) wholly below the
+// triangle's diagonal: the reduction does not read them.
+__device__ __forceinline__ void write_partial(const floatx4 (&acc)[8][4], const ItemWaves &w, float *__restrict__ out,
+                                              int rows, int cols, bool tri, int lane) {
+    // i - j of the wave's first element: below the diagonal where it is > 0
+    const int dij = row_pattern(w, w.a_off) - row_pattern(w, w.b_off);
+    const int ocol = lane & 15, orow = (lane >> 4) * 4;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int j = min(j0 + i, m);
-        r.q[i] = j * kTileS + (j < m ? 128 : 0);
-    }
-    r.nq = min(4, m + 1 - j0);
-    const int j = j0 + k;
-    if (j > m) return r;
-    r.a_off = k * 128;
-    r.b_off = k * 128 + h * 64;
-    r.out_tile = tri_index(j, j, nt);
-    r.out_off = (j < m ? 128 * kTileS + 128 : 0) + h * 64;
-    return r;
+    for (int rb = 0; rb < 8; ++rb)
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            if (rb * 16 >= rows || cb * 16 >= cols || (tri && dij + rb * 16 > cb * 16 + 15)) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                out[(rb * 16 + orow + r) * kTileS + cb * 16 + ocol] = acc[rb][cb][r];
+        }
 }
 
-// Items per slab of the triangle of `count` patterns (item_waves).
-__host__ __device__ inline int tri_items_per_slab(int count) {
-    const int Q = (count + 127) >> 7, m = Q >> 1;
-    return m * (m - 1) / 2 + ((Q & 1) ? m + (m + 4) / 4 : (6 * m + 7) / 8);
+// 16 bytes per lane from `base` + voff (below `bytes`) straight into LDS, lane
+// i at byte 16 i of `to`.
+__device__ __forceinline__ void lds_fill16(const uint8_t *base, int bytes, uint8_t *to, uint32_t voff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(3))) void *lptr;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr)to, 16, voff, 0, 0, 0);
+#endif
+}
+
+// gram_item for FP16 blocks with direct-to-LDS loads.  An FP16 stage is one
+// product per fragment pair, a third of split-BF16's, so with one 64 KiB stage
+// on its way while the other is multiplied the item waits for memory: 3 us a
+// stage where the fills come from HBM, 0.9 us of it MFMA.  Half blocks make
+// five stages of the CU's 160 KiB of LDS, four in flight: twice the bytes
+// (500, 300 and 120 patterns of 1, 3.1 and 12 M values in one plan: 2.0 ms
+// with the 64 KiB pair, 1.72 ms with the ring; the 120 alone 5.3 TB/s of its
+// blocks).
+// A stage is one K = 32 MFMA per fragment pair; rows are 64 bytes, their four
+// 16-byte chunks XOR-swizzled by (row >> 1) & 3 (conflict-free reads of 16
+// rows).  A wave waits for its own loads of the stage (vmcnt, 4 loads each)
+// and then for the other waves; the same barrier tells it that every wave is
+// done with the stage before, whose buffer the next fill takes.  The sums of
+// an element run over K in the same order as gram_item's: the same bits.
+template <bool SPLIT, bool PRIO>
+__device__ __forceinline__ void gram_item_fp16(const uint8_t *__restrict__ blocks, int64_t cap_bytes, int first,
+                                               int count, int first_b, int count_b, const ItemWaves &w,
+                                               int64_t b_begin, int64_t b_end, int64_t kcb, float *__restrict__ out,
+                                               int rows, int cols, bool tri, uint8_t *lds, int tid) {
+    const bool half = w.nq <= 2;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // load `it` of a stage fills LDS rows 128 it + 16 wave + [0, 16), lane l at
+    // byte 16 l: row l >> 2, slot l & 3, which holds chunk (l & 3) ^ ((row >> 1) & 3)
+    const int lr = lane >> 2, chunk = (lane & 3) ^ ((lr >> 1) & 3);
+    uint32_t voff[4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const int loc = w.q[it] + 16 * wave + lr;
+        const int slot = it < 2 ? first + min(loc, count - 1) : first_b + min(loc, count_b - 1);
+        voff[it] = (uint32_t)slot * kBlkBytes + (uint32_t)(chunk << 4);
+    }
+    // half blocks of the item and of this wave's own slab
+    const int nst = 2 * (int)(SPLIT ? min(kcb, b_end - b_begin) : b_end - b_begin);
+    const int own = out == nullptr ? 0 : SPLIT ? 2 * (int)min(kcb, b_end - b_begin - w.kw * kcb) : nst;
+    auto issue = [&](int q, uint8_t *buf) {
+        const int64_t b = b_begin + (q >> 1);
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            if (SPLIT || it < 2 || !half) {
+                const int64_t col = SPLIT ? min(b + w.kq[it] * kcb, b_end - 1) : b;
+                lds_fill16(blocks + col * cap_bytes, (int)cap_bytes, buf + (128 * it + 16 * wave) * kHalfRow,
+                           voff[it] + (q & 1) * kHalfRow);
+            }
+        }
+    };
+    floatx4 acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+    for (int d = 0; d < kRing16 - 1; ++d)
+        if (d < nst) issue(d, lds + d * kBuf16);
+    const int frow = lane & 15, ch = lane >> 4;
+    const int roff = frow * kHalfRow + ((ch ^ ((frow >> 1) & 3)) << 4);
+    const int aoff = w.a_off * kHalfRow + roff, boff = w.b_off * kHalfRow + roff;
+    int at = 0, to = kRing16 - 1;  // ring slots of stage q and of stage q + 4
+    for (int q = 0; q < nst; ++q) {
+        // stages asked for after q: wait until only their loads are outstanding
+        // (4 a stage, 2 where the item has two quarters).  s_waitcnt
+        // immediates: vmcnt 3:0, expcnt 6:4 (7: no wait), lgkmcnt 11:8 (0)
+        const int ahead = min(nst - 1 - q, kRing16 - 2);
+        static_assert(kRing16 == 5, "the waits below count three stages ahead");
+        const int left = (!SPLIT && half ? 2 : 4) * ahead;
+        if (left == 12) __builtin_amdgcn_s_waitcnt(0x007c);
+        else if (left == 8) __builtin_amdgcn_s_waitcnt(0x0078);
+        else if (left == 6) __builtin_amdgcn_s_waitcnt(0x0076);
+        else if (left == 4) __builtin_amdgcn_s_waitcnt(0x0074);
+        else if (left == 2) __builtin_amdgcn_s_waitcnt(0x0072);
+        else __builtin_amdgcn_s_waitcnt(0x0070);
+        asm volatile("s_barrier" ::: "memory");
+        if (q + kRing16 - 1 < nst) issue(q + kRing16 - 1, lds + to * kBuf16);
+        if (q < own) {
+            const uint8_t *buf = lds + at * kBuf16;
+            if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
+            halfx8 b0[4];
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) b0[cb] = *reinterpret_cast<const halfx8 *>(buf + boff + cb * 16 * kHalfRow);
+#pragma unroll
+            for (int rb = 0; rb < 8; ++rb) {
+                const halfx8 a0 = *reinterpret_cast<const halfx8 *>(buf + aoff + rb * 16 * kHalfRow);
+#pragma unroll
+                for (int cb = 0; cb < 4; ++cb)
+                    acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b0[cb], acc[rb][cb], 0, 0, 0);
+            }
+            if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
+        }
+        at = at + 1 == kRing16 ? 0 : at + 1;
+        to = to + 1 == kRing16 ? 0 : to + 1;
+    }
+    __syncthreads();  // a caller may start the next item on the same LDS
+    if (own > 0) write_partial(acc, w, out, rows, cols, tri, lane);
 }
 
 // One work item over the K blocks [b_begin, b_end): LDS rows
@@ -416,11 +423,15 @@ __host__ __device__ inline int tri_items_per_slab(int count) {
 // with a barrier, so a caller may start the next item on the same LDS.
 // VAR: 0 = direct-to-LDS loads, 1 = loads staged through registers,
 // 2 = direct-to-LDS loads and raised wave priority over the MFMA block.
-template <int FMT, int VAR>
+// SPLIT (direct loads): an item of w.ks slabs of kcb blocks from b_begin on,
+// cut at nkb = b_end; quarter k is read at slab w.kq[k], a wave stops where
+// its own slab (w.kw) ends.
+template <int FMT, int VAR, bool SPLIT>
 __device__ __forceinline__ void gram_item(const uint8_t *__restrict__ blocks, int64_t cap_bytes, int first, int count,
                                           int first_b, int count_b, const ItemWaves &w, int64_t b_begin,
-                                          int64_t b_end, float *__restrict__ out, uint8_t *lds,
-                                          int tid = threadIdx.x) {
+                                          int64_t b_end, int64_t kcb, float *__restrict__ out, int rows, int cols,
+                                          bool tri, uint8_t *lds, int tid = threadIdx.x) {
+    static_assert(!SPLIT || VAR != 1, "gram_item: the slab-split form loads directly");
     constexpr bool kSplit = FMT == PRNU_PREC_SPLIT_BF16;
     constexpr bool kFp8 = FMT == PRNU_PREC_FP8;
     constexpr bool kF16 = FMT == PRNU_PREC_FP16;
@@ -480,15 +491,22 @@ __device__ __forceinline__ void gram_item(const uint8_t *__restrict__ blocks, in
     }
     auto load_to = [&](int64_t b, uint8_t *buf) {
         if constexpr (DMA) {
-            const __amdgpu_buffer_rsrc_t rsrc =
-                __builtin_amdgcn_make_buffer_rsrc((void *)(blocks + b * cap_bytes), 0, (int)cap_bytes, 0x00020000);
             const int wbase = (tid >> 6) * 8;  // first row of this wave within a 64-row group
+            if constexpr (SPLIT) {  // each quarter from its own slab's block column
 #pragma unroll
-            for (int it = 0; it < 8; ++it) {
-                if (it < 4 || !half) {
-                    typedef __attribute__((address_space(3))) void *lptr;
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr)(buf + (64 * it + wbase) * kBlkBytes), 16,
-                                                             voff[it], 0, 0, 0);
+                for (int k = 0; k < 4; ++k) {
+                    const int64_t col = min(b + w.kq[k] * kcb, b_end - 1);
+#pragma unroll
+                    for (int it = 2 * k; it < 2 * k + 2; ++it)
+                        lds_fill16(blocks + col * cap_bytes, (int)cap_bytes, buf + (64 * it + wbase) * kBlkBytes,
+                                   voff[it]);
+                }
+            } else {
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    if (it < 4 || !half)
+                        lds_fill16(blocks + b * cap_bytes, (int)cap_bytes, buf + (64 * it + wbase) * kBlkBytes,
+                                   voff[it]);
                 }
             }
         } else {
@@ -646,14 +664,16 @@ __device__ __forceinline__ void gram_item(const uint8_t *__restrict__ blocks, in
         }
     };
 
-    const int64_t nst = b_end - b_begin;
+    // stages of the item and of this wave's own slab
+    const int64_t nst = SPLIT ? min(kcb, b_end - b_begin) : b_end - b_begin;
+    const int64_t own = SPLIT ? min(kcb, b_end - b_begin - w.kw * kcb) : nst;
     load_to(b_begin, lds);
     store(lds);
     __syncthreads();
     for (int64_t q = 0; q < nst; ++q) {
         const bool next = q + 1 < nst;
         if (next) load_to(b_begin + q + 1, lds + ((q + 1) & 1) * kBufS);
-        if (active) {
+        if (active && (!SPLIT || q < own)) {
             if constexpr (kPrio) __builtin_amdgcn_s_setprio(1);
             compute(lds + (q & 1) * kBufS);
             if constexpr (kPrio) __builtin_amdgcn_s_setprio(0);
@@ -662,37 +682,19 @@ __device__ __forceinline__ void gram_item(const uint8_t *__restrict__ blocks, in
         __syncthreads();
     }
 
-    if (!active) return;
-    const int ocol = lane & 15, orow = (lane >> 4) * 4;
-#pragma unroll
-    for (int rb = 0; rb < 8; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                out[(rb * 16 + orow + r) * kTileS + cb * 16 + ocol] = acc[rb][cb][r];
+    if (!active || own <= 0) return;
+    write_partial(acc, w, out, rows, cols, tri, lane);
 }
 
-// Run item u of slab s: partial tile t of slab s lives at partials + (t*S + s) * 256*256.
-// ntb > 0: a rectangle of nt x ntb tiles between slots [first, first+count)
-// (rows) and [first_b, first_b+count_b) (columns), item u = tile
-// (u / ntb, u % ntb); ntb == 0: the triangle of [first, first+count).
-__device__ __forceinline__ ItemWaves rect_waves(int u, int ntb, int wave) {
-    ItemWaves r;
-    const int wr = wave >> 2, wc = wave & 3;
-    item_tiles(r, u / ntb, u - (u / ntb) * ntb);
-    r.nq = 4;
-    r.a_off = wr * 128;
-    r.b_off = kTileS + wc * 64;
-    r.out_tile = u;
-    r.out_off = wr * 128 * kTileS + wc * 64;
-    return r;
-}
-
+// Item u of slab s: partial tile t of slab s lives at partials +
+// (t*S + s) * 256*256.  ntb > 0: the rectangle of slots [first, first+count)
+// (rows) and [first_b, first_b+count_b) (columns); ntb == 0: the triangle of
+// [first, first+count).
 template <int FMT, int VAR>
 __device__ __forceinline__ void run_item(const uint8_t *blocks, int64_t cap_bytes, int first, int count, int first_b,
                                          int count_b, int ntb, int S, int64_t nkb, int64_t kcb,
                                          float *partials, int u, int s, uint8_t *lds, int tid = threadIdx.x) {
+    constexpr bool kRing = FMT == PRNU_PREC_FP16 && VAR != 1;
     // wave-uniform: keep it in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     ItemWaves w = ntb > 0 ? rect_waves(u, ntb, wave) : item_waves(u, count, wave);
@@ -703,11 +705,31 @@ __device__ __forceinline__ void run_item(const uint8_t *blocks, int64_t cap_byte
     w.b_off = __builtin_amdgcn_readfirstlane(w.b_off >> 6) << 6;  // term (row & 7) stays per lane
     w.out_tile = __builtin_amdgcn_readfirstlane(w.out_tile);
     w.out_off = __builtin_amdgcn_readfirstlane(w.out_off);
+    w.ks = __builtin_amdgcn_readfirstlane(w.ks);
+    w.kw = __builtin_amdgcn_readfirstlane(w.kw);
     const int64_t b_begin = (int64_t)s * kcb;
+    float *out = w.out_tile < 0
+                     ? nullptr
+                     : partials + ((int64_t)w.out_tile * S + s + w.kw) * (kTileS * kTileS) + w.out_off;
+    const int rows = count - row_pattern(w, w.a_off), cols = count_b - row_pattern(w, w.b_off);
+    if (w.ks > 1) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w.kq[k] = __builtin_amdgcn_readfirstlane(w.kq[k]);
+        if constexpr (kRing)
+            gram_item_fp16<true, VAR == 2>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, nkb, kcb,
+                                           out, rows, cols, true, lds, tid);
+        else
+            gram_item<FMT, VAR == 1 ? 0 : VAR, true>(blocks, cap_bytes, first, count, first_b, count_b, w,
+                                                     b_begin, nkb, kcb, out, rows, cols, true, lds, tid);
+        return;
+    }
     const int64_t b_end = min(nkb, b_begin + kcb);
-    float *out = w.out_tile < 0 ? nullptr
-                                : partials + ((int64_t)w.out_tile * S + s) * (kTileS * kTileS) + w.out_off;
-    gram_item<FMT, VAR>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, b_end, out, lds, tid);
+    if constexpr (kRing)
+        gram_item_fp16<false, VAR == 2>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, b_end, kcb, out,
+                                        rows, cols, ntb == 0, lds, tid);
+    else
+        gram_item<FMT, VAR, false>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, b_end, kcb, out,
+                                   rows, cols, ntb == 0, lds, tid);
 }
 
 // ------------------------------------------------ 4-wave split-BF16 item
@@ -812,16 +834,11 @@ __global__ __launch_bounds__(kThr4, 1) void store_gram4_kernel(StoreGramArgs a) 
     for (int it = 0; it < 16; ++it) voff[it] = row_off(it) + (uint32_t)(dchunk << 4);
     const int wbase = (tid >> 6) * 8;
     auto load_to = [&](int64_t b, uint8_t *buf) {
-        __amdgpu_buffer_rsrc_t rsrc =
-            __builtin_amdgcn_make_buffer_rsrc((void *)(a.blocks + b * a.cap_bytes), (short)0,
-                                              (int)(a.cap_bytes), 0x00020000);
 #pragma unroll
         for (int it = 0; it < 16; ++it) {
-            if (it < 8 || !half) {
-                typedef __attribute__((address_space(3))) void *lptr;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr)(buf + (32 * it + wbase) * kBlkBytes), 16,
-                                                         voff[it], 0, 0, 0);
-            }
+            if (it < 8 || !half)
+                lds_fill16(a.blocks + b * a.cap_bytes, (int)a.cap_bytes, buf + (32 * it + wbase) * kBlkBytes,
+                           voff[it]);
         }
     };
 
@@ -950,18 +967,9 @@ __global__ __launch_bounds__(kThr4, 1) void store_gram4_kernel(StoreGramArgs a) 
 // a slab run on one XCD (workgroup ids are dealt to the 8 XCDs round-robin).
 template <int FMT, int VAR>
 __global__ __launch_bounds__(kThrS, 1) void store_gram_kernel(StoreGramArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBufS];
-    const int bid = blockIdx.x;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[item_lds<FMT, VAR>()];
     int u, s;
-    if (a.xcd_remap) {
-        const int local = bid >> 3;
-        u = local % a.T;
-        s = (local / a.T) * 8 + (bid & 7);
-    } else {
-        u = bid % a.T;
-        s = bid / a.T;
-    }
-    if (s >= a.S) return;
+    if (!ItemIndex(a.T, a.ks, a.S).at(blockIdx.x, a.xcd_remap, u, s)) return;
     run_item<FMT, VAR>(a.blocks, a.cap_bytes, a.first, a.count, a.first, a.count, 0, a.S, a.nkb, a.kcb,
                        a.partials, u, s, lds);
 }
@@ -969,9 +977,8 @@ __global__ __launch_bounds__(kThrS, 1) void store_gram_kernel(StoreGramArgs a) {
 // ------------------------------------------------------------ grouped plan
 // Several pattern groups (each all-pairs within itself) in one launch over
 // their concatenated work-item lists.  Group g (T items per slab) owns the
-// virtual ids [v_begin, v_begin + T*S8), with S8 = S rounded up to 8 and
-// v_begin a multiple of 8; id v maps to item ((v - v_begin) >> 3) % T and slab
-// ((v - v_begin) >> 3) / T * 8 + (v & 7).  Every slab has the same number of
+// virtual ids from v_begin (a multiple of 8) on, mapped by ItemIndex with the
+// slabs of a round on different XCDs.  Every slab has the same number of
 // K blocks in every group, so all items cost the same; the dispatcher hands
 // workgroups to CUs in id order as they free up, which is the work queue.
 // v & 7 is the XCD, so the T items of a slab share that XCD's L2.
@@ -981,12 +988,13 @@ struct GroupDev {
     int64_t cap_bytes, nkb, kcb, v_begin;
     int first, count, nt, T, S;
     int first_b, count_b, ntb;  // ntb > 0: rectangle rows x [first_b, first_b+count_b)
+    int ks;                     // slab_split of a triangle, 1 for a rectangle
 };
 
 template <int FMT, int VAR>
 __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_kernel(const GroupDev *__restrict__ groups,
                                                                     int ngroups) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBufS];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[item_lds<FMT, VAR>()];
     const int64_t v = blockIdx.x;
     int lo = 0, hi = ngroups - 1;  // last group with v_begin <= v
     while (lo < hi) {
@@ -995,11 +1003,8 @@ __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_kernel(const Group
         else hi = mid - 1;
     }
     const GroupDev &g = groups[lo];
-    const int64_t vl = v - g.v_begin;
-    const int local = (int)(vl >> 3);
-    const int u = local % g.T;
-    const int s = (local / g.T) * 8 + (int)(vl & 7);
-    if (s >= g.S) return;  // padding item
+    int u, s;
+    if (!ItemIndex(g.T, g.ks, g.S).at(v - g.v_begin, true, u, s)) return;  // padding item
     run_item<FMT, VAR>(g.blocks, g.cap_bytes, g.first, g.count, g.first_b, g.count_b, g.ntb, g.S, g.nkb,
                        g.kcb, g.partials, u, s, lds);
 }
@@ -1028,7 +1033,7 @@ template <int FMT>
 __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_persistent_kernel(const GroupDev *__restrict__ groups,
                                                                                int ngroups, int64_t v_total,
                                                                                int *__restrict__ queue) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBufS];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[item_lds<FMT, 0>()];
     int *taken = reinterpret_cast<int *>(lds);
     const int x = blockIdx.x & 7;
     for (;;) {
@@ -1044,11 +1049,8 @@ __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_persistent_kernel(
             else hi = mid - 1;
         }
         const GroupDev &g = groups[lo];
-        const int64_t vl = v - g.v_begin;
-        const int local = (int)(vl >> 3);
-        const int u = local % g.T;
-        const int s = (local / g.T) * 8 + (int)(vl & 7);
-        if (s >= g.S) continue;  // padding item (uniform across the workgroup)
+        int u, s;
+        if (!ItemIndex(g.T, g.ks, g.S).at(v - g.v_begin, true, u, s)) continue;  // padding item (uniform)
         // the thread id is opaque per item, so its address terms are not
         // hoisted out of this loop (they would stay live across every item)
         int tid = threadIdx.x;
@@ -1061,22 +1063,40 @@ __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_persistent_kernel(
 __global__ void store_queue_reset_kernel(int *queue) { queue[threadIdx.x] = 0; }
 
 // FP64 sum of the S partials + NCC epilogue (normalizedcrosscorrelation.cu:121-123).
-// Four consecutive elements of a partial tile per thread: one 16-byte load
-// per slab, four FP64 sums, each in slab order (the same order as one
-// element per thread, so the results do not depend on this grouping).
-// grid (kTileS * kTileS / 1024, tiles), 256 threads.
-__device__ __forceinline__ void sum_slabs4(const float *__restrict__ p, int S, double g[4]) {
+// A block takes 128 consecutive elements of a partial tile, 4 per thread (one
+// 16-byte load per slab); its 8 groups of 32 threads sum every 8th slab, and
+// the 8 sums are added in a fixed order, the same for triangles and
+// rectangles.  One group for all slabs left a set of few patterns with too few
+// loads in flight (three sets of 500, 300 and 120 patterns: 93 us each; now
+// 9 to 25 us with up to three times the slabs).
+// grid (kTileS * kTileS / 128, tiles), 256 threads.
+constexpr int kRedGroups = 8;
+
+__device__ __forceinline__ bool sum_slabs4(const float *__restrict__ p, int S, double (*sh)[32][4], double g[4]) {
+    const int grp = threadIdx.x >> 5, l = threadIdx.x & 31;
     g[0] = g[1] = g[2] = g[3] = 0.0;
     const float4 *q4 = reinterpret_cast<const float4 *>(p);
     constexpr int kStride = kTileS * kTileS / 4;
 #pragma unroll 8
-    for (int q = 0; q < S; ++q) {
+    for (int q = grp; q < S; q += kRedGroups) {
         const float4 v = q4[(int64_t)q * kStride];
         g[0] += (double)v.x;
         g[1] += (double)v.y;
         g[2] += (double)v.z;
         g[3] += (double)v.w;
     }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) sh[grp][l][c] = g[c];
+    __syncthreads();
+    if (grp) return false;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        double t[kRedGroups];
+#pragma unroll
+        for (int k = 0; k < kRedGroups; ++k) t[k] = sh[k][l][c];
+        g[c] = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+    }
+    return true;
 }
 
 __global__ __launch_bounds__(256) void store_reduce_kernel(const float *__restrict__ partials, int S, int nt,
@@ -1084,15 +1104,19 @@ __global__ __launch_bounds__(256) void store_reduce_kernel(const float *__restri
                                                            const double *__restrict__ sumsq,
                                                            const float *__restrict__ scale,
                                                            double *__restrict__ out, int64_t ld) {
+    __shared__ double sh[kRedGroups][32][4];
     const int t = blockIdx.y;
-    const int e = (blockIdx.x * 256 + threadIdx.x) * 4;
-    const int2 tile = tri_tile_s(t, nt);
-    const int i = tile.x * kTileS + (e >> 8);
+    const int e = (blockIdx.x * 32 + (threadIdx.x & 31)) * 4;
+    const int2 tile = tri_tile(t, nt);
+    const int i = tile.x * kTileS + (e >> 8);  // the same row for the whole block
     const int j0 = tile.y * kTileS + (e & 255);
-    if (i >= count || j0 >= count) return;
-    if (tile.x == tile.y && i > j0 + 3) return;
+    const int jb = j0 & ~127, je = jb + 127;   // the block's columns
+    if (i >= count || jb >= count || i > je) return;
+    const bool mine = j0 < count && !(tile.x == tile.y && i > j0 + 3);
     double g[4];
-    sum_slabs4(partials + (int64_t)t * S * (kTileS * kTileS) + e, S, g);
+    // threads past the set's end or below the diagonal read what the block's first needed thread reads
+    const int eo = mine ? e : (e & ~255) + (max(jb, min(i, je)) & 252 & 255);
+    if (!sum_slabs4(partials + (int64_t)t * S * (kTileS * kTileS) + eo, S, sh, g) || !mine) return;
     const double di = sqrt(sumsq[i] - sum[i] * sum[i]);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -1118,14 +1142,16 @@ __global__ __launch_bounds__(256) void store_reduce_rect_kernel(const float *__r
                                                                 const float *__restrict__ scale_a,
                                                                 const float *__restrict__ scale_b,
                                                                 double *__restrict__ out, int64_t ld) {
+    __shared__ double sh[kRedGroups][32][4];
     const int t = blockIdx.y;
-    const int e = (blockIdx.x * 256 + threadIdx.x) * 4;
+    const int e = (blockIdx.x * 32 + (threadIdx.x & 31)) * 4;
     const int I = t / ntb, J = t - (t / ntb) * ntb;
     const int i = I * kTileS + (e >> 8);
     const int j0 = J * kTileS + (e & 255);
-    if (i >= count_a || j0 >= count_b) return;
+    if (i >= count_a || (j0 & ~127) >= count_b) return;
+    const int eo = j0 < count_b ? e : e & ~127;  // past the end: the block's first column
     double g[4];
-    sum_slabs4(partials + (int64_t)t * S * (kTileS * kTileS) + e, S, g);
+    if (!sum_slabs4(partials + (int64_t)t * S * (kTileS * kTileS) + eo, S, sh, g)) return;
     const double di = sqrt(sumsq_a[i] - sum_a[i] * sum_a[i]);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -1149,6 +1175,14 @@ int block_values(int format) {
 // diagonal packs of 4 blocks (item_waves4).
 int items_per_slab4(int nt) { return nt * (nt - 1) / 2 + (3 * nt + 3) / 4; }
 
+int launch_tri_reduce(const float *partials, int S, int nt, int count, const double *sum, const double *sumsq,
+                      const float *scale, double *out, int64_t ld, hipStream_t st) {
+    hipLaunchKernelGGL(store_reduce_kernel, dim3(kTileS * kTileS / 128, nt * (nt + 1) / 2), dim3(256), 0, st,
+                       partials, S, nt, count, sum, sumsq, scale, out, ld);
+    PRNU_CHECK_LAUNCH();
+    return PRNU_OK;
+}
+
 int device_cus(int device) {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 256;
@@ -1159,17 +1193,22 @@ int device_cus(int device) {
 // cost about kcb block-stages and one CU runs one item at a time, so the
 // launch takes about ceil(items / cus) * kcb stages, plus a per-slab cost
 // (the partial tile each item writes and the reduction reads, ~2 stages).
+// splits[g]: the slabs the last item of group g takes at once (slab_split).
 // Searches kcb and returns the cheapest whose partial tiles fit `max_bytes`.
-int64_t choose_kcb(const int *items, const int *tiles, const int64_t *nkb, int ngroups, int cus, size_t max_bytes) {
+// `longest` (if > 0) bounds the slab: an FP32 accumulator's rounding error
+// grows with it.
+int64_t choose_kcb(const int *items, const int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
+                   size_t max_bytes, int64_t longest) {
     int64_t max_nkb = 1;
     for (int g = 0; g < ngroups; ++g) max_nkb = std::max(max_nkb, nkb[g]);
     double best = 1e300;
+    if (longest > 0) max_nkb = std::min(max_nkb, longest);
     int64_t best_kcb = max_nkb;
-    for (int64_t kcb = 16; kcb <= max_nkb; kcb += (kcb < 256 ? 8 : kcb < 2048 ? 32 : 256)) {
+    for (int64_t kcb = std::min<int64_t>(16, max_nkb); kcb <= max_nkb; kcb += (kcb < 256 ? 8 : kcb < 2048 ? 32 : 256)) {
         double total = 0.0, part = 0.0;
         for (int g = 0; g < ngroups; ++g) {
             const int64_t S = (nkb[g] + kcb - 1) / kcb;
-            total += (double)items[g] * S;
+            total += (double)ItemIndex(items[g], splits[g], (int)std::min<int64_t>(S, 1 << 30)).items();
             part += (double)tiles[g] * S * kTileS * kTileS * sizeof(float);
         }
         if (part > (double)max_bytes) continue;
@@ -1181,6 +1220,16 @@ int64_t choose_kcb(const int *items, const int *tiles, const int64_t *nkb, int n
         }
     }
     return best_kcb;
+}
+
+// The slab of a set of triangles and rectangles: no longer than the cheapest
+// one with every item taking one slab at a time, so that items of several
+// slabs shorten the launch and not the sums' precision.
+int64_t choose_slab(const int *items, const int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
+                    size_t max_bytes) {
+    const std::vector<int> one(ngroups, 1);
+    const int64_t longest = choose_kcb(items, one.data(), tiles, nkb, ngroups, cus, max_bytes, 0);
+    return choose_kcb(items, splits, tiles, nkb, ngroups, cus, max_bytes, longest);
 }
 
 int store_create(int64_t n, int capacity, int format, Store **out) {
@@ -1299,6 +1348,7 @@ int store_gram_ncc(Context *c, Store *s, int first, int count, double *d_ncc, hi
     const int var = cfg.variant;  // 0 direct-to-LDS, 1 register-staged, 2 + priority, 3 four waves (not FP32)
     const bool four = var == 3 && s->format != PRNU_PREC_FP32;
     a.T = four ? items_per_slab4(a.nt) : tri_items_per_slab(count);
+    a.ks = four ? 1 : slab_split(count);
     const int tiles = a.nt * (a.nt + 1) / 2;  // partial tiles per slab (triangle incl. diagonal)
     const int64_t tile_bytes = (int64_t)kTileS * kTileS * sizeof(float);
     if (cfg.slabs > 0) {
@@ -1307,14 +1357,13 @@ int store_gram_ncc(Context *c, Store *s, int first, int count, double *d_ncc, hi
         a.kcb = (s->nkb + S - 1) / S;
     } else {
         const int64_t nkb = s->nkb;
-        a.kcb = choose_kcb(&a.T, &tiles, &nkb, 1, device_cus(c->device), size_t(2) << 30);
+        a.kcb = choose_slab(&a.T, &a.ks, &tiles, &nkb, 1, device_cus(c->device), size_t(2) << 30);
     }
     a.S = (int)((s->nkb + a.kcb - 1) / a.kcb);
     a.xcd_remap = cfg.xcd_remap;
     PRNU_TRY(c->ws_gram.ensure((size_t)tile_bytes * tiles * a.S));
     a.partials = static_cast<float *>(c->ws_gram.ptr);
-    const int64_t S8 = a.xcd_remap ? (a.S + 7) / 8 * 8 : a.S;
-    const dim3 grid((unsigned)(a.T * S8));
+    const dim3 grid((unsigned)ItemIndex(a.T, a.ks, a.S).ids(a.xcd_remap));
     time_begin(c, st);
     if (four) {
         if (s->format == PRNU_PREC_FP8)
@@ -1325,11 +1374,8 @@ int store_gram_ncc(Context *c, Store *s, int first, int count, double *d_ncc, hi
             hipLaunchKernelGGL(store_gram4_kernel<PRNU_PREC_SPLIT_BF16>, grid, dim3(kThr4), 0, st, a);
         PRNU_CHECK_LAUNCH();
         time_end(c, st);
-        hipLaunchKernelGGL(store_reduce_kernel, dim3(kTileS * kTileS / 1024, tiles), dim3(256), 0, st, a.partials,
-                           a.S, a.nt, count, s->sum + first, s->sumsq + first, s->scale ? s->scale + first : nullptr,
-                           d_ncc, (int64_t)count);
-        PRNU_CHECK_LAUNCH();
-        return PRNU_OK;
+        return launch_tri_reduce(a.partials, a.S, a.nt, count, s->sum + first, s->sumsq + first,
+                                 s->scale ? s->scale + first : nullptr, d_ncc, (int64_t)count, st);
     }
 #define PRNU_STORE_GRAM(F)                                                                        \
     do {                                                                                          \
@@ -1351,11 +1397,8 @@ int store_gram_ncc(Context *c, Store *s, int first, int count, double *d_ncc, hi
 #undef PRNU_STORE_GRAM
     PRNU_CHECK_LAUNCH();
     time_end(c, st);
-    hipLaunchKernelGGL(store_reduce_kernel, dim3(kTileS * kTileS / 1024, tiles), dim3(256), 0, st, a.partials, a.S,
-                       a.nt, count, s->sum + first, s->sumsq + first, s->scale ? s->scale + first : nullptr, d_ncc,
-                       (int64_t)count);
-    PRNU_CHECK_LAUNCH();
-    return PRNU_OK;
+    return launch_tri_reduce(a.partials, a.S, a.nt, count, s->sum + first, s->sumsq + first,
+                             s->scale ? s->scale + first : nullptr, d_ncc, (int64_t)count, st);
 }
 
 // ------------------------------------------------------------ grouped plan
@@ -1370,6 +1413,7 @@ struct PlanBlock {
     int nta() const { return (row_count + kTileS - 1) / kTileS; }
     int ntb() const { return (col_count + kTileS - 1) / kTileS; }
     int items() const { return tri ? tri_items_per_slab(row_count) : nta() * ntb(); }
+    int split() const { return tri ? slab_split(row_count) : 1; }
     int tiles() const { return tri ? nta() * (nta() + 1) / 2 : nta() * ntb(); }
 };
 
@@ -1432,8 +1476,9 @@ int plan_layout(GramPlan *p, int64_t kcb) {
         d.S = (int)((s->nkb + d.kcb - 1) / d.kcb);
         d.v_begin = v;
         d.partials = reinterpret_cast<float *>((uintptr_t)part);  // offset for now
-        v += (int64_t)d.T * ((d.S + 7) / 8 * 8);
-        items += (int64_t)d.T * d.S;
+        d.ks = g.split();
+        v += ItemIndex(d.T, d.ks, d.S).ids(true);
+        items += ItemIndex(d.T, d.ks, d.S).items();
         part += tile_elems * sizeof(float) * g.tiles() * d.S;
     }
     PRNU_REQUIRE(v < (int64_t(1) << 31), "gram_plan: %lld work items; use longer slabs", (long long)v);
@@ -1466,14 +1511,16 @@ int plan_layout(GramPlan *p, int64_t kcb) {
 
 // Default slab: the cheapest by the rounds model of choose_kcb.
 int64_t plan_default_kcb(const GramPlan *p) {
-    std::vector<int> items, tiles;
+    std::vector<int> items, splits, tiles;
     std::vector<int64_t> nkb;
     for (const PlanBlock &g : p->groups) {
         items.push_back(g.items());
+        splits.push_back(g.split());
         tiles.push_back(g.tiles());
         nkb.push_back(g.store->nkb);
     }
-    return choose_kcb(items.data(), tiles.data(), nkb.data(), (int)items.size(), p->cus, kPlanPartialCap);
+    return choose_slab(items.data(), splits.data(), tiles.data(), nkb.data(), (int)items.size(), p->cus,
+                       kPlanPartialCap);
 }
 
 // Persistent launch: one workgroup per CU, a multiple of 8 so blockIdx.x & 7
@@ -1517,11 +1564,10 @@ int plan_launch(GramPlan *p, hipStream_t st) {
         const PlanBlock &g = p->groups[i];
         const Store *s = g.store;
         if (g.tri) {
-            hipLaunchKernelGGL(store_reduce_kernel, dim3(kTileS * kTileS / 1024, g.tiles()), dim3(256), 0, st,
-                               d.partials, d.S, d.nt, d.count, s->sum + d.first, s->sumsq + d.first,
-                               s->scale ? s->scale + d.first : nullptr, g.out, g.ld);
+            PRNU_TRY(launch_tri_reduce(d.partials, d.S, d.nt, d.count, s->sum + d.first, s->sumsq + d.first,
+                                       s->scale ? s->scale + d.first : nullptr, g.out, g.ld, st));
         } else {
-            hipLaunchKernelGGL(store_reduce_rect_kernel, dim3(kTileS * kTileS / 1024, g.tiles()), dim3(256), 0, st,
+            hipLaunchKernelGGL(store_reduce_rect_kernel, dim3(kTileS * kTileS / 128, g.tiles()), dim3(256), 0, st,
                                d.partials, d.S, d.ntb, d.count, d.count_b, s->sum + d.first, s->sumsq + d.first,
                                s->sum + d.first_b, s->sumsq + d.first_b, s->scale ? s->scale + d.first : nullptr,
                                s->scale ? s->scale + d.first_b : nullptr, g.out, g.ld);

@@ -1,0 +1,70 @@
+"""The Gram kernels at the counts and lengths where their work items change
+form: one 128-pattern quarter (four slabs at once), three quarters (two), five
+(one), nine (four, in the second of two one-quarter items), a single short
+slab, ragged last slabs and K blocks.
+
+Tolerances against FP64: 1e-5 for FP32 and split-BF16 products; FP16 and FP8
+values are rounded once per element (relative 2^-11 and 2^-4, rms 0.29 and
+0.036 / 2^-4 of that), so an entry errs by that share of 1/sqrt(n) for
+unrelated patterns and of the entry for related ones: 6 sigma of sqrt(2) such
+roundings, with the diagonal's bias 2 * rms^2.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle import prnu_oracle as O  # noqa: E402
+from rocket_amd import _lib, csi  # noqa: E402
+from test_gpu_ncc import patterns  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def tolerance(fmt, n):
+    rms = {"fp16": 2.0 ** -11, "fp8": 0.04}.get(fmt)
+    return 1e-5 if rms is None else 6 * rms * np.sqrt(2.0 / n) * 2 + 2 * rms * rms + 1e-5
+
+
+@pytest.mark.parametrize("fmt", ["split_bf16", "fp32", "fp16", "fp8"])
+@pytest.mark.parametrize("count,h,w", [(1, 8, 9), (5, 20, 21), (120, 64, 67), (128, 100, 100), (300, 61, 50),
+                                       (384, 33, 64), (600, 40, 41), (1100, 30, 31)])
+def test_items(fmt, count, h, w):
+    p = patterns(count, h, w, 4, seed=900 + count, gain=0.3)
+    want = O.ncc_matrix(p.cpu().numpy())
+    tol = tolerance(fmt, h * w)
+    gram = csi.GramNCC(h, w)
+    store = csi.PatternStore(h * w, count + 2, fmt)
+    store.put(p, first_slot=2)
+    for slabs in (0, 1, 3, 7):
+        cfg = (ctypes.c_int32 * 3)(slabs, 1, 0)
+        _lib.call("prnu_gram_set_config", gram._ctx.handle, _lib.PRECISIONS[fmt], cfg)
+        got = store.gram(gram, count, 2).cpu().numpy()
+        assert np.abs(got - want).max() <= tol
+        assert np.array_equal(got, got.T)
+        if fmt != "fp16":
+            assert np.abs(gram.ncc(p, fmt).cpu().numpy() - want).max() <= tol
+    store.close()
+    gram.close()
+
+
+@pytest.mark.parametrize("slab_blocks", [1, 4, 9])
+def test_split_item_keeps_the_slabs(slab_blocks):
+    """The same slabs give the same bits whether a pair lies in a set of one
+    quarter (four slabs at once) or of two (one at a time)."""
+    h, w, n = 40, 44, 40 * 44
+    p = patterns(200, h, w, 4, seed=77, gain=0.3)
+    gram = csi.GramNCC(h, w)
+    store = csi.PatternStore(n, 200, "split_bf16")
+    store.put(p)
+    plans = [csi.GramPlan(gram, [(store, 0, c)], slab_values=32 * slab_blocks) for c in (100, 200)]
+    small, large = (pl.run()[0].cpu().numpy() for pl in plans)
+    assert np.array_equal(small, large[:100, :100])
+    plans[0].persistent = True
+    assert np.array_equal(plans[0].run()[0].cpu().numpy(), small)
+    for pl in plans:
+        pl.close()
+    store.close()
+    gram.close()
