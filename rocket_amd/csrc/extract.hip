@@ -13,16 +13,15 @@
 //   SpectralFilter.java:44-54     R2C FFT2, h x (w/2+1)
 //
 // Layout in HBM: images and patterns are row-major h x w FP32.  The Wiener
-// filter runs its row FFTs in LDS (one row per workgroup), then its column
-// FFTs: for columns up to 1024 long, in LDS over strips of >= 4 adjacent
-// columns read row by row (no transpose, variance stencil in the natural
-// layout); for longer columns through a transpose (w x h) so they are LDS row
-// FFTs, the stencil in that transposed domain (the zero-padded box-min is
-// transpose invariant), and a transpose back.  It ends with the inverse row
-// FFTs.
+// filter runs its row FFTs in LDS (two rows per workgroup), then its column
+// FFTs over strips of adjacent columns through LDS (cols.hip), whose results
+// leave transposed (w x h); the variance stencil works in that transposed
+// domain (the zero-padded box-min is transpose invariant), the inverse column
+// pass writes row-major again, and the inverse row FFTs end it.
 #include "prnu_internal.hpp"
 #include "fft_device.hpp"
 #include "fft_host.hpp"
+#include "cols_host.hpp"
 
 #include <algorithm>
 
@@ -626,18 +625,16 @@ __global__ __launch_bounds__(256) void zm_apply_kernel(float *img_all, int64_t i
 // sums from the same two bins.  No row sums are taken before the transform
 // (32 frames of 2048x1536: 304 -> 275 us, two loads and two subtractions less
 // per value pair).
-// PAD2048: rows of 2048 by fft_block_2048_r8 (LDS kFft2048PadLds values).
-template <int MAXN, bool PAD2048 = false, bool ZM_EVEN = false>
-__global__ __launch_bounds__(kFftThreads) void wiener_rows_fwd_kernel(FftDesc d, const float *img_all,
-                                                                      int64_t img_stride, int h, float2 *A_all,
-                                                                      int64_t plane, double *rowsq_all,
-                                                                      const float *cz_all, const float *rz_all,
-                                                                      int lda) {
+template <class R, bool ZM_EVEN>
+__global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float *img_all, int64_t img_stride, int h,
+                                                               float2 *A_all, int64_t plane, double *rowsq_all,
+                                                               const float *cz_all, const float *rz_all, int lda) {
     extern __shared__ float2 buf[];
-    __shared__ double sh[8];
+    constexpr int T = R::T, NW = T / 64;
+    __shared__ double sh[2][NW];
     const int i0 = 2 * blockIdx.x, i1 = i0 + 1, b = blockIdx.y;
     const bool two = i1 < h;
-    const int w = d.n, wh = w / 2 + 1;
+    const int w = pl.n(), wh = w / 2 + 1;
     const float *img = img_all + (int64_t)b * img_stride;
     const bool zm = ZM_EVEN || cz_all != nullptr;
     // rows i0 (even) and i1 (odd): column terms of parities 0 and 1
@@ -664,12 +661,9 @@ __global__ __launch_bounds__(kFftThreads) void wiener_rows_fwd_kernel(FftDesc d,
             return make_float2(va, vb);
         };
     auto put = [&](int j, float2 f) { buf[j] = f; };  // the last pass has read buf before it writes
-    if constexpr (PAD2048)
-        fft_block_2048_r8<-1>(buf, d.tw, get, put);
-    else
-        fft_row<-1, MAXN>(buf, d, get, put);
+    pl.template run<-1>(buf, get, put);
     float2 *a0 = A_all + (int64_t)b * plane + (int64_t)i0 * lda;  // rows lda values apart
-    for (int k = threadIdx.x; k < wh; k += kFftThreads) {
+    for (int k = threadIdx.x; k < wh; k += T) {
         const float2 zk = buf[k], zm_ = buf[k == 0 ? 0 : w - k];
         float2 fa = make_float2(0.5f * (zk.x + zm_.x), 0.5f * (zk.y - zm_.y));
         float2 fb = make_float2(0.5f * (zk.y + zm_.y), -0.5f * (zk.x - zm_.x));
@@ -681,12 +675,17 @@ __global__ __launch_bounds__(kFftThreads) void wiener_rows_fwd_kernel(FftDesc d,
     sq0 = wave_sum_d(sq0);
     sq1 = wave_sum_d(sq1);
     if ((threadIdx.x & 63) == 0) {
-        sh[threadIdx.x >> 6] = sq0;
-        sh[4 + (threadIdx.x >> 6)] = sq1;
+        sh[0][threadIdx.x >> 6] = sq0;
+        sh[1][threadIdx.x >> 6] = sq1;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double s0 = (sh[0] + sh[1]) + (sh[2] + sh[3]), s1 = (sh[4] + sh[5]) + (sh[6] + sh[7]);
+        double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+        for (int k = 0; k < NW; k += 4) {
+            s0 += (sh[0][k] + sh[0][k + 1]) + (sh[0][k + 2] + sh[0][k + 3]);
+            s1 += (sh[1][k] + sh[1][k + 1]) + (sh[1][k + 2] + sh[1][k + 3]);
+        }
         if (ZM_EVEN) {
             // Z_0 = Se + So, Z_{w/2} = Se - So (row i0 the real, i1 the imaginary parts):
             // Se^2 + So^2 = (Z_0^2 + Z_{w/2}^2) / 2
@@ -721,24 +720,16 @@ __global__ __launch_bounds__(256) void wiener_var_kernel(const double *rowsq_all
 // differences, which would carry the rounding error of a large bin past its
 // window).  Tiles are numbered image by image, row by row, and dealt to the
 // XCDs in ranges as in fastnoise_kernel.  grid (8 * per)
-// P holds half of the power spectrum, which is symmetric, P(-k) = P(k):
-// MIRROR_ROWS, rows [0, rows/2] of length cols (full row r > rows/2 is row
-// rows - r reversed: P(r, c) = P(rows - r, (cols - c) % cols)); otherwise
-// all rows with columns [0, cols/2] (P(r, c) = P((rows - r) % rows, cols - c)
-// for c > cols/2).  S is written on the full rows x cols grid.
+// P holds half of the power spectrum, which is symmetric, P(-k) = P(k): rows
+// [0, rows/2] of length cols (full row r > rows/2 is row rows - r reversed:
+// P(r, c) = P(rows - r, (cols - c) % cols)).  S is written on the full rows x
+// cols grid.
 constexpr int kVX = 64, kVY = 128, kVB = 4, kVRows = 32;
-template <bool MIRROR_ROWS>
 __device__ __forceinline__ float power_full(const float *P, int r, int c, int rows, int cols) {
-    if (MIRROR_ROWS) {
-        if (r <= rows / 2) return P[(int64_t)r * cols + c];
-        return P[(int64_t)(rows - r) * cols + (c == 0 ? 0 : cols - c)];
-    }
-    const int ch = cols / 2 + 1;
-    if (c <= cols / 2) return P[(int64_t)r * ch + c];
-    return P[(int64_t)(r == 0 ? 0 : rows - r) * ch + (cols - c)];
+    if (r <= rows / 2) return P[(int64_t)r * cols + c];
+    return P[(int64_t)(rows - r) * cols + (c == 0 ? 0 : cols - c)];
 }
 
-template <bool MIRROR_ROWS>
 __global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, float *S_all, int rows, int cols,
                                                            const double *var_all, int ntx, int nty, int ntiles) {
     constexpr int LW = kVX + 2 * kVB, LH = kVY + 2 * kVB;
@@ -751,12 +742,12 @@ __global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, f
     const int64_t plane = (int64_t)rows * cols;
     const float *P = P_all + (int64_t)b * plane;
     float *S = S_all + (int64_t)b * plane;
-    // thread -> (LDS row, group of 4 columns): 18 groups per row.  In the
-    // transposed layout (MIRROR_ROWS) a group inside the grid is 4
+    // thread -> (LDS row, group of 4 columns): 18 groups per row.  A group
+    // inside the grid is 4
     // consecutive values of one source row -- forward (one 16-byte load when
     // cols is a multiple of 4: gx0 is) or backward in the mirrored half --
     // so only groups at the grid's edges take the per-value path.
-    const bool vec4 = MIRROR_ROWS && (cols & 3) == 0;
+    const bool vec4 = (cols & 3) == 0;
     for (int q = threadIdx.x; q < LH * (LW / 4); q += 256) {
         const int ly = q / (LW / 4), lx = (q - ly * (LW / 4)) * 4;
         const int gy = r0 + ly - kVB;
@@ -778,7 +769,7 @@ __global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, f
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int gx = gx0 + k;
-                e[k] = (gx >= 0 && gx < cols) ? power_full<MIRROR_ROWS>(P, gy, gx, rows, cols) : 0.f;
+                e[k] = (gx >= 0 && gx < cols) ? power_full(P, gy, gx, rows, cols) : 0.f;
             }
             val = make_float4(e[0], e[1], e[2], e[3]);
         }
@@ -822,18 +813,13 @@ __global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, f
     }
 }
 
-int launch_varest(const float *P, float *S, int rows, int cols, bool mirror_rows, int nb, const double *var,
-                  hipStream_t st) {
+int launch_varest(const float *P, float *S, int rows, int cols, int nb, const double *var, hipStream_t st) {
     const int ntx = (cols + kVX - 1) / kVX, nty = (rows + kVY - 1) / kVY;
     const int64_t ntiles = (int64_t)ntx * nty * nb;
     PRNU_REQUIRE(ntiles < (int64_t(1) << 30), "wiener: %lld variance tiles", (long long)ntiles);
     const int per = (int)((ntiles + 7) / 8);
-    if (mirror_rows)
-        hipLaunchKernelGGL(varest_scale_kernel<true>, dim3((unsigned)(8 * per)), dim3(256), 0, st, P, S, rows, cols,
-                           var, ntx, nty, (int)ntiles);
-    else
-        hipLaunchKernelGGL(varest_scale_kernel<false>, dim3((unsigned)(8 * per)), dim3(256), 0, st, P, S, rows, cols,
-                           var, ntx, nty, (int)ntiles);
+    hipLaunchKernelGGL(varest_scale_kernel, dim3((unsigned)(8 * per)), dim3(256), 0, st, P, S, rows, cols, var, ntx,
+                       nty, (int)ntiles);
     PRNU_CHECK_LAUNCH();
     return PRNU_OK;
 }
@@ -843,17 +829,13 @@ int launch_varest(const float *P, float *S, int rows, int cols, bool mirror_rows
 // imaginary parts of bins 0 and w/2 dropped, as a real transform does);
 // out = z / (w*h), row 2r the real, row 2r+1 the imaginary part
 // (normalizeToReal).  grid (ceil(h/2), B)
-// BLOCKN = 2048: rows of 2048 by the two-wave transform (fft_block_2048, 128
-// threads, LDS fft_wave_lds<2048>() values); 0: fft_row on kFftThreads.
-template <int MAXN, int BLOCKN = 0>
-__global__ __launch_bounds__(BLOCKN ? 128 : kFftThreads) void rows_c2r_kernel(FftDesc d, const float2 *A,
-                                                                              int64_t plane, int h, float *out_all,
-                                                                              int64_t out_stride, float inv_n,
-                                                                              int lda) {
+template <class R>
+__global__ __launch_bounds__(R::T) void rows_c2r_kernel(R pl, const float2 *A, int64_t plane, int h, float *out_all,
+                                                        int64_t out_stride, float inv_n, int lda) {
     extern __shared__ float2 buf[];
     const int i0 = 2 * blockIdx.x, i1 = i0 + 1;
     const bool two = i1 < h;
-    const int w = d.n;
+    const int w = pl.n();
     const float2 *a0 = A + (int64_t)blockIdx.y * plane + (int64_t)i0 * lda;  // rows lda values apart
     float *out = out_all + (int64_t)blockIdx.y * out_stride + (int64_t)i0 * w;
     auto get = [&](int k) {
@@ -874,312 +856,39 @@ __global__ __launch_bounds__(BLOCKN ? 128 : kFftThreads) void rows_c2r_kernel(Ff
         out[j] = z.x * inv_n;
         if (two) out[w + j] = z.y * inv_n;
     };
-    if constexpr (BLOCKN == 2048)
-        fft_block_2048<1>(buf, d.tw, get, put);
-    else
-        fft_row<1, MAXN>(buf, d, get, put);
+    pl.template run<1>(buf, get, put);
 }
 
 // ---------------------------------------------------------------- spectrum
 // Forward FFTs (length w) of real rows 2r and 2r+1 as one complex transform
 // (z = a + i b, split as in wiener_rows_fwd_kernel); the w/2+1 bins of each
 // row go to A (h x wh, rows wh apart).  grid (ceil(h/2), B)
-// PAD2048 as wiener_rows_fwd_kernel's.
-template <int MAXN, bool PAD2048 = false>
-__global__ __launch_bounds__(kFftThreads) void rows_fft_half_kernel(FftDesc d, const float *img_all,
-                                                                    int64_t img_stride, float2 *A, int64_t plane,
-                                                                    int h, int lda) {
+template <class R>
+__global__ __launch_bounds__(R::T) void rows_fft_half_kernel(R pl, const float *img_all, int64_t img_stride, float2 *A,
+                                                             int64_t plane, int h, int lda) {
     extern __shared__ float2 buf[];
     const int i0 = 2 * blockIdx.x, i1 = i0 + 1;
     const bool two = i1 < h;
-    const int w = d.n, wh = w / 2 + 1;
+    const int w = pl.n(), wh = w / 2 + 1;
     const float *r0 = img_all + (int64_t)blockIdx.y * img_stride + (int64_t)i0 * w;
     const float *r1 = two ? r0 + w : r0;
     auto get = [&](int j) { return make_float2(r0[j], two ? r1[j] : 0.f); };
     auto put = [&](int j, float2 f) { buf[j] = f; };  // the last pass has read buf before it writes
-    if constexpr (PAD2048)
-        fft_block_2048_r8<-1>(buf, d.tw, get, put);
-    else
-        fft_row<-1, MAXN>(buf, d, get, put);
+    pl.template run<-1>(buf, get, put);
     float2 *a0 = A + (int64_t)blockIdx.y * plane + (int64_t)i0 * lda;  // rows lda values apart
-    for (int k = threadIdx.x; k < wh; k += kFftThreads) {
+    for (int k = threadIdx.x; k < wh; k += R::T) {
         const float2 zk = buf[k], zm_ = buf[k == 0 ? 0 : w - k];
         a0[k] = make_float2(0.5f * (zk.x + zm_.x), 0.5f * (zk.y - zm_.y));
         if (two) a0[lda + k] = make_float2(0.5f * (zk.y + zm_.y), -0.5f * (zk.x - zm_.x));
     }
 }
 
-// ------------------------------------------- transposed-layout row kernels
-// Used when a column strip would be narrower than 4 columns (long columns):
-// the plane is transposed and columns become LDS row transforms.
-// In-place forward FFT of the rows of B (length d.n) and |F|^2 into P.
-// grid (rows, batch); planes `plane` elements apart.
-template <int MAXN>
-__global__ __launch_bounds__(kFftThreads) void rows_fft_power_kernel(FftDesc d, float2 *B, float *P, int64_t plane) {
-    extern __shared__ float2 buf[];
-    const int r = blockIdx.x;
-    const int n = d.n;
-    float2 *row = B + (int64_t)blockIdx.y * plane + (int64_t)r * n;
-    float *prow = P + (int64_t)blockIdx.y * plane + (int64_t)r * n;
-    fft_row<-1, MAXN>(
-        buf, d, [&](int j) { return row[j]; },
-        [&](int j, float2 f) {
-            row[j] = f;
-            prow[j] = f.x * f.x + f.y * f.y;
-        });
-}
-
-// Row r of B (r <= R/2, length d.n = C) times S'(r, c) = (S(r, c) +
-// S((R - r) % R, (C - c) % C)) / 2 from the full R x C scale S, then the
-// inverse FFT in place.  grid (R/2 + 1, B); planes `plane` apart.
-template <int MAXN>
-__global__ __launch_bounds__(kFftThreads) void rows_ifft_scaled_kernel(FftDesc d, float2 *B, const float *S,
-                                                                       int64_t plane, int R) {
-    extern __shared__ float2 buf[];
-    const int r = blockIdx.x;
-    const int n = d.n;
-    float2 *row = B + (int64_t)blockIdx.y * plane + (int64_t)r * n;
-    const float *srow = S + (int64_t)blockIdx.y * plane + (int64_t)r * n;
-    const float *mrow = S + (int64_t)blockIdx.y * plane + (int64_t)(r == 0 ? 0 : R - r) * n;
-    fft_row<1, MAXN>(
-        buf, d, [&](int j) { return cscale(row[j], 0.5f * (srow[j] + mrow[j == 0 ? 0 : n - j])); },
-        [&](int j, float2 f) { row[j] = f; });
-}
-
-// grid (rows, B)
-// rows_fft_power_kernel for columns of N = 1024 or 1536 points, reading the
-// row-major half spectra A (h x wh per frame) itself, so no transpose
-// precedes it: each column by one wave (fft_wave: every lane works in every
-// pass).  A workgroup of 8 waves
-// stages a strip of 8 adjacent columns into LDS (64-byte row pieces, each
-// column in its own padded buffer), then wave c transforms column c there and
-// writes B, P in the transposed layout as before.  Workgroup g takes strip
-// (g mod 8) * per + g / 8 (neighbouring strips on one XCD); the columns of
-// the last strip past wh are neither loaded nor stored.  grid (8 per, frames).
-template <int N>
-__global__ __launch_bounds__(512) void cols_fft_power_strip_kernel(const float2 *__restrict__ tw,
-                                                                  const float2 *__restrict__ A, int wh, float2 *B,
-                                                                  float *P, int64_t plane, int per, int lda) {
-    constexpr int SH = FftWavePlan<N>::kPadShift;
-    constexpr int SB = fft_wave_lds<N>() + 4;  // +4 spreads the staging writes of the 8 buffers over banks
-    __shared__ __attribute__((aligned(16))) float2 lds[8 * SB];
-    const int g = blockIdx.x;
-    const int strip = (g & 7) * per + (g >> 3);
-    if (strip >= (wh + 7) / 8) return;
-    const int j0 = strip * 8;
-    const float2 *Af = A + (int64_t)blockIdx.y * plane;
-    const int t = (int)threadIdx.x;
-    {
-        // two adjacent columns per thread, one 16-byte load when lda is even
-        // (j0 is, and the plane is 16-byte aligned); the second column of a
-        // strip's last pair may lie past wh, in the row's pitch or the next
-        // row, inside the plane, and is never stored
-        const int c2 = (t & 3) * 2, r = t >> 2;
-        if (j0 + c2 < wh) {
-#pragma unroll 4
-            for (int k = 0; k < N / 128; ++k) {
-                const int i = r + 128 * k;
-                const float2 *src = Af + (int64_t)i * lda + j0 + c2;
-                float4 v;
-                if ((lda & 1) == 0) {  // 16-byte aligned pairs
-                    v = *reinterpret_cast<const float4 *>(src);
-                } else {  // an odd (unpadded) pitch: two 8-byte loads
-                    const float2 a = src[0], b = src[1];
-                    v = make_float4(a.x, a.y, b.x, b.y);
-                }
-                lds[c2 * SB + fft_wave_pad<SH>(i)] = make_float2(v.x, v.y);
-                lds[(c2 + 1) * SB + fft_wave_pad<SH>(i)] = make_float2(v.z, v.w);
-            }
-        }
-    }
-    __syncthreads();
-    const int wave = t >> 6, col = j0 + wave;
-    float2 *buf = lds + wave * SB;
-    const bool store = col < wh;
-    float2 *row = B + (int64_t)blockIdx.y * plane + (int64_t)col * N;
-    float *prow = P + (int64_t)blockIdx.y * plane + (int64_t)col * N;
-    fft_wave<-1, N, true, true>(  // after the staging barrier each wave works in its own buffer
-        buf, tw, [&](int i) { return buf[fft_wave_pad<SH>(i)]; },
-        [&](int j, float2 f) {
-            if (store) {
-                row[j] = f;
-                prow[j] = f.x * f.x + f.y * f.y;
-            }
-        });
-}
-
-// The spectrum's column FFTs in the row-major layout, without transposes:
-// strips of 8 columns of A (h x wh per frame) staged into LDS as in
-// cols_fft_power_strip_kernel, transformed there in place by one wave per
-// column, and written to out (h x wh per frame, frames out_stride apart) as
-// 64-byte row pieces.  grid (8 per, frames).
-template <int N>
-__global__ __launch_bounds__(512) void spectrum_cols_strip_kernel(const float2 *__restrict__ tw,
-                                                            const float2 *__restrict__ A, int64_t plane, int wh,
-                                                            float2 *__restrict__ out, int64_t out_stride, int per,
-                                                            int lda) {
-    constexpr int SH = FftWavePlan<N>::kPadShift;
-    constexpr int SB = fft_wave_lds<N>() + 4;
-    __shared__ __attribute__((aligned(16))) float2 lds[8 * SB];
-    const int g = blockIdx.x;
-    const int strip = (g & 7) * per + (g >> 3);
-    if (strip >= (wh + 7) / 8) return;
-    const int j0 = strip * 8;
-    const float2 *Af = A + (int64_t)blockIdx.y * plane;
-    const int t = (int)threadIdx.x, c = t & 7, r = t >> 3;
-    const bool cin = j0 + c < wh;
-    {
-        // two adjacent columns per thread, one 16-byte load (as in
-        // cols_fft_power_strip_kernel)
-        const int c2 = (t & 3) * 2, r2 = t >> 2;
-        if (j0 + c2 < wh) {
-#pragma unroll 4
-            for (int k = 0; k < N / 128; ++k) {
-                const int i = r2 + 128 * k;
-                const float2 *src = Af + (int64_t)i * lda + j0 + c2;
-                float4 v;
-                if ((lda & 1) == 0) {  // 16-byte aligned pairs
-                    v = *reinterpret_cast<const float4 *>(src);
-                } else {  // an odd (unpadded) pitch: two 8-byte loads
-                    const float2 a = src[0], b = src[1];
-                    v = make_float4(a.x, a.y, b.x, b.y);
-                }
-                lds[c2 * SB + fft_wave_pad<SH>(i)] = make_float2(v.x, v.y);
-                lds[(c2 + 1) * SB + fft_wave_pad<SH>(i)] = make_float2(v.z, v.w);
-            }
-        }
-    }
-    __syncthreads();
-    float2 *buf = lds + (t >> 6) * SB;
-    // the last pass has read buf before it writes (a barrier between); each
-    // wave works in its own buffer until the store of the whole strip
-    fft_wave<-1, N, true, true>(
-        buf, tw, [&](int i) { return buf[fft_wave_pad<SH>(i)]; },
-        [&](int j, float2 f) { buf[fft_wave_pad<SH>(j)] = f; });
-    __syncthreads();
-    float2 *of = out + (int64_t)blockIdx.y * out_stride;
-    if (cin) {
-#pragma unroll 4
-        for (int k = 0; k < N / 64; ++k) {
-            const int i = r + 64 * k;
-            of[(int64_t)i * wh + j0 + c] = lds[c * SB + fft_wave_pad<SH>(i)];
-        }
-    }
-}
-
-// rows_ifft_scaled_kernel for N = 1024 or 1536 writing the row-major plane A
-// (h x wh per frame) itself, so no transpose follows it: wave c of a
-// workgroup transforms transposed row col = j0 + c of B (scaled as there) by
-// one-wave transforms into its LDS
-// buffer, then the workgroup writes the strip's 8 columns as 64-byte row
-// pieces.  Strip mapping as cols_fft_power_strip_kernel; R as there.
-template <int N>
-__global__ __launch_bounds__(512) void cols_ifft_scaled_strip_kernel(const float2 *__restrict__ tw,
-                                                                    const float2 *__restrict__ B,
-                                                                    const float *__restrict__ S, int64_t plane,
-                                                                    int R, int wh, float2 *__restrict__ A, int per,
-                                                                    int lda) {
-    constexpr int SH = FftWavePlan<N>::kPadShift;
-    constexpr int SB = fft_wave_lds<N>() + 4;
-    __shared__ __attribute__((aligned(16))) float2 lds[8 * SB];
-    const int g = blockIdx.x;
-    const int strip = (g & 7) * per + (g >> 3);
-    if (strip >= (wh + 7) / 8) return;
-    const int j0 = strip * 8;
-    const int t = (int)threadIdx.x, wave = t >> 6;
-    const int col = min(j0 + wave, wh - 1);  // a column past wh transforms the last one again and stores nothing
-    float2 *buf = lds + wave * SB;
-    const float2 *row = B + (int64_t)blockIdx.y * plane + (int64_t)col * N;
-    const float *srow = S + (int64_t)blockIdx.y * plane + (int64_t)col * N;
-    const float *mrow = S + (int64_t)blockIdx.y * plane + (int64_t)(col == 0 ? 0 : R - col) * N;
-    fft_wave<1, N, false, true>(  // each wave in its own buffer until the store of the whole strip
-        buf, tw, [&](int j) { return cscale(row[j], 0.5f * (srow[j] + mrow[j == 0 ? 0 : N - j])); },
-        [&](int j, float2 f) { buf[fft_wave_pad<SH>(j)] = f; });  // the last pass has read buf before it writes
-    __syncthreads();
-    const int c = t & 7, r = t >> 3;
-    if (j0 + c < wh) {
-        float2 *Af = A + (int64_t)blockIdx.y * plane;
-#pragma unroll 4
-        for (int k = 0; k < N / 64; ++k) {
-            const int i = r + 64 * k;
-            Af[(int64_t)i * lda + j0 + c] = lds[c * SB + fft_wave_pad<SH>(i)];
-        }
-    }
-}
-
-template <int MAXN>
-__global__ __launch_bounds__(kFftThreads) void rows_fft_fwd_inplace_kernel(FftDesc d, float2 *B, int64_t plane) {
-    extern __shared__ float2 buf[];
-    const int n = d.n;
-    float2 *row = B + (int64_t)blockIdx.y * plane + (int64_t)blockIdx.x * n;
-    fft_row<-1, MAXN>(buf, d, [&](int j) { return row[j]; }, [&](int j, float2 f) { row[j] = f; });
-}
-
-// ------------------------------------------------------ column transforms
-// Column FFTs (length h = d.n) of a row-major plane, strip by strip: a
-// workgroup reads `sw` adjacent columns row by row (contiguous pieces of
-// each row, no transpose), transforms them together in LDS (column-major
-// there) and writes them back in place.  MODE 0: plain; MODE 1: also write
-// |F|^2 to P (laid out as A); MODE 2: multiply element (i, j) by
-// (S(i, j) + S((h - i) % h, (scols - j) % scols)) / 2 on the way in, S the
-// full h x scols scale.  BIG: one column longer
-// than kFftMultiMax through fft_lds.  grid (ceil(ncols/sw), images); planes
-// `plane` elements apart, rows `ld` elements apart.
-template <int DIR, int MODE, bool BIG>
-__global__ __launch_bounds__(kFftThreads, BIG ? 1 : 2) void cols_fft_strip_kernel(FftDesc d, float2 *A, int64_t plane,
-                                                                                   int ld, int ncols, int sw,
-                                                                                   const float *S, float *P,
-                                                                                   int scols) {
-    extern __shared__ float2 buf[];
-    const int h = d.n;
-    const int j0 = blockIdx.x * sw;
-    const int ncol = min(sw, ncols - j0);
-    float2 *a = A + (int64_t)blockIdx.y * plane;
-    for (int idx = threadIdx.x; idx < h * ncol; idx += kFftThreads) {
-        const int i = idx / ncol, c = idx - (idx / ncol) * ncol;
-        const int64_t at = (int64_t)i * ld + j0 + c;
-        float2 v = a[at];
-        if (MODE == 2) {
-            const float *Sb = S + (int64_t)blockIdx.y * plane;
-            const int j = j0 + c;
-            const float s1 = Sb[(int64_t)i * scols + j];
-            const float s2 = Sb[(int64_t)(i == 0 ? 0 : h - i) * scols + (j == 0 ? 0 : scols - j)];
-            v = cscale(v, 0.5f * (s1 + s2));
-        }
-        buf[c * h + i] = v;
-    }
-    __syncthreads();
-    if constexpr (BIG)
-        fft_lds<DIR>(buf, d);
-    else
-        fft_lds_multi<DIR>(buf, d, ncol);
-    for (int idx = threadIdx.x; idx < h * ncol; idx += kFftThreads) {
-        const int i = idx / ncol, c = idx - (idx / ncol) * ncol;
-        const int64_t at = (int64_t)i * ld + j0 + c;
-        const float2 f = buf[c * h + i];
-        a[at] = f;
-        if (MODE == 1) P[(int64_t)blockIdx.y * plane + at] = f.x * f.x + f.y * f.y;
-    }
-}
-
 // ------------------------------------------------------------- workspace
-// Columns per strip: a power of two <= 16 with sw * h <= kFftMultiMax.
-int col_strip(int h) {
-    int sw = 16;
-    while (sw > 1 && (size_t)sw * h > (size_t)kFftMultiMax) sw >>= 1;
-    return sw;
-}
-// Column transforms by strips up to 128 rows, through transposes above
-// (batches of 32 measured both ways, NCC / PCE images/s): 1024 x 1024
-// 26.1k / 20.8k by 4-column strips (32-byte row pieces) -> 37.5k / 29.2k;
-// 512 x 512 99k / 78k by 8-column strips -> 123k / 98k.
-bool strips_for(int h) { return h <= 128; }
-
 // Per-image buffers, each an array over the batch with the given stride.
 struct ExtractWs {
     int nb;                 // images the workspace holds
     int64_t n;              // plane stride (elements) of A, P, S
-    float2 *A, *B;          // complex planes of the Wiener filter (B: transposed path only)
+    float2 *A, *B;          // complex planes of the Wiener filter (B transposed)
     float *P, *S;           // power spectrum / scale (S also holds the FastNoise output)
     double *rowsq, *var, *colpart, *rowpart, *colmean, *rowmean, *g;
     float *cz, *rz;         // FP32 zero-mean column terms (2w) and row means (2h) per image
@@ -1196,7 +905,7 @@ int zm_tiles_y_max(int h, int w) { return std::max((h + kZmTileRows - 1) / kZmTi
 size_t per_image_bytes(int h, int w) {
     const int64_t n = (int64_t)h * w;
     const int tx = zm_tiles_x_max(w), ty = zm_tiles_y_max(h, w);
-    return (strips_for(h) ? 16 : 24) * (size_t)n + 8 * (size_t)(h + 1 + 2 * w * ty + 2 * h * tx + 2 * w + 2 * h + 4) +
+    return 24 * (size_t)n + 8 * (size_t)(h + 1 + 2 * w * ty + 2 * h * tx + 2 * w + 2 * h + 4) +
            4 * (size_t)(2 * w + 2 * h) + 13 * 256;
 }
 
@@ -1211,7 +920,7 @@ int get_ws(Context *c, int nb, ExtractWs &e) {
     e.cp_stride = 2 * (int64_t)w * zm_tiles_y_max(h, w);
     e.rp_stride = 2 * (int64_t)h * zm_tiles_x_max(w);
     const size_t sz[] = {align256(sizeof(float2) * n * nb),
-                         strips_for(h) ? 0 : align256(sizeof(float2) * n * nb),
+                         align256(sizeof(float2) * n * nb),
                          align256(sizeof(float) * n * nb),    align256(sizeof(float) * n * nb),
                          align256(sizeof(double) * h * nb),   align256(sizeof(double) * nb),
                          align256(sizeof(double) * e.cp_stride * nb), align256(sizeof(double) * e.rp_stride * nb),
@@ -1232,20 +941,6 @@ int get_ws(Context *c, int nb, ExtractWs &e) {
     }
     return PRNU_OK;
 }
-
-size_t fft_smem(const FftDesc &d) { return sizeof(float2) * d.n; }
-
-// Row-FFT kernel K<MAXN> over rows of length n: the register budget of the
-// smallest of kFftSmallN, kFftMidN, kFftMaxN that holds the row.
-#define PRNU_LAUNCH_ROW(K, n, grid, st, ...)                                                                    \
-    do {                                                                                                        \
-        if ((n) <= kFftSmallN)                                                                                  \
-            hipLaunchKernelGGL((K<kFftSmallN>), grid, dim3(kFftThreads), fft_row_smem(n), st, __VA_ARGS__);     \
-        else if ((n) <= kFftMidN)                                                                               \
-            hipLaunchKernelGGL((K<kFftMidN>), grid, dim3(kFftThreads), fft_row_smem(n), st, __VA_ARGS__);       \
-        else                                                                                                    \
-            hipLaunchKernelGGL((K<kFftMaxN>), grid, dim3(kFftThreads), fft_row_smem(n), st, __VA_ARGS__);       \
-    } while (0)
 
 // The row-walking kernel needs widths that are multiples of 4 (>= 8), two
 // rows, and 16-byte aligned output rows (the chain's workspace planes).  The
@@ -1316,46 +1011,36 @@ int launch_zm_means(Context *c, ExtractWs &e, int nb, hipStream_t st) {
     return PRNU_OK;
 }
 
-template <int DIR, int MODE>
-int launch_cols_fft(const FftDesc &dh, float2 *A, int64_t plane, int ld, int ncols, int nb, const float *S, float *P,
-                    hipStream_t st, int scols = 0) {
-    const int h = dh.n;
-    const bool big = h > kFftMultiMax;
-    const int sw = big ? 1 : col_strip(h);
-    const dim3 grid((ncols + sw - 1) / sw, nb);
-    const size_t smem = sizeof(float2) * (size_t)sw * h;
-    if (big)
-        hipLaunchKernelGGL((cols_fft_strip_kernel<DIR, MODE, true>), grid, dim3(kFftThreads), smem, st, dh, A, plane,
-                           ld, ncols, sw, S, P, scols);
-    else
-        hipLaunchKernelGGL((cols_fft_strip_kernel<DIR, MODE, false>), grid, dim3(kFftThreads), smem, st, dh, A, plane,
-                           ld, ncols, sw, S, P, scols);
-    PRNU_CHECK_LAUNCH();
-    return PRNU_OK;
-}
-
 // Sizes whose zero-mean takes the ZM_EVEN form of wiener_rows_fwd_kernel.
 // (With one row or column of a parity the zero-mean image is nothing but
 // rounding: those keep the general form and its results.)
 bool zm_even_form(int h, int w) { return w % 2 == 0 && w >= 4 && h >= 3; }
 
 // Row pitch of the chain's half-spectrum plane A: 128-byte rows (a multiple
-// of 16 complex values) where the strip kernels read or write A in 64-byte
-// row pieces (1024 and 1536 rows), so that no piece straddles two lines;
-// w/2 + 1 elsewhere (transposes and short-column strips take A packed).  A
-// plane holds h x w complex values, so the padded pitch is used only when it
-// fits in w.
-int half_plane_pitch(int h, int w) {
+// of 16 complex values), so that no piece of a row that the column strips read
+// or write straddles two lines.  A plane holds h x w complex values, so the
+// padded pitch is used only when it fits in w.
+int half_plane_pitch(int w) {
     const int wh = w / 2 + 1, padded = (wh + 15) & ~15;
-    return (h == 1024 || h == 1536) && padded <= w ? padded : wh;
+    return padded <= w ? padded : wh;
+}
+
+int launch_rows_c2r(const FftDesc &dw, const float2 *A, int64_t plane, int h, int nb, float *out, int64_t out_stride,
+                    float inv_n, int lda, hipStream_t st) {
+    return with_row_plan<true>(dw, [&](auto pl) -> int {
+        typedef decltype(pl) Plan;
+        hipLaunchKernelGGL(rows_c2r_kernel<Plan>, dim3((h + 1) / 2, nb), dim3(Plan::T), pl.smem(), st, pl, A, plane,
+                           h, out, out_stride, inv_n, lda);
+        PRNU_CHECK_LAUNCH();
+        return PRNU_OK;
+    });
 }
 
 // Wiener filter of nb images (img, img_stride floats apart) into out, on
 // half spectra: row FFTs two rows at a time, column FFTs (+ |F|^2) over the
 // w/2+1 columns, the variance stencil on the full grid (mirrored reads of
 // the half power spectrum), the symmetrized scale + inverse column FFTs,
-// real inverse row FFTs two rows at a time; columns by strips or through
-// transposes (strips_for).
+// real inverse row FFTs two rows at a time.
 int launch_wiener(Context *c, ExtractWs &e, int nb, const float *img, int64_t img_stride, float *out,
                   int64_t out_stride, bool zm, hipStream_t st) {
     const int h = c->h, w = c->w, wh = w / 2 + 1;
@@ -1363,113 +1048,49 @@ int launch_wiener(Context *c, ExtractWs &e, int nb, const float *img, int64_t im
     const FftDesc &dw = fft_desc(c->fft_w);
     const FftDesc &dh = fft_desc(c->fft_h);
     const int pairs = (h + 1) / 2;
-    const int lda = half_plane_pitch(h, w);
+    const int lda = half_plane_pitch(w);
     // (the two-wave 2048-point form measured slower here, 331 -> 365 us per
     // 32 frames of 2048x1536: four loads per value and FP64 sums at 4 waves
     // per SIMD; it pays in rows_c2r_kernel)
     const bool zm_even = zm && zm_even_form(h, w);
-#define PRNU_WIENER_ROWS(M, PAD, ZE)                                                                                \
-    hipLaunchKernelGGL((wiener_rows_fwd_kernel<M, PAD, ZE>), dim3(pairs, nb), dim3(kFftThreads),                    \
-                       PAD ? sizeof(float2) * kFft2048PadLds : fft_row_smem(w), st, dw, img, img_stride, h, e.A, n, \
-                       e.rowsq, zm ? e.cz : nullptr, zm ? e.rz : nullptr, lda)
-    if (zm_even) {
-        if (w == 2048) PRNU_WIENER_ROWS(kFftSmallN, true, true);
-        else if (w <= kFftSmallN) PRNU_WIENER_ROWS(kFftSmallN, false, true);
-        else if (w <= kFftMidN) PRNU_WIENER_ROWS(kFftMidN, false, true);
-        else PRNU_WIENER_ROWS(kFftMaxN, false, true);
-    } else {
-        if (w == 2048) PRNU_WIENER_ROWS(kFftSmallN, true, false);
-        else if (w <= kFftSmallN) PRNU_WIENER_ROWS(kFftSmallN, false, false);
-        else if (w <= kFftMidN) PRNU_WIENER_ROWS(kFftMidN, false, false);
-        else PRNU_WIENER_ROWS(kFftMaxN, false, false);
-    }
-#undef PRNU_WIENER_ROWS
-    PRNU_CHECK_LAUNCH();
+    PRNU_TRY(with_row_plan<false>(dw, [&](auto pl) -> int {
+        typedef decltype(pl) Plan;
+        const dim3 grid(pairs, nb), block(Plan::T);
+        if (zm_even)
+            hipLaunchKernelGGL((wiener_rows_fwd_kernel<Plan, true>), grid, block, pl.smem(), st, pl, img, img_stride,
+                               h, e.A, n, e.rowsq, e.cz, nullptr, lda);
+        else
+            hipLaunchKernelGGL((wiener_rows_fwd_kernel<Plan, false>), grid, block, pl.smem(), st, pl, img, img_stride,
+                               h, e.A, n, e.rowsq, zm ? e.cz : nullptr, zm ? e.rz : nullptr, lda);
+        PRNU_CHECK_LAUNCH();
+        return PRNU_OK;
+    }));
     hipLaunchKernelGGL(wiener_var_kernel, dim3(nb), dim3(256), 0, st, e.rowsq, h, n, e.var);
     PRNU_CHECK_LAUNCH();
-    if (strips_for(h)) {
-        PRNU_TRY((launch_cols_fft<-1, 1>(dh, e.A, n, wh, wh, nb, nullptr, e.P, st)));
-        PRNU_TRY(launch_varest(e.P, e.S, h, w, false, nb, e.var, st));
-        PRNU_TRY((launch_cols_fft<1, 2>(dh, e.A, n, wh, wh, nb, e.S, nullptr, st, w)));
-    } else {
-        // transposed layout: B = A^T (wh x h), column FFTs as rows of B; the
-        // zero-padded box-min stencil is transpose invariant
-        const int per = ((wh + 7) / 8 + 7) / 8;
-        if (h == 1024) {
-            hipLaunchKernelGGL(cols_fft_power_strip_kernel<1024>, dim3(8 * per, nb), dim3(512), 0, st, dh.tw, e.A,
-                               wh, e.B, e.P, n, per, lda);
-        } else if (h == 1536) {
-            hipLaunchKernelGGL(cols_fft_power_strip_kernel<1536>, dim3(8 * per, nb), dim3(512), 0, st, dh.tw, e.A,
-                               wh, e.B, e.P, n, per, lda);
-        } else {
-            PRNU_TRY(launch_transpose_c(e.A, e.B, h, wh, nb, n, st));
-            PRNU_LAUNCH_ROW(rows_fft_power_kernel, h, dim3(wh, nb), st, dh, e.B, e.P, n);
-        }
-        PRNU_CHECK_LAUNCH();
-        PRNU_TRY(launch_varest(e.P, e.S, w, h, true, nb, e.var, st));
-        if (h == 1024) {
-            hipLaunchKernelGGL(cols_ifft_scaled_strip_kernel<1024>, dim3(8 * per, nb), dim3(512), 0, st, dh.tw, e.B,
-                               e.S, n, w, wh, e.A, per, lda);
-        } else if (h == 1536) {
-            hipLaunchKernelGGL(cols_ifft_scaled_strip_kernel<1536>, dim3(8 * per, nb), dim3(512), 0, st, dh.tw, e.B,
-                               e.S, n, w, wh, e.A, per, lda);
-        } else {
-            PRNU_LAUNCH_ROW(rows_ifft_scaled_kernel, h, dim3(wh, nb), st, dh, e.B, e.S, n, w);
-            PRNU_CHECK_LAUNCH();
-            PRNU_TRY(launch_transpose_c(e.B, e.A, wh, h, nb, n, st));
-        }
-        PRNU_CHECK_LAUNCH();
-    }
-    if (w == 2048)
-        hipLaunchKernelGGL((rows_c2r_kernel<kFftSmallN, 2048>), dim3(pairs, nb), dim3(128),
-                           sizeof(float2) * fft_wave_lds<2048>(), st, dw, e.A, n, h, out, out_stride,
-                           1.0f / (float)((double)w * h), lda);
-    else
-        PRNU_LAUNCH_ROW(rows_c2r_kernel, w, dim3(pairs, nb), st, dw, e.A, n, h, out, out_stride,
-                        1.0f / (float)((double)w * h), lda);
-    PRNU_CHECK_LAUNCH();
-    return PRNU_OK;
+    // B = A^T (wh x h); the zero-padded box-min stencil is transpose invariant
+    PRNU_TRY(launch_cols_power(dh, e.A, lda, wh, e.B, e.P, n, nb, st));
+    PRNU_TRY(launch_varest(e.P, e.S, w, h, nb, e.var, st));
+    PRNU_TRY(launch_cols_inverse(dh, e.B, e.S, w, wh, e.A, lda, n, nb, st));
+    return launch_rows_c2r(dw, e.A, n, h, nb, out, out_stride, 1.0f / (float)((double)w * h), lda, st);
 }
 
 // R2C spectrum of nb images into out (h x (w/2+1) complex each, out_stride
-// float2 apart): half-row FFTs, then column FFTs (strips in place in out, or
-// through transposes).
+// float2 apart): half-row FFTs, then column FFTs.
 int launch_spectrum(Context *c, ExtractWs &e, int nb, const float *img, int64_t img_stride, float2 *out,
                     int64_t out_stride, hipStream_t st) {
     const int h = c->h, w = c->w, wh = w / 2 + 1;
     const FftDesc &dw = fft_desc(c->fft_w);
     const FftDesc &dh = fft_desc(c->fft_h);
-    if (strips_for(h)) {
-        PRNU_LAUNCH_ROW(rows_fft_half_kernel, w, dim3((h + 1) / 2, nb), st, dw, img, img_stride, out, out_stride, h,
-                        wh);
-        PRNU_CHECK_LAUNCH();
-        PRNU_TRY((launch_cols_fft<-1, 0>(dh, out, out_stride, wh, wh, nb, nullptr, nullptr, st)));
-        return PRNU_OK;
-    }
     const int64_t n = c->pixels();
-    const int lda = half_plane_pitch(h, w);
-    if (w == 2048)
-        hipLaunchKernelGGL((rows_fft_half_kernel<kFftSmallN, true>), dim3((h + 1) / 2, nb), dim3(kFftThreads),
-                           sizeof(float2) * kFft2048PadLds, st, dw, img, img_stride, e.A, n, h, lda);
-    else
-        PRNU_LAUNCH_ROW(rows_fft_half_kernel, w, dim3((h + 1) / 2, nb), st, dw, img, img_stride, e.A, n, h, lda);
-    PRNU_CHECK_LAUNCH();
-    if (h == 1024 || h == 1536) {  // no transposes: strips of 8 columns through LDS
-        const int per = ((wh + 7) / 8 + 7) / 8;
-        if (h == 1024)
-            hipLaunchKernelGGL(spectrum_cols_strip_kernel<1024>, dim3(8 * per, nb), dim3(512), 0, st, dh.tw, e.A, n,
-                               wh, out, out_stride, per, lda);
-        else
-            hipLaunchKernelGGL(spectrum_cols_strip_kernel<1536>, dim3(8 * per, nb), dim3(512), 0, st, dh.tw, e.A, n,
-                               wh, out, out_stride, per, lda);
+    const int lda = half_plane_pitch(w);
+    PRNU_TRY(with_row_plan<false>(dw, [&](auto pl) -> int {
+        typedef decltype(pl) Plan;
+        hipLaunchKernelGGL(rows_fft_half_kernel<Plan>, dim3((h + 1) / 2, nb), dim3(Plan::T), pl.smem(), st, pl, img,
+                           img_stride, e.A, n, h, lda);
         PRNU_CHECK_LAUNCH();
         return PRNU_OK;
-    }
-    PRNU_TRY(launch_transpose_c(e.A, e.B, h, wh, nb, n, st));
-    PRNU_LAUNCH_ROW(rows_fft_fwd_inplace_kernel, h, dim3(wh, nb), st, dh, e.B, n);
-    PRNU_CHECK_LAUNCH();
-    PRNU_TRY(launch_transpose_c(e.B, out, wh, h, nb, n, st, out_stride));
-    return PRNU_OK;
+    }));
+    return launch_cols_spectrum(dh, e.A, lda, wh, n, out, out_stride, nb, st);
 }
 
 int input_bytes_per_pixel(int fmt) {

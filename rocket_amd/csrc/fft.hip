@@ -1,9 +1,10 @@
-// FFT plans (twiddle tables) and the row/transposition kernels shared by the
-// Wiener filter, the spectral filter and PCE.
+// FFT plans (radices, twiddle tables) shared by the Wiener filter, the spectral
+// filter and PCE.
 #include "prnu_internal.hpp"
 #include "fft_device.hpp"
 #include "fft_host.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <new>
 #include <vector>
@@ -11,29 +12,71 @@
 namespace prnu {
 
 struct FftPlan {
-    FftDesc desc;
+    FftDesc desc, basic;
     float2 *d_tw = nullptr;
 };
 
-// Radices 8, 4, 2 first (the twiddle exponent's j mod Ns is then a mask),
-// then 3 and 5; a power-of-two part 8^k * 2 becomes 8^(k-1) * 4 * 4 (the
-// same number of passes, no radix-2 pass).
-bool fft_factor(int n, int *radix, int *passes) {
+// Radices whose product is n, as few as possible (a pass is an LDS round trip
+// and a barrier), then with the smallest sum (the least arithmetic and the
+// evenest split over the threads); the power-of-two ones first, so the twiddle
+// exponent's j mod Ns stays a mask.  4000 = 20 20 10 instead of 8 4 5 5 5.
+static bool fft_factor(int n, int *radix, int *passes) {
+    static const int kRadices[] = {16, 8, 4, 2, 20, 12, 10, 6, 15, 9, 5, 3};
+    std::vector<int> best, cur;
+    int best_sum = 0;
+    auto search = [&](auto &self, int left, int from, int sum) -> void {
+        if (left == 1) {
+            if (best.empty() || cur.size() < best.size() || (cur.size() == best.size() && sum < best_sum)) {
+                best = cur;
+                best_sum = sum;
+            }
+            return;
+        }
+        if (!best.empty() && cur.size() >= best.size()) return;
+        for (int i = from; i < (int)(sizeof(kRadices) / sizeof(int)); ++i) {
+            if (left % kRadices[i]) continue;
+            cur.push_back(kRadices[i]);
+            self(self, left / kRadices[i], i, sum + kRadices[i]);
+            cur.pop_back();
+        }
+    };
+    search(search, n, 0, 0);
+    if (best.empty() || best.size() > (size_t)kFftMaxPasses) return false;
+    *passes = (int)best.size();
+    std::copy(best.begin(), best.end(), radix);
+    return true;
+}
+
+// Radices 8, 4, 2, then 3 and 5 alone (a power-of-two part 8^k * 2 becomes
+// 8^(k-1) * 4 * 4): the plan of PCE's row pass, whose rounding the scores keep
+// (the peak is one value of the plane, its error is not averaged).
+static void fft_factor_basic(int n, int *radix, int *passes) {
     int p = 0, e2 = 0;
-    while (n % 2 == 0) { ++e2; n /= 2; }
-    int n8 = e2 / 3, n4 = 0, n2 = 0;
-    if (e2 % 3 == 2) n4 = 1;
-    else if (e2 % 3 == 1) {
-        if (n8 > 0) { --n8; n4 = 2; } else n2 = 1;
+    for (; n % 2 == 0; n /= 2) ++e2;
+    int n8 = e2 / 3, n4 = e2 % 3 == 2 ? 1 : 0, n2 = 0;
+    if (e2 % 3 == 1) {
+        if (n8 > 0) {
+            --n8;
+            n4 = 2;
+        } else {
+            n2 = 1;
+        }
     }
-    for (int i = 0; i < n8 && p < kFftMaxPasses; ++i) radix[p++] = 8;
-    for (int i = 0; i < n4 && p < kFftMaxPasses; ++i) radix[p++] = 4;
-    for (int i = 0; i < n2 && p < kFftMaxPasses; ++i) radix[p++] = 2;
-    if (p < n8 + n4 + n2) return false;
-    while (n % 3 == 0 && p < kFftMaxPasses) { radix[p++] = 3; n /= 3; }
-    while (n % 5 == 0 && p < kFftMaxPasses) { radix[p++] = 5; n /= 5; }
+    while (n8-- > 0) radix[p++] = 8;
+    while (n4-- > 0) radix[p++] = 4;
+    while (n2-- > 0) radix[p++] = 2;
+    for (; n % 3 == 0; n /= 3) radix[p++] = 3;
+    for (; n % 5 == 0; n /= 5) radix[p++] = 5;
     *passes = p;
-    return n == 1;
+}
+
+static void fft_steps(FftDesc &d) {
+    int64_t Ns = 1;
+    for (int k = 0; k < d.passes; ++k) {
+        d.step[k] = (int)(d.n / (Ns * d.radix[k]));
+        d.inv[k] = (Ns & (Ns - 1)) ? (uint32_t)((int64_t(1) << 32) / Ns + 1) : 0;
+        Ns *= d.radix[k];
+    }
 }
 
 int fft_plan_create(int n, FftPlan **out) {
@@ -50,6 +93,10 @@ int fft_plan_create(int n, FftPlan **out) {
         set_error("fft: length %d has a prime factor other than 2, 3, 5", n);
         return PRNU_ENOTSUP;
     }
+    p->basic.n = n;
+    fft_factor_basic(n, p->basic.radix, &p->basic.passes);
+    fft_steps(p->desc);
+    fft_steps(p->basic);
     std::vector<float2> tw(n);
     const double two_pi = 6.283185307179586476925286766559;
     for (int t = 0; t < n; ++t) {
@@ -65,7 +112,7 @@ int fft_plan_create(int n, FftPlan **out) {
         set_error("fft: twiddle table: %s", hipGetErrorString(e));
         return PRNU_EDEVICE;
     }
-    p->desc.tw = p->d_tw;
+    p->desc.tw = p->basic.tw = p->d_tw;
     *out = p;
     return PRNU_OK;
 }
@@ -77,6 +124,7 @@ void fft_plan_destroy(FftPlan *p) {
 }
 
 const FftDesc &fft_desc(const FftPlan *p) { return p->desc; }
+const FftDesc &fft_desc_basic(const FftPlan *p) { return p->basic; }
 
 int ensure_fft_plans(Context *c) {
     if (!c->fft_w) PRNU_TRY(fft_plan_create(c->w, &c->fft_w));
@@ -87,40 +135,6 @@ int ensure_fft_plans(Context *c) {
             PRNU_TRY(fft_plan_create(c->h, &c->fft_h));
         }
     }
-    return PRNU_OK;
-}
-
-// ------------------------------------------------------------ transposition
-// out[b][c][r] = in[b][r][c] for an (rows x cols) complex matrix per batch item.
-namespace {
-constexpr int kTT = 32;
-
-__global__ __launch_bounds__(256) void transpose_c_kernel(const float2 *__restrict__ in, float2 *__restrict__ out,
-                                                          int rows, int cols, int64_t in_stride, int64_t out_stride) {
-    __shared__ float2 tile[kTT][kTT + 1];
-    const int64_t off = (int64_t)blockIdx.z * in_stride, ooff = (int64_t)blockIdx.z * out_stride;
-    const int c0 = blockIdx.x * kTT, r0 = blockIdx.y * kTT;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-#pragma unroll
-    for (int i = 0; i < kTT; i += 8) {
-        const int r = r0 + ty + i, c = c0 + tx;
-        if (r < rows && c < cols) tile[ty + i][tx] = in[off + (int64_t)r * cols + c];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kTT; i += 8) {
-        const int c = c0 + ty + i, r = r0 + tx;
-        if (r < rows && c < cols) out[ooff + (int64_t)c * rows + r] = tile[tx][ty + i];
-    }
-}
-}  // namespace
-
-int launch_transpose_c(const float2 *in, float2 *out, int rows, int cols, int batch, int64_t batch_stride,
-                       hipStream_t st, int64_t out_batch_stride) {
-    dim3 grid((cols + kTT - 1) / kTT, (rows + kTT - 1) / kTT, batch);
-    hipLaunchKernelGGL(transpose_c_kernel, grid, dim3(256), 0, st, in, out, rows, cols, batch_stride,
-                       out_batch_stride < 0 ? batch_stride : out_batch_stride);
-    PRNU_CHECK_LAUNCH();
     return PRNU_OK;
 }
 

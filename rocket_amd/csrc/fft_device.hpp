@@ -1,4 +1,4 @@
-// Mixed-radix (2, 3, 4, 5, 8) Stockham FFT of one row held in LDS.
+// Mixed-radix Stockham FFT of one row or column held in LDS.
 //
 // A length-n transform, n = prod(radix[p]), runs as `passes` autosorting
 // passes.  Pass p with radix R and Ns = radix[0]*...*radix[p-1] does, for each
@@ -24,6 +24,8 @@ struct FftDesc {
     int n;
     int passes;
     int radix[kFftMaxPasses];
+    int step[kFftMaxPasses];       // per pass: twiddle step n / (Ns * R)
+    uint32_t inv[kFftMaxPasses];   // per pass: floor(2^32 / Ns) + 1 where Ns is no power of two
     const float2 *tw;  // n twiddles, device memory
 };
 
@@ -187,90 +189,200 @@ __device__ __forceinline__ void dft<16, -1>(float2 *a) { dft16<-1>(a); }
 template <>
 __device__ __forceinline__ void dft<16, 1>(float2 *a) { dft16<1>(a); }
 
-// j mod Ns for the butterfly's twiddle exponent; Ns is a power of two in
-// every pass before the first radix-3 or radix-5 pass (fft_factor orders the
-// radices 8, 4, 2, 3, 5).
-__device__ __forceinline__ int fft_mod(int j, int Ns) { return (Ns & (Ns - 1)) == 0 ? (j & (Ns - 1)) : j % Ns; }
+// cos and sin of 2 pi k / n as compile-time constants (Taylor series of an
+// angle in [-pi, pi]).
+struct CosSin {
+    double c, s;
+};
+constexpr CosSin cos_sin(int k, int n) {
+    const int q = ((k % n) + n) % n;
+    const double x = 6.283185307179586476925286766559 * (double)(2 * q > n ? q - n : q) / (double)n;
+    double c = 1.0, s = x, tc = 1.0, ts = x;
+    for (int i = 1; i < 20; ++i) {
+        tc *= -x * x / ((2 * i - 1) * (2 * i));
+        ts *= -x * x / ((2 * i) * (2 * i + 1));
+        c += tc;
+        s += ts;
+    }
+    return {c, s};
+}
 
-// One Stockham pass of radix R over buf[0..n) with kFftThreads threads.
-template <int R, int DIR>
-__device__ __forceinline__ void fft_pass(float2 *buf, int n, int Ns, const float2 *tw) {
-    constexpr int kMaxB = (kFftMaxN / R + kFftThreads - 1) / kFftThreads;
-    const int nb = n / R;
-    const int twstep = n / (Ns * R);
-    const int tid = threadIdx.x;
+// a * exp(DIR * 2 pi i k / n) for compile-time k, n.
+template <int DIR, int K, int N>
+__device__ __forceinline__ float2 rotate(float2 a) {
+    constexpr int k = K % N;
+    if constexpr (k == 0) return a;
+    else if constexpr (4 * k == N) return DIR < 0 ? make_float2(a.y, -a.x) : make_float2(-a.y, a.x);
+    else if constexpr (2 * k == N) return make_float2(-a.x, -a.y);
+    else if constexpr (4 * k == 3 * N) return DIR < 0 ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
+    else {
+        constexpr CosSin w = cos_sin(k, N);
+        return cmul(a, make_float2((float)w.c, (float)(DIR * w.s)));
+    }
+}
+
+// Radix A * B (n = B n1 + n2, k = k1 + A k2): DFT-A over n1, the twiddle
+// W^(n2 k1), DFT-B over n2.
+template <int A, int B, int DIR, int N2, int K1>
+__device__ __forceinline__ void dft_twist(float2 (&t)[B][A]) {
+    if constexpr (K1 < A) {
+        t[N2][K1] = rotate<DIR, N2 * K1, A * B>(t[N2][K1]);
+        dft_twist<A, B, DIR, N2, K1 + 1>(t);
+    } else if constexpr (N2 + 1 < B) {
+        dft_twist<A, B, DIR, N2 + 1, 1>(t);
+    }
+}
+template <int A, int B, int DIR>
+__device__ __forceinline__ void dft_comp(float2 *a) {
+    float2 t[B][A];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < A; ++n1) t[n2][n1] = a[B * n1 + n2];
+        dft<A, DIR>(t[n2]);
+    }
+    dft_twist<A, B, DIR, 1, 1>(t);
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        float2 u[B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) u[n2] = t[n2][k1];
+        dft<B, DIR>(u);
+#pragma unroll
+        for (int k2 = 0; k2 < B; ++k2) a[k1 + A * k2] = u[k2];
+    }
+}
+#define PRNU_DFT_COMP(A, B)                                                                          \
+    template <>                                                                                      \
+    __device__ __forceinline__ void dft<A * B, -1>(float2 *a) { dft_comp<A, B, -1>(a); }             \
+    template <>                                                                                      \
+    __device__ __forceinline__ void dft<A * B, 1>(float2 *a) { dft_comp<A, B, 1>(a); }
+PRNU_DFT_COMP(2, 3)
+PRNU_DFT_COMP(3, 3)
+PRNU_DFT_COMP(2, 5)
+PRNU_DFT_COMP(4, 3)
+PRNU_DFT_COMP(3, 5)
+PRNU_DFT_COMP(4, 5)
+#undef PRNU_DFT_COMP
+
+// j mod Ns for the butterfly's twiddle exponent: a mask where Ns is a power of
+// two, else by the multiplier inv = floor(2^32 / Ns) + 1 (exact for j, Ns <=
+// kFftMaxN: the multiplier's excess times j stays below 2^32).
+__device__ __forceinline__ int fft_mod(int j, int Ns, uint32_t inv) {
+    return (Ns & (Ns - 1)) == 0 ? (j & (Ns - 1)) : j - Ns * (int)__umulhi((uint32_t)j, inv);
+}
+
+// ------------------------------------------ transforms of a run-time length
+// A transform of d.n <= MAXN values by T threads (lane = 0 .. T-1) through
+// LDS buf, with one pad slot per 16 values against the bank conflicts of the
+// strided writes (index p at p + p/16; fft_pad_lds(n) values).  The first
+// pass takes its inputs from get(i), the last hands its outputs to put(i, X);
+// both see i = j + r * (n/R), or j + q * Ns, for consecutive j across the
+// threads.  The passes between go through LDS.
+// WSYNC (T = 64): the buffer is one wave's own, its passes are ordered by
+// wave_lds_sync; otherwise by workgroup barriers, which every thread of the
+// workgroup reaches the same number of times.
+// SYNC_FIRST: get reads buf (a barrier between the first pass's reads and
+// writes).
+__host__ __device__ constexpr int fft_pad_lds(int n) { return n + n / 16; }
+__device__ __forceinline__ int fft_pad(int p) { return p + (p >> 4); }
+
+__device__ __forceinline__ void wave_lds_sync();
+
+template <int R, int DIR, int T, int MAXN, bool WSYNC, bool SYNC_FIRST, class Get, class Put>
+__device__ __forceinline__ void fft_pass_rt(float2 *buf, const FftDesc &d, int p, int Ns, int lane, Get &get,
+                                            Put &put) {
+    constexpr int kMaxB = (MAXN / R + T - 1) / T;
+    const bool first = p == 0, last = p == d.passes - 1;
+    const int nb = d.n / R, step = d.step[p];
+    const uint32_t inv = d.inv[p];
     float2 v[kMaxB][R];
 #pragma unroll
     for (int b = 0; b < kMaxB; ++b) {
-        const int j = tid + b * kFftThreads;
+        const int j = lane + T * b;
         if (j < nb) {
-            const int k = fft_mod(j, Ns);
-            v[b][0] = buf[j];
+            if (first) {
 #pragma unroll
-            for (int r = 1; r < R; ++r) v[b][r] = cmul(buf[j + r * nb], twiddle<DIR>(tw, r * k * twstep));
+                for (int r = 0; r < R; ++r) v[b][r] = get(j + r * nb);
+            } else {
+                const int k = fft_mod(j, Ns, inv) * step;
+                v[b][0] = buf[fft_pad(j)];
+#pragma unroll
+                for (int r = 1; r < R; ++r) v[b][r] = cmul(buf[fft_pad(j + r * nb)], twiddle<DIR>(d.tw, r * k));
+            }
         }
     }
-    __syncthreads();
+    if (!first || SYNC_FIRST) {  // every read precedes the writes below
+        if constexpr (WSYNC) wave_lds_sync();
+        else __syncthreads();
+    }
 #pragma unroll
     for (int b = 0; b < kMaxB; ++b) {
-        const int j = tid + b * kFftThreads;
+        const int j = lane + T * b;
         if (j < nb) {
             dft<R, DIR>(v[b]);
-            const int k = fft_mod(j, Ns);
+            const int k = first ? 0 : fft_mod(j, Ns, inv);
             const int base = (j - k) * R + k;
+            if (last) {
 #pragma unroll
-            for (int q = 0; q < R; ++q) buf[base + q * Ns] = v[b][q];
+                for (int q = 0; q < R; ++q) put(base + q * Ns, v[b][q]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < R; ++q) buf[fft_pad(base + q * Ns)] = v[b][q];
+            }
         }
     }
-    __syncthreads();
+    if constexpr (WSYNC) wave_lds_sync();
+    else __syncthreads();
 }
 
-// Full in-LDS transform of buf[0..d.n).  Callers synchronise before (data in
-// LDS) and may read buf after return (the last pass ends with a barrier).
-template <int DIR>
-__device__ inline void fft_lds(float2 *buf, const FftDesc &d) {
+template <int DIR, int T, int MAXN, bool WSYNC, bool SYNC_FIRST, class Get, class Put>
+__device__ __forceinline__ void fft_rt(float2 *buf, const FftDesc &d, int lane, Get &get, Put &put) {
     int Ns = 1;
     for (int p = 0; p < d.passes; ++p) {
         const int R = d.radix[p];
-        if (R == 8)
-            fft_pass<8, DIR>(buf, d.n, Ns, d.tw);
-        else if (R == 4)
-            fft_pass<4, DIR>(buf, d.n, Ns, d.tw);
-        else if (R == 2)
-            fft_pass<2, DIR>(buf, d.n, Ns, d.tw);
-        else if (R == 3)
-            fft_pass<3, DIR>(buf, d.n, Ns, d.tw);
-        else
-            fft_pass<5, DIR>(buf, d.n, Ns, d.tw);
+        // opaque per pass: otherwise every radix's addresses and input loads,
+        // which do not depend on the pass, are hoisted out of this loop and
+        // live across it (hundreds of registers, spills)
+        asm volatile("" : "+v"(lane));
+#define PRNU_PASS(RR)                                                                              \
+    case RR:                                                                                       \
+        fft_pass_rt<RR, DIR, T, MAXN, WSYNC, SYNC_FIRST>(buf, d, p, Ns, lane, get, put);           \
+        break;
+        switch (R) {
+            PRNU_PASS(2)
+            PRNU_PASS(3)
+            PRNU_PASS(4)
+            PRNU_PASS(5)
+            PRNU_PASS(6)
+            PRNU_PASS(8)
+            PRNU_PASS(9)
+            PRNU_PASS(10)
+            PRNU_PASS(12)
+            PRNU_PASS(15)
+            PRNU_PASS(16)
+            PRNU_PASS(20)
+            default: break;
+        }
+#undef PRNU_PASS
         Ns *= R;
     }
 }
 
-// One pass of fft_row: as fft_pass, but the first pass (FIRST, Ns = 1, no
-// twiddles) takes its inputs from get(i) instead of LDS and the last pass
-// (LAST, Ns * R = n) hands its outputs to put(i, v) instead of LDS.  Both
-// touch i = j + r * (n/R) and i = j + q * Ns for consecutive j across the
-// threads, so global accesses made by get/put are coalesced.
-// LDS bytes fft_row needs for a row of n values.  (A pad slot per 8 values
-// against bank conflicts of the strided writes measured slower: the padded
-// addresses cost registers, hence occupancy.)
-inline size_t fft_row_smem(int n) { return sizeof(float2) * (size_t)n; }
+// One pass of a row whose length is known at compile time.  The first pass
+// (FIRST, Ns = 1, no twiddles) takes its inputs from get(i) instead of LDS and
+// the last (LAST, Ns * R = n) hands its outputs to put(i, v).
+// LDS bytes of a run-time-plan row of n values.
+inline size_t fft_row_smem(int n) { return sizeof(float2) * (size_t)fft_pad_lds(n); }
 
-// Rows up to kFftSmallN (kFftMidN) values run with per-thread butterfly
-// arrays sized for that length (fewer registers, more waves per SIMD).
-constexpr int kFftSmallN = 2048;
-constexpr int kFftMidN = 4096;
-
-// CN > 0: the length (and CNS the pass's Ns) are compile-time constants, so
-// strides, twiddle steps and the butterfly index's modulus fold into
-// immediates (no integer division, LDS offsets in the instructions).
-template <int R, int DIR, bool FIRST, bool LAST, int MAXN, int CN = 0, int CNS = 0, class Get, class Put>
-__device__ __forceinline__ void fft_pass_io(float2 *buf, int n_rt, int Ns_rt, const float2 *tw, Get &get, Put &put) {
-    constexpr int kMaxB = ((CN > 0 ? CN : MAXN) / R + kFftThreads - 1) / kFftThreads;
-    const int n = CN > 0 ? CN : n_rt;
-    const int Ns = CN > 0 ? CNS : Ns_rt;
-    const int nb = n / R;
-    const int twstep = n / (Ns * R);
+// The length N and the pass's Ns are compile-time constants: strides, twiddle
+// steps and the butterfly index's modulus fold into immediates.  (A pad slot
+// per 8 values measured slower here: the padded addresses cost registers.)
+template <int R, int DIR, bool FIRST, bool LAST, int N, int NS, class Get, class Put>
+__device__ __forceinline__ void fft_pass_c(float2 *buf, const float2 *tw, Get &get, Put &put) {
+    constexpr int nb = N / R;
+    constexpr int kMaxB = (nb + kFftThreads - 1) / kFftThreads;
+    constexpr int twstep = N / (NS * R);
     const int tid = threadIdx.x;
     float2 v[kMaxB][R];
 #pragma unroll
@@ -281,7 +393,7 @@ __device__ __forceinline__ void fft_pass_io(float2 *buf, int n_rt, int Ns_rt, co
 #pragma unroll
                 for (int r = 0; r < R; ++r) v[b][r] = get(j + r * nb);
             } else {
-                const int k = fft_mod(j, Ns);
+                const int k = j % NS;
                 v[b][0] = buf[j];
 #pragma unroll
                 for (int r = 1; r < R; ++r) v[b][r] = cmul(buf[j + r * nb], twiddle<DIR>(tw, r * k * twstep));
@@ -294,37 +406,22 @@ __device__ __forceinline__ void fft_pass_io(float2 *buf, int n_rt, int Ns_rt, co
         const int j = tid + b * kFftThreads;
         if (j < nb) {
             dft<R, DIR>(v[b]);
-            const int k = FIRST ? 0 : fft_mod(j, Ns);
+            const int k = FIRST ? 0 : j % NS;
             const int base = (j - k) * R + k;
 #pragma unroll
             for (int q = 0; q < R; ++q) {
                 if constexpr (LAST)
-                    put(base + q * Ns, v[b][q]);
+                    put(base + q * NS, v[b][q]);
                 else
-                    buf[base + q * Ns] = v[b][q];
+                    buf[base + q * NS] = v[b][q];
             }
         }
     }
     __syncthreads();
 }
 
-template <int DIR, bool FIRST, bool LAST, int MAXN, class Get, class Put>
-__device__ __forceinline__ void fft_pass_io_r(int R, float2 *buf, int n, int Ns, const float2 *tw, Get &get,
-                                              Put &put) {
-    if (R == 8)
-        fft_pass_io<8, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
-    else if (R == 4)
-        fft_pass_io<4, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
-    else if (R == 2)
-        fft_pass_io<2, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
-    else if (R == 3)
-        fft_pass_io<3, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
-    else
-        fft_pass_io<5, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
-}
-
-// Radix plan of fft_factor (fft.hip) as a compile-time value, for the row
-// lengths the chain and PCE run most.
+// Radices 8, 4, 2, then 3 and 5, as a compile-time value, for the row lengths
+// the chain and PCE run most.
 struct RadixPlanC {
     int passes;
     int radix[kFftMaxPasses];
@@ -366,12 +463,12 @@ __device__ __forceinline__ void fft_passes_c(float2 *buf, const float2 *tw, Get 
     constexpr RadixPlanC pl = radix_plan_c(N);
     if constexpr (P < pl.passes) {
         constexpr int R = pl.radix[P];
-        fft_pass_io<R, DIR, P == 0, P == pl.passes - 1, N, N, NS>(buf, N, NS, tw, get, put);
+        fft_pass_c<R, DIR, P == 0, P == pl.passes - 1, N, NS>(buf, tw, get, put);
         fft_passes_c<DIR, N, P + 1, NS * R>(buf, tw, get, put);
     }
 }
 
-// fft_row for a compile-time length N (at least two passes).
+// A row of compile-time length N (at least two passes).
 template <int DIR, int N, class Get, class Put>
 __device__ __forceinline__ void fft_row_c(float2 *buf, const float2 *tw, Get &get, Put &put) {
     static_assert(radix_plan_c(N).passes >= 2, "fft_row_c: at least two passes");
@@ -473,7 +570,7 @@ __device__ __forceinline__ void fft_wave_pass(float2 *buf, const float2 *tw, Get
 }
 
 // 1024 points as radix 16, 16, 4 (16 values per lane); get(i) and put(i, X)
-// as fft_row's.  buf: fft_wave_lds(1024) values.
+// as fft_rt's.  buf: fft_wave_lds(1024) values.
 template <int DIR, bool SYNC_FIRST = false, bool WSYNC = false, class Get, class Put>
 __device__ __forceinline__ void fft_wave_1024(float2 *buf, const float2 *tw, Get get, Put put) {
     fft_wave_pass<16, DIR, true, false, 1024, 1, SYNC_FIRST, 4, 64, WSYNC>(buf, tw, get, put);
@@ -521,95 +618,72 @@ __device__ __forceinline__ void fft_wave(float2 *buf, const float2 *tw, Get get,
         fft_wave_1536<DIR, SYNC_FIRST, WSYNC>(buf, tw, get, put);
 }
 
-// Transform of one row of length d.n <= MAXN from get(i) (i in [0, n), each
-// read once) to put(i, X[i]) (each written once), through LDS buf
-// (fft_row_smem(n) bytes) for the passes between; ends with a barrier, so
-// the caller may reuse buf.
-template <int DIR, int MAXN, class Get, class Put>
-__device__ inline void fft_row(float2 *buf, const FftDesc &d, Get get, Put put) {
-    // the hot lengths with compile-time strides
-    if constexpr (MAXN >= 2048) {
-        if (d.n == 2048) return fft_row_c<DIR, 2048>(buf, d.tw, get, put);
-        if (d.n == 1536) return fft_row_c<DIR, 1536>(buf, d.tw, get, put);
+// ------------------------------------------------------------- row plans
+// How a kernel transforms rows of n() values on T threads: run<DIR>(buf, get,
+// put) from get(i) (i in [0, n), each read once) to put(i, X[i]) (each written
+// once) through smem() bytes of LDS for the passes between; it ends with a
+// barrier, and the last pass has read buf before it puts, so put may write it.
+// A plan is a kernel's template argument: the hot lengths fold their strides
+// into immediates, and their registers are not those of the widest radix of
+// the run-time plan (a real inverse row: 126 registers against 61).
+template <int N>
+struct RowC {  // radices 8, 4, 2, 3, 5
+    static constexpr int T = kFftThreads;
+    const float2 *tw;
+    __host__ __device__ static constexpr int n() { return N; }
+    static constexpr size_t smem() { return sizeof(float2) * N; }
+    template <int DIR, class Get, class Put>
+    __device__ __forceinline__ void run(float2 *buf, Get get, Put put) const {
+        fft_row_c<DIR, N>(buf, tw, get, put);
     }
-    if constexpr (MAXN >= 1024) {
-        if (d.n == 1024) return fft_row_c<DIR, 1024>(buf, d.tw, get, put);
+};
+struct Row2048 {  // radix 8, 8, 8, 4, padded (fft_block_2048_r8)
+    static constexpr int T = 256;
+    const float2 *tw;
+    __host__ __device__ static constexpr int n() { return 2048; }
+    static constexpr size_t smem() { return sizeof(float2) * kFft2048PadLds; }
+    template <int DIR, class Get, class Put>
+    __device__ __forceinline__ void run(float2 *buf, Get get, Put put) const {
+        fft_block_2048_r8<DIR>(buf, tw, get, put);
     }
-    const int P = d.passes;
-    if (P == 1) {
-        fft_pass_io_r<DIR, true, true, MAXN>(d.radix[0], buf, d.n, 1, d.tw, get, put);
-        return;
+};
+struct Row2048Waves {  // radix 16, 16, 8 on two waves (fft_block_2048)
+    static constexpr int T = 128;
+    const float2 *tw;
+    __host__ __device__ static constexpr int n() { return 2048; }
+    static constexpr size_t smem() { return sizeof(float2) * fft_wave_lds<2048>(); }
+    template <int DIR, class Get, class Put>
+    __device__ __forceinline__ void run(float2 *buf, Get get, Put put) const {
+        fft_block_2048<DIR>(buf, tw, get, put);
     }
-    fft_pass_io_r<DIR, true, false, MAXN>(d.radix[0], buf, d.n, 1, d.tw, get, put);
-    int Ns = d.radix[0];
-    for (int p = 1; p < P - 1; ++p) {
-        fft_pass_io_r<DIR, false, false, MAXN>(d.radix[p], buf, d.n, Ns, d.tw, get, put);
-        Ns *= d.radix[p];
+};
+// Any length up to 8 T (few registers at every length: longer per-thread
+// arrays cost occupancy and an LDS-bound pass does not need them).
+template <int T_>
+struct RowRt {
+    static constexpr int T = T_;
+    FftDesc d;
+    __host__ __device__ int n() const { return d.n; }
+    size_t smem() const { return fft_row_smem(d.n); }
+    template <int DIR, class Get, class Put>
+    __device__ __forceinline__ void run(float2 *buf, Get get, Put put) const {
+        fft_rt<DIR, T, 8 * T, false, false>(buf, d, (int)threadIdx.x, get, put);
     }
-    fft_pass_io_r<DIR, false, true, MAXN>(d.radix[P - 1], buf, d.n, Ns, d.tw, get, put);
-}
+};
 
-// Values held in LDS by one multi-transform call (cols * n), bounded so the
-// per-thread butterfly registers stay small.
-constexpr int kFftMultiMax = 4096;
-
-// One Stockham pass of radix R over `cols` independent transforms of length
-// n stored back to back (buf[c*n .. c*n+n)), all butterflies of all
-// transforms spread over the block: cols * n <= kFftMultiMax.
-template <int R, int DIR>
-__device__ __forceinline__ void fft_pass_multi(float2 *buf, int n, int cols, int Ns, const float2 *tw) {
-    constexpr int kMaxB = (kFftMultiMax / R + kFftThreads - 1) / kFftThreads;
-    const int nb = n / R;
-    const int total = nb * cols;
-    const int twstep = n / (Ns * R);
-    const int tid = threadIdx.x;
-    float2 v[kMaxB][R];
-#pragma unroll
-    for (int b = 0; b < kMaxB; ++b) {
-        const int t = tid + b * kFftThreads;
-        if (t < total) {
-            const int c = t / nb, j = t - c * nb;
-            const int k = fft_mod(j, Ns);
-            const float2 *col = buf + c * n;
-            v[b][0] = col[j];
-#pragma unroll
-            for (int r = 1; r < R; ++r) v[b][r] = cmul(col[j + r * nb], twiddle<DIR>(tw, r * k * twstep));
-        }
+// Calls f(plan) with the plan of rows of d.n values; TWO_WAVES: 2048 on two waves.
+template <bool TWO_WAVES, class F>
+auto with_row_plan(const FftDesc &d, F f) {
+    if (d.n == 1024) return f(RowC<1024>{d.tw});
+    if (d.n == 1536) return f(RowC<1536>{d.tw});
+    if constexpr (TWO_WAVES) {
+        if (d.n == 2048) return f(Row2048Waves{d.tw});
+    } else {
+        if (d.n == 2048) return f(Row2048{d.tw});
     }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < kMaxB; ++b) {
-        const int t = tid + b * kFftThreads;
-        if (t < total) {
-            const int c = t / nb, j = t - c * nb;
-            dft<R, DIR>(v[b]);
-            const int k = fft_mod(j, Ns);
-            const int base = c * n + (j - k) * R + k;
-#pragma unroll
-            for (int q = 0; q < R; ++q) buf[base + q * Ns] = v[b][q];
-        }
-    }
-    __syncthreads();
-}
-
-// `cols` in-LDS transforms of length d.n at buf + c*d.n (cols*d.n <= kFftMultiMax).
-template <int DIR>
-__device__ inline void fft_lds_multi(float2 *buf, const FftDesc &d, int cols) {
-    int Ns = 1;
-    for (int p = 0; p < d.passes; ++p) {
-        const int R = d.radix[p];
-        if (R == 8)
-            fft_pass_multi<8, DIR>(buf, d.n, cols, Ns, d.tw);
-        else if (R == 4)
-            fft_pass_multi<4, DIR>(buf, d.n, cols, Ns, d.tw);
-        else if (R == 2)
-            fft_pass_multi<2, DIR>(buf, d.n, cols, Ns, d.tw);
-        else if (R == 3)
-            fft_pass_multi<3, DIR>(buf, d.n, cols, Ns, d.tw);
-        else
-            fft_pass_multi<5, DIR>(buf, d.n, cols, Ns, d.tw);
-        Ns *= R;
-    }
+    if (d.n <= 2048) return f(RowRt<256>{d});
+    if (d.n <= 4096) return f(RowRt<512>{d});
+    return f(RowRt<1024>{d});
 }
 
 }  // namespace prnu

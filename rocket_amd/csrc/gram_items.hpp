@@ -46,7 +46,8 @@ __device__ inline int2 tri_tile(int t, int nt) {
 // LDS quarter k holds unit k % (4 / ks) at slab k / (4 / ks) of the group, so
 // every wave pair multiplies one unit of one slab, adds it up in that slab's
 // own order and writes that slab's own partial (the same bits as one slab at
-// a time), and the item runs once per ks slabs (slab_split, ItemIndex).  A set
+// a time), and the item runs once per ks slabs (slab_split, ItemIndex), where
+// that shortens the launch (choose_slab).  A set
 // of at most 128 patterns then multiplies with all eight waves instead of two,
 // and 300 patterns take 1.5 items per slab instead of 2 (whole 256-row tiles:
 // 3; 300 of 640x480 over a pointer table in FP32: 1,056 -> 585 us).
@@ -81,7 +82,7 @@ __device__ __forceinline__ void item_tiles(ItemWaves &r, int x, int y) {
     r.q[3] = y * kGramTile + 128;
 }
 
-// Slabs the last item of a slab of the triangle takes at once: 4 or 2 where it
+// Slabs the last item of a slab of the triangle can take at once: 4 or 2 where it
 // holds one or two one-quarter units (odd Q, (m + 1) mod 4 = 1 or 2), else 1.
 __host__ __device__ inline int slab_split(int count) {
     const int Q = (count + 127) >> 7, m = Q >> 1;
@@ -90,9 +91,10 @@ __host__ __device__ inline int slab_split(int count) {
     return rest == 1 ? 4 : rest == 2 ? 2 : 1;
 }
 
-// Item u of a slab of the triangle of `count` patterns (nt = ceil(count /
+// Item u of a slab of the triangle of `count` patterns, the last one taking ks
+// slabs (1 or slab_split(count)) (nt = ceil(count /
 // 256) partial tiles), for wave `wave`.
-__device__ __forceinline__ ItemWaves item_waves(int u, int count, int wave) {
+__device__ __forceinline__ ItemWaves item_waves(int u, int count, int wave, int ks) {
     ItemWaves r;
     r.ks = 1;
     r.kq[0] = r.kq[1] = r.kq[2] = r.kq[3] = r.kw = 0;
@@ -151,8 +153,8 @@ __device__ __forceinline__ ItemWaves item_waves(int u, int count, int wave) {
     }
     // one-quarter units 4j' .. 4j'+3 of the list (2j+1, 2j+1) j < m, then (L, L)
     const int j0 = 4 * (p - m);
-    const int ks = slab_split(count), units = 4 / ks;  // ks > 1 only if this is the last item
-    const bool split = ks > 1 && m + 1 - j0 <= units;
+    const int units = 4 / ks;
+    const bool split = ks > 1 && m + 1 - j0 <= units;  // the last item
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int j = min(j0 + (split ? i % units : i), m);
@@ -227,9 +229,11 @@ __device__ __forceinline__ ItemWaves rect_waves(int u, int ntb, int wave) {
 }
 
 
-// Blocks of K per slab: store.hip.
-int64_t choose_kcb(const int *items, const int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
-                   size_t max_bytes, int64_t longest);
+// Blocks of K per slab, at most `longest` (0: no limit), and per set g the
+// slabs splits[g] (in: slab_split, out: that or 1) its last item takes:
+// store.hip.
+int64_t choose_slab(const int *items, int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
+                    size_t max_bytes, int64_t longest);
 int device_cus(int device);
 // FP64 sum of the S partials of every element and the NCC epilogue: store.hip.
 int launch_tri_reduce(const float *partials, int S, int nt, int count, const double *sum, const double *sumsq,

@@ -218,7 +218,7 @@ struct GramArgs {
     int M;
     int nt;  // tiles per side
     int T;   // work items per slab (variant 1: tiles in the upper triangle)
-    int ks;  // slabs the last of them takes at once (slab_split)
+    int ks;  // slabs the last of them takes at once
     int S;   // K slabs
     int xcd_remap;  // 1: the T items of a slab run on one XCD
 };
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(kGramThreads, 1) void gram_tile_kernel(GramArgs a) 
     if (!ItemIndex(a.T, a.ks, a.S).at(blockIdx.x, a.xcd_remap, u, s)) return;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    ItemWaves w = item_waves(u, a.M, __builtin_amdgcn_readfirstlane(tid >> 6));
+    ItemWaves w = item_waves(u, a.M, __builtin_amdgcn_readfirstlane(tid >> 6), a.ks);
     // wave-uniform: keep it in scalar registers
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -713,13 +713,13 @@ int launch_pair_ncc(const float *x, const float *y, int64_t n, double *d_out, Wo
 namespace {
 
 struct GramPlan {
-    int nt, T, ks, tiles;  // items per slab, the slabs of the last (slab_split), partial tiles per slab
+    int nt, T, ks, tiles;  // items per slab, the slabs the last takes, partial tiles per slab
     int64_t S, kchunk;
     int xcd_remap;
     int variant;
 };
 
-// K split of the Gram: `slabs` per tile (0: the slab length choose_kcb finds
+// K split of the Gram: `slabs` per tile (0: the slab length choose_slab finds
 // cheapest, no longer than about 5 workgroups per CU of whole tiles give at 16
 // stages and more, for the FP32 sums' precision), partials capped at 2 GiB.
 GramPlan plan_gram(const Context *c, int count, int precision) {
@@ -736,12 +736,13 @@ GramPlan plan_gram(const Context *c, int count, int precision) {
         int64_t S = std::min<int64_t>(c->gram_cfg[precision].slabs, stages);
         S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * p.tiles)));
         p.kchunk = ((stages + S - 1) / S) * kKT;
+        if (p.T * S <= device_cus(c->device)) p.ks = 1;  // (choose_slab)
     } else {
         int64_t S = std::max<int64_t>(1, (256 * 5 + p.tiles - 1) / p.tiles);
         S = std::min<int64_t>(S, std::max<int64_t>(1, stages / 16));
         S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * p.tiles)));
-        p.kchunk = kKT * choose_kcb(&p.T, &p.ks, &p.tiles, &stages, 1, device_cus(c->device), size_t(2) << 30,
-                                    (stages + S - 1) / S);
+        p.kchunk = kKT * choose_slab(&p.T, &p.ks, &p.tiles, &stages, 1, device_cus(c->device), size_t(2) << 30,
+                                     (stages + S - 1) / S);
     }
     p.S = (K + p.kchunk - 1) / p.kchunk;
     p.xcd_remap = c->gram_cfg[precision].xcd_remap;

@@ -5,15 +5,13 @@
 // H(k) = (C(k) + conj(C(-k)))/2 Hermitian, so IFFT2 of Z = H_a + i H_b gives
 // Re c_a + i Re c_b: two pairs share one complex transform.  Pipeline per
 // couple of pairs, inputs are R2C half spectra h x (w/2+1):
-//   1. pce_rows2_kernel  builds row i of Z and runs the inverse row FFT
-//                        (length w) in LDS;
-//   2. transpose         the row-pass output, so that a column is a
-//                        contiguous run of h values;
-//      pce_cols_kernel   one column per workgroup: inverse FFT (length h)
-//                        through fft_row, whose first pass loads the column
-//                        and whose last pass hands every output to the
-//                        per-column sums: the max |Re c| with its index and
-//                        sum (Re c)^2 in FP64 for each pair of the couple
+//   1. pce_rows_*        build rows u and h - u of Z and run their inverse row
+//                        FFTs (length w) in LDS;
+//   2. pce_cols_kernel   strips of adjacent columns of the row-pass output
+//                        through LDS (cols_device.hpp): inverse FFT (length h)
+//                        of each column, whose last pass hands every output to
+//                        the per-column sums: the max |Re c| with its index
+//                        and sum (Re c)^2 in FP64 for each pair of the couple
 //                        (the correlation planes themselves are never
 //                        written);
 //   3. pce_window_kernel per pair and window row: argmax over columns; the
@@ -32,6 +30,7 @@
 // the argmax with cyclic wrap; peak value = c at the argmax; sign kept.
 #include "prnu_internal.hpp"
 #include "fft_device.hpp"
+#include "cols_device.hpp"
 #include "fft_host.hpp"
 
 #include <algorithm>
@@ -166,9 +165,9 @@ __device__ __forceinline__ void herm_pair(const float2 *X, const float2 *Y, int 
 // batch; the second may be absent), inverse row FFT: the first pass reads
 // the Hermitian parts straight from the half spectra, the last pass writes
 // the row of A.  grid (16 ceil((h/2 + 1) / 8), couples), LDS w complex.
-template <int VARIANT, int MAXN>
-__global__ __launch_bounds__(kFftThreads) void pce_rows2_kernel(FftDesc d, int h, int nb, PceBatch bt,
-                                                                float2 *__restrict__ Aall, int64_t pstride) {
+template <int VARIANT, class R>
+__global__ __launch_bounds__(R::T) void pce_rows2_kernel(R pl, int h, int nb, PceBatch bt, float2 *__restrict__ Aall,
+                                                         int64_t pstride) {
     extern __shared__ float2 buf[];
     // Row i reads spectrum rows i and (h - i) mod h (the mirrored half of the
     // cross spectrum), and so does row (h - i) mod h: workgroups x and x + 8
@@ -183,14 +182,14 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows2_kernel(FftDesc d, int h
     const int i = side ? (h - u) % h : u;
     if (side && i == u) return;
     const int q = blockIdx.y;
-    const int w = d.n;
+    const int w = pl.n();
     const float2 *Xa, *Ya, *Xb = nullptr, *Yb = nullptr;
     pce_operands(bt, 2 * q, Xa, Ya);
     const bool two = 2 * q + 1 < nb;
     if (two) pce_operands(bt, 2 * q + 1, Xb, Yb);
     float2 *A = Aall + (int64_t)q * pstride + (int64_t)i * w;
-    fft_row<1, MAXN>(
-        buf, d,
+    pl.template run<1>(
+        buf,
         [&](int j) {
             const float2 ha = herm_at<VARIANT>(Xa, Ya, h, w, i, j);
             if (!two) return ha;
@@ -207,13 +206,13 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows2_kernel(FftDesc d, int h
 // in both variants), so its transform input is
 // Z(-u, j) = conj(H_a(u, -j)) + i conj(H_b(u, -j)).  That halves the
 // spectrum reads of pce_rows2_kernel, whose two workgroups per pair each
-// form their own row's Hermitian parts.  grid (h/2 + 1, couples), LDS 3w
-// complex (H_a, H_b of row u, the transform buffer).
-template <int VARIANT, int MAXN>
-__global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d, int h, int nb, PceBatch bt,
-                                                                      float2 *__restrict__ Aall, int64_t pstride) {
+// form their own row's Hermitian parts.  grid (h/2 + 1, couples), LDS 2w
+// complex and the transform buffer (H_a, H_b of row u).
+template <int VARIANT, class R>
+__global__ __launch_bounds__(R::T) void pce_rows_mirror_kernel(R pl, int h, int nb, PceBatch bt,
+                                                               float2 *__restrict__ Aall, int64_t pstride) {
     extern __shared__ float2 smem[];
-    const int w = d.n;
+    const int w = pl.n();
     float2 *ha = smem, *hb = smem + w, *buf = smem + 2 * w;
     const int u = blockIdx.x;
     if (u > h / 2) return;
@@ -223,7 +222,7 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d,
     pce_operands(bt, 2 * q, Xa, Ya);
     const bool two = 2 * q + 1 < nb;
     if (two) pce_operands(bt, 2 * q + 1, Xb, Yb);
-    for (int j = threadIdx.x; j <= w / 2; j += kFftThreads) {  // each spectrum value read once
+    for (int j = threadIdx.x; j <= w / 2; j += R::T) {  // each spectrum value read once
         float2 a, am, b = make_float2(0.f, 0.f), bm = make_float2(0.f, 0.f);
         herm_pair<VARIANT>(Xa, Ya, w, u, um, j, a, am);
         if (two) herm_pair<VARIANT>(Xb, Yb, w, u, um, j, b, bm);
@@ -236,16 +235,16 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d,
     }
     __syncthreads();
     float2 *A = Aall + (int64_t)q * pstride;
-    fft_row<1, MAXN>(
-        buf, d,
+    pl.template run<1>(
+        buf,
         [&](int j) {
             const float2 a = ha[j], b = hb[j];
             return make_float2(a.x - b.y, a.y + b.x);
         },
         [&](int j, float2 f) { A[(int64_t)u * w + j] = f; });
     if (um == u) return;
-    fft_row<1, MAXN>(
-        buf, d,
+    pl.template run<1>(
+        buf,
         [&](int j) {
             const int mj = j == 0 ? 0 : w - j;
             const float2 a = ha[mj], b = hb[mj];
@@ -254,80 +253,25 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d,
         [&](int j, float2 f) { A[(int64_t)um * w + j] = f; });
 }
 
-// Column j of couple blockIdx.y from the transposed row-pass output
-// (B[j*h + i] = A[i][j]): inverse FFT of length h; every output value goes
-// straight into this thread's sums of Re (pair 2q) and Im (pair 2q + 1) --
-// FP64 energy and the max |value| with its linear index i*w + j, smallest
-// index on ties -- which a fixed-order block reduction turns into the
-// column's partials.  grid (w, couples), LDS h complex.
-template <int MAXN>
-__global__ __launch_bounds__(kFftThreads) void pce_cols_kernel(FftDesc d, int w, int nb, const float2 *__restrict__ Ball,
-                                                               int64_t pstride, PeakPart *__restrict__ partall) {
-    extern __shared__ float2 buf[];
-    __shared__ double sh_e[2][4];
-    __shared__ float sh_v[2][4];
-    __shared__ int sh_i[2][4];
-    const int h = d.n, q = blockIdx.y, j = blockIdx.x;
-    const float2 *col = Ball + (int64_t)q * pstride + (int64_t)j * h;
-    double e0 = 0.0, e1 = 0.0;
-    float b0 = -1.0f, b1 = -1.0f;
-    int i0 = 0x7fffffff, i1 = 0x7fffffff;
-    fft_row<1, MAXN>(
-        buf, d, [&](int i) { return col[i]; },
-        [&](int i, float2 z) {
-            const int idx = i * w + j;
-            e0 += (double)z.x * (double)z.x;
-            e1 += (double)z.y * (double)z.y;
-            argmax_merge(b0, i0, fabsf(z.x), idx);
-            argmax_merge(b1, i1, fabsf(z.y), idx);
-        });
-    const int halves = 2 * q + 1 < nb ? 2 : 1;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    e0 = wave_sum_d(e0);
-    e1 = wave_sum_d(e1);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        float v2 = __shfl_xor(b0, off, 64);
-        int k2 = __shfl_xor(i0, off, 64);
-        argmax_merge(b0, i0, v2, k2);
-        v2 = __shfl_xor(b1, off, 64);
-        k2 = __shfl_xor(i1, off, 64);
-        argmax_merge(b1, i1, v2, k2);
-    }
-    if (lane == 0) {
-        sh_e[0][wave] = e0;
-        sh_e[1][wave] = e1;
-        sh_v[0][wave] = b0;
-        sh_v[1][wave] = b1;
-        sh_i[0][wave] = i0;
-        sh_i[1][wave] = i1;
-    }
-    __syncthreads();
-    const int t = threadIdx.x;
-    if (t < halves) {  // fixed-order merge of the 4 waves
-        PeakPart p;
-        p.energy = (sh_e[t][0] + sh_e[t][1]) + (sh_e[t][2] + sh_e[t][3]);
-        float best = sh_v[t][0];
-        int bi = sh_i[t][0];
-        for (int k = 1; k < 4; ++k) argmax_merge(best, bi, sh_v[t][k], sh_i[t][k]);
-        p.absmax = best;
-        p.index = bi;
-        partall[(int64_t)(2 * q + t) * w + j] = p;
-    }
-}
-
-// pce_rows_mirror_kernel for w = 1024 with one wave per row: the two waves
-// form H_a, H_b of row u into LDS together, then wave 0 transforms row u and
-// wave 1 row -u at the same time (fft_wave_1024), their transform buffers
-// laid over H_a, H_b once the first pass has read them.  When u is its own
-// mirror, wave 1 transforms and stores nothing of its own (it still takes
-// part in every barrier).  grid (h/2 + 1, couples), 128 threads.
-template <int VARIANT>
-__global__ __launch_bounds__(128) void pce_rows_mirror_wave_kernel(const float2 *__restrict__ tw, int h, int nb,
-                                                                   PceBatch bt, float2 *__restrict__ Aall,
-                                                                   int64_t pstride) {
-    constexpr int w = 1024;
-    __shared__ float2 smem[2 * fft_wave_lds(w)];
+// pce_rows_mirror_kernel for w = W = 1024 with one wave per row and W = 2048
+// with four: all waves form H_a, H_b of row u into LDS together, then the first
+// half transforms row u and the second row -u at the same time (the passes of
+// fft_wave_1024 / fft_block_2048_r8; two waves per row at 2048, radix 16, 16,
+// 8, round a little less well: 1.3e-7 against 1.1e-7 of the score), their transform buffers laid over H_a, H_b
+// once the first pass has read them.  When u is its own mirror, the second
+// half transforms and stores nothing of its own (it still takes part in every
+// barrier).  At 2048 columns each row by its own workgroup, reading its
+// Hermitian parts for itself, measured 597 us per 66 pairs of 2048x1536.
+// grid (h/2 + 1, couples), 2 T threads.
+template <int W>
+constexpr int mirror_row_threads() { return W == 1024 ? 64 : 256; }
+template <int VARIANT, int W>
+__global__ __launch_bounds__(2 * mirror_row_threads<W>()) void pce_rows_mirror_wave_kernel(const float2 *__restrict__ tw, int h, int nb,
+                                                                     PceBatch bt, float2 *__restrict__ Aall,
+                                                                     int64_t pstride) {
+    constexpr int w = W, T = mirror_row_threads<W>();  // threads per row
+    constexpr int kBuf = W == 1024 ? fft_wave_lds<1024>() : kFft2048PadLds;
+    __shared__ float2 smem[2 * kBuf];
     float2 *ha = smem, *hb = smem + w;
     const int u = blockIdx.x;
     const int um = (h - u) % h;
@@ -336,7 +280,7 @@ __global__ __launch_bounds__(128) void pce_rows_mirror_wave_kernel(const float2 
     pce_operands(bt, 2 * q, Xa, Ya);
     const bool two = 2 * q + 1 < nb;
     if (two) pce_operands(bt, 2 * q + 1, Xb, Yb);
-    for (int j = threadIdx.x; j <= w / 2; j += 128) {  // each spectrum value read once
+    for (int j = threadIdx.x; j <= w / 2; j += 2 * T) {  // each spectrum value read once
         float2 a, am, b = make_float2(0.f, 0.f), bm = make_float2(0.f, 0.f);
         herm_pair<VARIANT>(Xa, Ya, w, u, um, j, a, am);
         if (two) herm_pair<VARIANT>(Xb, Yb, w, u, um, j, b, bm);
@@ -348,13 +292,13 @@ __global__ __launch_bounds__(128) void pce_rows_mirror_wave_kernel(const float2 
         }
     }
     __syncthreads();
-    const int wave = threadIdx.x >> 6;
-    float2 *buf = smem + wave * fft_wave_lds(w);
+    const int half = threadIdx.x / T;
+    float2 *buf = smem + half * kBuf;
     float2 *A = Aall + (int64_t)q * pstride;
-    const int row = wave == 0 ? u : um;
-    const bool store = wave == 0 || um != u;
+    const int row = half == 0 ? u : um;
+    const bool store = half == 0 || um != u;
     auto get = [&](int j) {
-        if (wave == 0) {
+        if (half == 0) {
             const float2 a = ha[j], b = hb[j];
             return make_float2(a.x - b.y, a.y + b.x);
         }
@@ -365,36 +309,59 @@ __global__ __launch_bounds__(128) void pce_rows_mirror_wave_kernel(const float2 
     auto put = [&](int j, float2 f) {
         if (store) A[(int64_t)row * w + j] = f;
     };
-    // fft_wave_1024's passes; the first with workgroup barriers (both waves
-    // read H_a, H_b, which their buffers overlay), the others each in its
-    // own buffer with wave-level ordering
-    fft_wave_pass<16, 1, true, false, 1024, 1, true>(buf, tw, get, put);
-    fft_wave_pass<16, 1, false, false, 1024, 16, false, 4, 64, true>(buf, tw, get, put);
-    fft_wave_pass<4, 1, false, true, 1024, 256, false, 4, 64, true>(buf, tw, get, put);
+    // the first pass with workgroup barriers (every wave reads H_a, H_b, which
+    // the buffers overlay); at 1024 the others each in its wave's own buffer
+    // with wave-level ordering
+    if constexpr (W == 1024) {
+        fft_wave_pass<16, 1, true, false, 1024, 1, true>(buf, tw, get, put);
+        fft_wave_pass<16, 1, false, false, 1024, 16, false, 4, 64, true>(buf, tw, get, put);
+        fft_wave_pass<4, 1, false, true, 1024, 256, false, 4, 64, true>(buf, tw, get, put);
+    } else {
+        static_assert(W == 2048, "pce_rows_mirror_wave_kernel: rows of 1024 or 2048");
+        fft_wave_pass<8, 1, true, false, 2048, 1, true, 3, 256>(buf, tw, get, put);
+        fft_wave_pass<8, 1, false, false, 2048, 8, false, 3, 256>(buf, tw, get, put);
+        fft_wave_pass<8, 1, false, false, 2048, 64, false, 3, 256>(buf, tw, get, put);
+        fft_wave_pass<4, 1, false, true, 2048, 512, false, 3, 256>(buf, tw, get, put);
+    }
 }
 
-// pce_cols_kernel for h = 1024 with one wave per column (fft_wave_1024: 16
-// values per lane, radix 16, 16, 4): every lane works in every pass and the
-// barriers between passes are one wave's.  Same sums; the FP64 energy is
-// added in another order (one wave's lanes instead of four waves' partials).
-__global__ __launch_bounds__(64) void pce_cols_wave_kernel(const float2 *__restrict__ tw, int w, int nb,
-                                                           const float2 *__restrict__ Ball, int64_t pstride,
-                                                           PeakPart *__restrict__ partall) {
-    __shared__ float2 buf[fft_wave_lds(1024)];
-    const int q = blockIdx.y, j = blockIdx.x;
-    const float2 *col = Ball + (int64_t)q * pstride + (int64_t)j * 1024;
+// Columns of couple blockIdx.y's row-pass output A (h x w, row-major) by
+// strips (cols_device.hpp): inverse FFT of length h; every output value goes
+// straight into its thread's sums of Re (pair 2q) and Im (pair 2q + 1) -- FP64
+// energy and the max |value| with its linear index i*w + j, smallest index on
+// ties -- which a fixed-order reduction over the column's waves turns into the
+// column's partials.  grid (8 per, couples).
+template <class P>
+__global__ __launch_bounds__(P::kThreads) void pce_cols_kernel(P pl, int w, int nb, const float2 *__restrict__ Aall,
+                                                               int64_t pstride, PeakPart *__restrict__ partall,
+                                                               int per) {
+    extern __shared__ __attribute__((aligned(16))) float2 pce_smem[];
+    const int strip = cols_strip<P>(per);
+    if (strip >= (w + P::COLS - 1) / P::COLS) return;
+    const int q = blockIdx.y, j0 = strip * P::COLS;
+    stage_cols(pl, Aall + (int64_t)q * pstride, w, j0, w, pce_smem);
+    const int c = (int)threadIdx.x / P::T, j = j0 + c;
+    float2 *buf = pce_smem + c * pl.stride();
     double e0 = 0.0, e1 = 0.0;
     float b0 = -1.0f, b1 = -1.0f;
     int i0 = 0x7fffffff, i1 = 0x7fffffff;
-    fft_wave_1024<1>(
-        buf, tw, [&](int i) { return col[i]; },
-        [&](int i, float2 z) {
-            const int idx = i * w + j;
-            e0 += (double)z.x * (double)z.x;
-            e1 += (double)z.y * (double)z.y;
-            argmax_merge(b0, i0, fabsf(z.x), idx);
-            argmax_merge(b1, i1, fabsf(z.y), idx);
-        });
+    constexpr int kWaves = P::T / 64;  // of a column
+    const int t = (int)threadIdx.x & (P::T - 1);
+    auto add = [&](int i, float2 z) {
+        const int idx = i * w + j;
+        e0 += (double)z.x * (double)z.x;
+        e1 += (double)z.y * (double)z.y;
+        argmax_merge(b0, i0, fabsf(z.x), idx);
+        argmax_merge(b1, i1, fabsf(z.y), idx);
+    };
+    if constexpr (P::kConst) {
+        pl.template run<1, true>(buf, [&](int i) { return buf[pl.pad(i)]; }, add);
+    } else {  // the sums inside every radix's last pass would spill: through LDS once more
+        pl.template run<1, true>(
+            buf, [&](int i) { return buf[pl.pad(i)]; }, [&](int i, float2 z) { buf[pl.pad(i)] = z; });
+        for (int i = t; i < pl.n(); i += P::T) add(i, buf[pl.pad(i)]);
+        if constexpr (kWaves > 1) __syncthreads();
+    }
     e0 = wave_sum_d(e0);
     e1 = wave_sum_d(e1);
 #pragma unroll
@@ -406,81 +373,30 @@ __global__ __launch_bounds__(64) void pce_cols_wave_kernel(const float2 *__restr
         k2 = __shfl_xor(i1, off, 64);
         argmax_merge(b1, i1, v2, k2);
     }
-    const int t = threadIdx.x;
     const int halves = 2 * q + 1 < nb ? 2 : 1;
-    if (t < halves) {
+    if constexpr (kWaves > 1) {  // every wave has read its column
+        PeakPart *sh = reinterpret_cast<PeakPart *>(buf);
+        if ((t & 63) < 2) {
+            PeakPart &p = sh[2 * (t >> 6) + (t & 63)];
+            p.energy = (t & 63) == 0 ? e0 : e1;
+            p.absmax = (t & 63) == 0 ? b0 : b1;
+            p.index = (t & 63) == 0 ? i0 : i1;
+        }
+        __syncthreads();
+        if (t < halves && j < w) {
+            PeakPart p = sh[t];
+            for (int k = 1; k < kWaves; ++k) {
+                p.energy += sh[2 * k + t].energy;
+                argmax_merge(p.absmax, p.index, sh[2 * k + t].absmax, sh[2 * k + t].index);
+            }
+            partall[(int64_t)(2 * q + t) * w + j] = p;
+        }
+    } else if (t < halves && j < w) {
         PeakPart p;
         p.energy = t == 0 ? e0 : e1;
         p.absmax = t == 0 ? b0 : b1;
         p.index = t == 0 ? i0 : i1;
         partall[(int64_t)(2 * q + t) * w + j] = p;
-    }
-}
-
-// pce_cols_wave_kernel for h = 1024 reading the row-major row-pass output A
-// itself, so no transpose precedes it: a workgroup of 8 waves stages a strip
-// of 8 adjacent columns into LDS (every load a 64-byte piece of a row, each
-// column in its own padded buffer), then wave c transforms column c there.
-// Workgroup g takes strip (g mod 8) * per + g / 8, so that neighbouring strips
-// (the two halves of a 128-byte line) run on one XCD.  grid (8 per, couples).
-constexpr int kStripBuf = 1092;  // fft_wave_lds(1024) = 1088, +4 spreads the staging writes over banks
-__global__ __launch_bounds__(512) void pce_cols_strip_kernel(const float2 *__restrict__ tw, int w, int nb,
-                                                             const float2 *__restrict__ Aall, int64_t pstride,
-                                                             PeakPart *__restrict__ partall, int per) {
-    __shared__ __attribute__((aligned(16))) float2 lds[8 * kStripBuf];
-    const int g = blockIdx.x;
-    const int strip = (g & 7) * per + (g >> 3);
-    if (strip >= w / 8) return;
-    const int q = blockIdx.y;
-    const int j0 = strip * 8;
-    const float2 *A = Aall + (int64_t)q * pstride;
-    const int t = (int)threadIdx.x;
-    {
-        // two adjacent columns per thread, one 16-byte load (w and j0 even)
-        const int c2 = (t & 3) * 2, r = t >> 2;
-#pragma unroll 4
-        for (int k = 0; k < 1024 / 128; ++k) {
-            const int i = r + 128 * k;
-            const float4 v = *reinterpret_cast<const float4 *>(A + (int64_t)i * w + j0 + c2);
-            lds[c2 * kStripBuf + fft_wave_pad<4>(i)] = make_float2(v.x, v.y);
-            lds[(c2 + 1) * kStripBuf + fft_wave_pad<4>(i)] = make_float2(v.z, v.w);
-        }
-    }
-    __syncthreads();
-    const int wave = t >> 6;
-    float2 *buf = lds + wave * kStripBuf;
-    const int j = j0 + wave;
-    double e0 = 0.0, e1 = 0.0;
-    float b0 = -1.0f, b1 = -1.0f;
-    int i0 = 0x7fffffff, i1 = 0x7fffffff;
-    fft_wave_1024<1, true, true>(  // after the staging barrier each wave works in its own buffer
-        buf, tw, [&](int i) { return buf[fft_wave_pad<4>(i)]; },
-        [&](int i, float2 z) {
-            const int idx = i * w + j;
-            e0 += (double)z.x * (double)z.x;
-            e1 += (double)z.y * (double)z.y;
-            argmax_merge(b0, i0, fabsf(z.x), idx);
-            argmax_merge(b1, i1, fabsf(z.y), idx);
-        });
-    e0 = wave_sum_d(e0);
-    e1 = wave_sum_d(e1);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        float v2 = __shfl_xor(b0, off, 64);
-        int k2 = __shfl_xor(i0, off, 64);
-        argmax_merge(b0, i0, v2, k2);
-        v2 = __shfl_xor(b1, off, 64);
-        k2 = __shfl_xor(i1, off, 64);
-        argmax_merge(b1, i1, v2, k2);
-    }
-    const int lane = t & 63;
-    const int halves = 2 * q + 1 < nb ? 2 : 1;
-    if (lane < halves) {
-        PeakPart p;
-        p.energy = lane == 0 ? e0 : e1;
-        p.absmax = lane == 0 ? b0 : b1;
-        p.index = lane == 0 ? i0 : i1;
-        partall[(int64_t)(2 * q + lane) * w + j] = p;
     }
 }
 
@@ -661,6 +577,36 @@ __global__ __launch_bounds__(64) void pce_score_kernel(const double *__restrict_
     outall[base + p] = pce;
 }
 
+template <int V>
+int launch_pce_rows(const FftDesc &dw, dim3 mgrid, dim3 rgrid, int h, int nb, const PceBatch &bt, float2 *A,
+                    int64_t pstride, hipStream_t st) {
+    if (dw.n == 1024) {
+        hipLaunchKernelGGL((pce_rows_mirror_wave_kernel<V, 1024>), mgrid, dim3(128), 0, st, dw.tw, h, nb, bt, A,
+                           pstride);
+    } else if (dw.n == 2048) {
+        hipLaunchKernelGGL((pce_rows_mirror_wave_kernel<V, 2048>), mgrid, dim3(512), 0, st, dw.tw, h, nb, bt, A,
+                           pstride);
+    } else if (dw.n == 1536) {
+        const RowC<1536> pl{dw.tw};
+        hipLaunchKernelGGL((pce_rows_mirror_kernel<V, RowC<1536>>), mgrid, dim3(pl.T),
+                           2 * sizeof(float2) * dw.n + pl.smem(), st, pl, h, nb, bt, A, pstride);
+    } else if (dw.n < 2048) {
+        const RowRt<256> pl{dw};
+        hipLaunchKernelGGL((pce_rows_mirror_kernel<V, RowRt<256>>), mgrid, dim3(pl.T),
+                           2 * sizeof(float2) * dw.n + pl.smem(), st, pl, h, nb, bt, A, pstride);
+    } else if (dw.n <= 4096) {
+        const RowRt<512> pl{dw};
+        hipLaunchKernelGGL((pce_rows2_kernel<V, RowRt<512>>), rgrid, dim3(pl.T), pl.smem(), st, pl, h, nb, bt, A,
+                           pstride);
+    } else {
+        const RowRt<1024> pl{dw};
+        hipLaunchKernelGGL((pce_rows2_kernel<V, RowRt<1024>>), rgrid, dim3(pl.T), pl.smem(), st, pl, h, nb, bt, A,
+                           pstride);
+    }
+    PRNU_CHECK_LAUNCH();
+    return PRNU_OK;
+}
+
 int pce_batch(Context *c, int variant, const PceBatch &bt, int nb, double *out, hipStream_t st) {
     const int h = c->h, w = c->w;
     const int64_t n = c->pixels();
@@ -669,63 +615,28 @@ int pce_batch(Context *c, int variant, const PceBatch &bt, int nb, double *out, 
     const size_t pbytes = ((sizeof(PeakPart) * w) + 255) & ~size_t(255);
     const int64_t pstride = (int64_t)(plane / sizeof(float2));
     const size_t wbytes = ((sizeof(double) * kWinSlots * nb) + 255) & ~size_t(255);
-    PRNU_TRY(c->ws_pce.ensure(2 * plane * couples + pbytes * nb + wbytes));
+    PRNU_TRY(c->ws_pce.ensure(plane * couples + pbytes * nb + wbytes));
     char *base = static_cast<char *>(c->ws_pce.ptr);
-    float2 *A = reinterpret_cast<float2 *>(base);                  // row-pass output, h x w per couple
-    float2 *B = reinterpret_cast<float2 *>(base + plane * couples);  // its transpose, w x h per couple
-    PeakPart *part = reinterpret_cast<PeakPart *>(base + 2 * plane * couples);
-    double *wbuf = reinterpret_cast<double *>(base + 2 * plane * couples + pbytes * nb);
-    const FftDesc &dw = fft_desc(c->fft_w);
+    float2 *A = reinterpret_cast<float2 *>(base);  // row-pass output, h x w per couple
+    PeakPart *part = reinterpret_cast<PeakPart *>(base + plane * couples);
+    double *wbuf = reinterpret_cast<double *>(base + plane * couples + pbytes * nb);
+    const FftDesc &dw = fft_desc_basic(c->fft_w);
     const FftDesc &dh = fft_desc(c->fft_h);
     const dim3 rgrid((unsigned)((h / 2 + 1 + 7) / 8 * 16), couples);  // mirror pairs of rows (pce_rows2_kernel)
-    const size_t rsm = fft_row_smem(w);
-    // rows up to 1024: both rows of a mirror pair in one workgroup (24 KiB of LDS)
-    const bool mirror = w <= 1024;
+    // rows up to 2048: both rows of a mirror pair in one workgroup (at most 50
+    // KiB of LDS, three workgroups per CU)
     const dim3 mgrid((unsigned)(h / 2 + 1), couples);
-    const size_t msm = 3 * sizeof(float2) * (size_t)w;
-#define PRNU_PCE_ROWS(V, M)                                                                                          \
-    do {                                                                                                             \
-        if (w == 1024)                                                                                               \
-            hipLaunchKernelGGL((pce_rows_mirror_wave_kernel<V>), mgrid, dim3(128), 0, st, dw.tw, h, nb, bt, A,       \
-                               pstride);                                                                             \
-        else if (mirror)                                                                                             \
-            hipLaunchKernelGGL((pce_rows_mirror_kernel<V, M>), mgrid, dim3(kFftThreads), msm, st, dw, h, nb, bt, A, \
-                               pstride);                                                                             \
-        else                                                                                                         \
-            hipLaunchKernelGGL((pce_rows2_kernel<V, M>), rgrid, dim3(kFftThreads), rsm, st, dw, h, nb, bt, A,       \
-                               pstride);                                                                             \
-    } while (0)
-    if (variant == PRNU_PCE_REFERENCE) {
-        if (w <= kFftSmallN) PRNU_PCE_ROWS(PRNU_PCE_REFERENCE, kFftSmallN);
-        else if (w <= kFftMidN) PRNU_PCE_ROWS(PRNU_PCE_REFERENCE, kFftMidN);
-        else PRNU_PCE_ROWS(PRNU_PCE_REFERENCE, kFftMaxN);
-    } else {
-        if (w <= kFftSmallN) PRNU_PCE_ROWS(PRNU_PCE_TEXTBOOK, kFftSmallN);
-        else if (w <= kFftMidN) PRNU_PCE_ROWS(PRNU_PCE_TEXTBOOK, kFftMidN);
-        else PRNU_PCE_ROWS(PRNU_PCE_TEXTBOOK, kFftMaxN);
-    }
-#undef PRNU_PCE_ROWS
-    PRNU_CHECK_LAUNCH();
-    const dim3 cgrid(w, couples);
-    const size_t csm = fft_row_smem(h);
-    const bool strips = h == 1024 && w % 8 == 0;
-    if (!strips) PRNU_TRY(launch_transpose_c(A, B, h, w, couples, pstride, st));
-    if (strips) {
-        const int per = (w / 8 + 7) / 8;
-        hipLaunchKernelGGL(pce_cols_strip_kernel, dim3(8 * per, couples), dim3(512), 0, st, dh.tw, w, nb, A, pstride,
-                           part, per);
-    } else if (h == 1024)
-        hipLaunchKernelGGL(pce_cols_wave_kernel, cgrid, dim3(64), 0, st, dh.tw, w, nb, B, pstride, part);
-    else if (h <= kFftSmallN)
-        hipLaunchKernelGGL((pce_cols_kernel<kFftSmallN>), cgrid, dim3(kFftThreads), csm, st, dh, w, nb, B, pstride,
-                           part);
-    else if (h <= kFftMidN)
-        hipLaunchKernelGGL((pce_cols_kernel<kFftMidN>), cgrid, dim3(kFftThreads), csm, st, dh, w, nb, B, pstride,
-                           part);
-    else
-        hipLaunchKernelGGL((pce_cols_kernel<kFftMaxN>), cgrid, dim3(kFftThreads), csm, st, dh, w, nb, B, pstride,
-                           part);
-    PRNU_CHECK_LAUNCH();
+    PRNU_TRY(variant == PRNU_PCE_REFERENCE
+                 ? launch_pce_rows<PRNU_PCE_REFERENCE>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st)
+                 : launch_pce_rows<PRNU_PCE_TEXTBOOK>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st));
+    PRNU_TRY(with_cols_plan(dh, [&](auto pl) -> int {
+        typedef decltype(pl) Plan;
+        const int per = cols_per<Plan>(w);
+        hipLaunchKernelGGL(pce_cols_kernel<Plan>, dim3(8 * per, couples), dim3(Plan::kThreads), cols_lds(pl), st, pl, w,
+                           nb, A, pstride, part, per);
+        PRNU_CHECK_LAUNCH();
+        return PRNU_OK;
+    }));
     // window rows (and, for the reference variant, the last element's value)
     const dim3 wgrid_ref(nb, kSquare + 1), wgrid_txt(nb, kSquare), sgrid((nb + 63) / 64);
     hipLaunchKernelGGL(pce_peak_kernel, dim3(nb), dim3(256), 0, st, part, h, w, wbuf);
@@ -774,7 +685,7 @@ int run_pce_pairs(Context *c, int variant, const void *const *d_tab, const int *
         // about 2 GiB of planes: 256 pairs of 1024x1024 (a sweep of 8 to 2048
         // pairs there peaks at 256; smaller batches pay each launch's ramp and
         // tail more often, larger ones lose the planes' L2 and cache reuse)
-        const int64_t per = 8 * c->pixels();  // half of a couple's complex plane and of its transpose per pair
+        const int64_t per = 8 * c->pixels();
         batch = (int)std::max<int64_t>(2, std::min<int64_t>(512, (int64_t(2) << 30) / per)) & ~1;
     }
     time_begin(c, st);

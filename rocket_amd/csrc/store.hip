@@ -271,7 +271,7 @@ struct StoreGramArgs {
     int64_t kcb;         // blocks per slab
     int first, count;
     int nt, T, S;        // T: work items per slab
-    int ks;              // slabs the last of them takes at once (slab_split)
+    int ks;              // slabs the last of them takes at once
     int xcd_remap;
 };
 
@@ -692,12 +692,12 @@ __device__ __forceinline__ void gram_item(const uint8_t *__restrict__ blocks, in
 // [first, first+count).
 template <int FMT, int VAR>
 __device__ __forceinline__ void run_item(const uint8_t *blocks, int64_t cap_bytes, int first, int count, int first_b,
-                                         int count_b, int ntb, int S, int64_t nkb, int64_t kcb,
+                                         int count_b, int ntb, int ks, int S, int64_t nkb, int64_t kcb,
                                          float *partials, int u, int s, uint8_t *lds, int tid = threadIdx.x) {
     constexpr bool kRing = FMT == PRNU_PREC_FP16 && VAR != 1;
     // wave-uniform: keep it in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    ItemWaves w = ntb > 0 ? rect_waves(u, ntb, wave) : item_waves(u, count, wave);
+    ItemWaves w = ntb > 0 ? rect_waves(u, ntb, wave) : item_waves(u, count, wave, ks);
 #pragma unroll
     for (int k = 0; k < 4; ++k) w.q[k] = __builtin_amdgcn_readfirstlane(w.q[k]);
     w.nq = __builtin_amdgcn_readfirstlane(w.nq);
@@ -724,12 +724,8 @@ __device__ __forceinline__ void run_item(const uint8_t *blocks, int64_t cap_byte
         return;
     }
     const int64_t b_end = min(nkb, b_begin + kcb);
-    if constexpr (kRing)
-        gram_item_fp16<false, VAR == 2>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, b_end, kcb, out,
-                                        rows, cols, ntb == 0, lds, tid);
-    else
-        gram_item<FMT, VAR, false>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, b_end, kcb, out,
-                                   rows, cols, ntb == 0, lds, tid);
+    gram_item<FMT, VAR, false>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, b_end, kcb, out, rows,
+                               cols, ntb == 0, lds, tid);
 }
 
 // ------------------------------------------------ 4-wave split-BF16 item
@@ -970,7 +966,7 @@ __global__ __launch_bounds__(kThrS, 1) void store_gram_kernel(StoreGramArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[item_lds<FMT, VAR>()];
     int u, s;
     if (!ItemIndex(a.T, a.ks, a.S).at(blockIdx.x, a.xcd_remap, u, s)) return;
-    run_item<FMT, VAR>(a.blocks, a.cap_bytes, a.first, a.count, a.first, a.count, 0, a.S, a.nkb, a.kcb,
+    run_item<FMT, VAR>(a.blocks, a.cap_bytes, a.first, a.count, a.first, a.count, 0, a.ks, a.S, a.nkb, a.kcb,
                        a.partials, u, s, lds);
 }
 
@@ -988,7 +984,7 @@ struct GroupDev {
     int64_t cap_bytes, nkb, kcb, v_begin;
     int first, count, nt, T, S;
     int first_b, count_b, ntb;  // ntb > 0: rectangle rows x [first_b, first_b+count_b)
-    int ks;                     // slab_split of a triangle, 1 for a rectangle
+    int ks;                     // slabs the last item of a slab takes at once
 };
 
 template <int FMT, int VAR>
@@ -1005,7 +1001,7 @@ __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_kernel(const Group
     const GroupDev &g = groups[lo];
     int u, s;
     if (!ItemIndex(g.T, g.ks, g.S).at(v - g.v_begin, true, u, s)) return;  // padding item
-    run_item<FMT, VAR>(g.blocks, g.cap_bytes, g.first, g.count, g.first_b, g.count_b, g.ntb, g.S, g.nkb,
+    run_item<FMT, VAR>(g.blocks, g.cap_bytes, g.first, g.count, g.first_b, g.count_b, g.ntb, g.ks, g.S, g.nkb,
                        g.kcb, g.partials, u, s, lds);
 }
 
@@ -1055,7 +1051,7 @@ __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_persistent_kernel(
         // hoisted out of this loop (they would stay live across every item)
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
-        run_item<FMT, 0>(g.blocks, g.cap_bytes, g.first, g.count, g.first_b, g.count_b, g.ntb, g.S, g.nkb,
+        run_item<FMT, 0>(g.blocks, g.cap_bytes, g.first, g.count, g.first_b, g.count_b, g.ntb, g.ks, g.S, g.nkb,
                          g.kcb, g.partials, u, s, lds, tid);
     }
 }
@@ -1197,8 +1193,8 @@ int device_cus(int device) {
 // Searches kcb and returns the cheapest whose partial tiles fit `max_bytes`.
 // `longest` (if > 0) bounds the slab: an FP32 accumulator's rounding error
 // grows with it.
-int64_t choose_kcb(const int *items, const int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
-                   size_t max_bytes, int64_t longest) {
+static int64_t choose_kcb(const int *items, const int *splits, const int *tiles, const int64_t *nkb, int ngroups,
+                          int cus, size_t max_bytes, int64_t longest, double *best_cost) {
     int64_t max_nkb = 1;
     for (int g = 0; g < ngroups; ++g) max_nkb = std::max(max_nkb, nkb[g]);
     double best = 1e300;
@@ -1219,17 +1215,26 @@ int64_t choose_kcb(const int *items, const int *splits, const int *tiles, const 
             best_kcb = kcb;
         }
     }
+    *best_cost = best;
     return best_kcb;
 }
 
-// The slab of a set of triangles and rectangles: no longer than the cheapest
-// one with every item taking one slab at a time, so that items of several
-// slabs shorten the launch and not the sums' precision.
-int64_t choose_slab(const int *items, const int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
-                    size_t max_bytes) {
+// The slab of a set of triangles and rectangles: the cheapest with every item
+// taking one slab at a time, or a shorter one whose split items cost less (not
+// longer: items of several slabs are there to shorten the launch, not at the
+// price of the sums' precision).  A set that does not fill the CUs keeps one
+// slab per item: its launch is one item's length either way, and an item of
+// four slabs loads four times the rows (3 patterns of 162x72: 81 us a call,
+// 92 with split items).
+int64_t choose_slab(const int *items, int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
+                    size_t max_bytes, int64_t longest) {
     const std::vector<int> one(ngroups, 1);
-    const int64_t longest = choose_kcb(items, one.data(), tiles, nkb, ngroups, cus, max_bytes, 0);
-    return choose_kcb(items, splits, tiles, nkb, ngroups, cus, max_bytes, longest);
+    double cost_one = 0.0, cost = 0.0;
+    const int64_t kcb_one = choose_kcb(items, one.data(), tiles, nkb, ngroups, cus, max_bytes, longest, &cost_one);
+    const int64_t kcb = choose_kcb(items, splits, tiles, nkb, ngroups, cus, max_bytes, kcb_one, &cost);
+    if (cost < cost_one) return kcb;
+    std::copy(one.begin(), one.end(), splits);
+    return kcb_one;
 }
 
 int store_create(int64_t n, int capacity, int format, Store **out) {
@@ -1355,9 +1360,10 @@ int store_gram_ncc(Context *c, Store *s, int first, int count, double *d_ncc, hi
         int64_t S = std::min<int64_t>(cfg.slabs, s->nkb);
         S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * tiles)));
         a.kcb = (s->nkb + S - 1) / S;
+        if (a.T * S <= device_cus(c->device)) a.ks = 1;  // (choose_slab)
     } else {
         const int64_t nkb = s->nkb;
-        a.kcb = choose_slab(&a.T, &a.ks, &tiles, &nkb, 1, device_cus(c->device), size_t(2) << 30);
+        a.kcb = choose_slab(&a.T, &a.ks, &tiles, &nkb, 1, device_cus(c->device), size_t(2) << 30, 0);
     }
     a.S = (int)((s->nkb + a.kcb - 1) / a.kcb);
     a.xcd_remap = cfg.xcd_remap;
@@ -1429,6 +1435,7 @@ struct GramPlan {
     int64_t v_total = 0, items = 0;  // workgroups launched, work items (padding excluded)
     int cus = 0;
     int var = 0;                     // load variant (the context's config of the format)
+    bool split = true;               // last items take several slabs where they can
     int persistent = 0;              // 1: one workgroup per CU takes items from per-XCD queues
     int *queue = nullptr;            // 8 counters, 64 bytes apart
     double flop = 0.0;               // one product over every block (triangles incl. diagonal)
@@ -1457,7 +1464,12 @@ int plan_layout(GramPlan *p, int64_t kcb) {
     plan_drop_graph(p);
     const int64_t tile_elems = (int64_t)kTileS * kTileS;
     std::vector<GroupDev> gd(p->groups.size());
-    int64_t v = 0, items = 0, part = 0;
+    int64_t v = 0, items = 0, part = 0, whole = 0;
+    for (const PlanBlock &g : p->groups) {
+        const int64_t k = std::min<int64_t>(kcb, g.store->nkb);
+        whole += g.items() * ((g.store->nkb + k - 1) / k);
+    }
+    const bool split = p->split && whole > p->cus;  // (choose_slab)
     for (size_t i = 0; i < p->groups.size(); ++i) {
         const PlanBlock &g = p->groups[i];
         const Store *s = g.store;
@@ -1476,7 +1488,7 @@ int plan_layout(GramPlan *p, int64_t kcb) {
         d.S = (int)((s->nkb + d.kcb - 1) / d.kcb);
         d.v_begin = v;
         d.partials = reinterpret_cast<float *>((uintptr_t)part);  // offset for now
-        d.ks = g.split();
+        d.ks = split ? g.split() : 1;
         v += ItemIndex(d.T, d.ks, d.S).ids(true);
         items += ItemIndex(d.T, d.ks, d.S).items();
         part += tile_elems * sizeof(float) * g.tiles() * d.S;
@@ -1510,7 +1522,7 @@ int plan_layout(GramPlan *p, int64_t kcb) {
 }
 
 // Default slab: the cheapest by the rounds model of choose_kcb.
-int64_t plan_default_kcb(const GramPlan *p) {
+int64_t plan_default_kcb(GramPlan *p) {
     std::vector<int> items, splits, tiles;
     std::vector<int64_t> nkb;
     for (const PlanBlock &g : p->groups) {
@@ -1519,8 +1531,10 @@ int64_t plan_default_kcb(const GramPlan *p) {
         tiles.push_back(g.tiles());
         nkb.push_back(g.store->nkb);
     }
-    return choose_slab(items.data(), splits.data(), tiles.data(), nkb.data(), (int)items.size(), p->cus,
-                       kPlanPartialCap);
+    const int64_t kcb = choose_slab(items.data(), splits.data(), tiles.data(), nkb.data(), (int)items.size(), p->cus,
+                                    kPlanPartialCap, 0);
+    p->split = std::any_of(splits.begin(), splits.end(), [](int k) { return k > 1; });
+    return kcb;
 }
 
 // Persistent launch: one workgroup per CU, a multiple of 8 so blockIdx.x & 7

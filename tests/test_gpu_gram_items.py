@@ -29,7 +29,7 @@ def tolerance(fmt, n):
 
 
 @pytest.mark.parametrize("fmt", ["split_bf16", "fp32", "fp16", "fp8"])
-@pytest.mark.parametrize("count,h,w", [(1, 8, 9), (5, 20, 21), (120, 64, 67), (128, 100, 100), (300, 61, 50),
+@pytest.mark.parametrize("count,h,w", [(1, 8, 9), (5, 20, 21), (120, 164, 167), (128, 100, 100), (300, 161, 150),
                                        (384, 33, 64), (600, 40, 41), (1100, 30, 31)])
 def test_items(fmt, count, h, w):
     p = patterns(count, h, w, 4, seed=900 + count, gain=0.3)
@@ -38,7 +38,7 @@ def test_items(fmt, count, h, w):
     gram = csi.GramNCC(h, w)
     store = csi.PatternStore(h * w, count + 2, fmt)
     store.put(p, first_slot=2)
-    for slabs in (0, 1, 3, 7):
+    for slabs in (0, 1, 3, 7, 300):
         cfg = (ctypes.c_int32 * 3)(slabs, 1, 0)
         _lib.call("prnu_gram_set_config", gram._ctx.handle, _lib.PRECISIONS[fmt], cfg)
         got = store.gram(gram, count, 2).cpu().numpy()
@@ -50,11 +50,12 @@ def test_items(fmt, count, h, w):
     gram.close()
 
 
-@pytest.mark.parametrize("slab_blocks", [1, 4, 9])
+@pytest.mark.parametrize("slab_blocks", [1, 4, 9, 40])
 def test_split_item_keeps_the_slabs(slab_blocks):
     """The same slabs give the same bits whether a pair lies in a set of one
-    quarter (four slabs at once) or of two (one at a time)."""
-    h, w, n = 40, 44, 40 * 44
+    quarter (four slabs at once, where there are more slabs than CUs) or of two
+    (one at a time)."""
+    h, w, n = 240, 440, 240 * 440
     p = patterns(200, h, w, 4, seed=77, gain=0.3)
     gram = csi.GramNCC(h, w)
     store = csi.PatternStore(n, 200, "split_bf16")
