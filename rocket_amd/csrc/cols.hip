@@ -34,14 +34,14 @@ __global__ __launch_bounds__(P::kThreads) void cols_power_kernel(P pl, const flo
         });
 }
 
-// Column r of B (r <= R/2) times S'(r, c) = (S(r, c) + S((R - r) % R,
-// (C - c) % C)) / 2 from the full R x C scale S (R = w, C = h), inverse FFT,
-// into A's columns.  grid (8 per, frames)
+// Column r of B times its row of the scale S (column 0: the mean of S(0, c) and
+// S(0, -c), which the other rows hold already), inverse FFT, into A's columns.
+// grid (8 per, frames)
 template <class P>
 __global__ __launch_bounds__(P::kThreads) void cols_inverse_kernel(P pl, const float2 *__restrict__ B,
-                                                                    const float *__restrict__ S, int R, int wh,
-                                                                    float2 *__restrict__ A, int lda, int64_t plane,
-                                                                    int per) {
+                                                                   const float *__restrict__ S, int wh,
+                                                                   float2 *__restrict__ A, int lda, int64_t plane,
+                                                                   int per) {
     extern __shared__ __attribute__((aligned(16))) float2 cols_smem[];
     const int strip = cols_strip<P>(per);
     if (strip >= (wh + P::COLS - 1) / P::COLS) return;
@@ -51,9 +51,12 @@ __global__ __launch_bounds__(P::kThreads) void cols_inverse_kernel(P pl, const f
     float2 *buf = cols_smem + c * pl.stride();
     const float2 *row = B + (int64_t)blockIdx.y * plane + (int64_t)col * n;
     const float *srow = S + (int64_t)blockIdx.y * plane + (int64_t)col * n;
-    const float *mrow = S + (int64_t)blockIdx.y * plane + (int64_t)(col == 0 ? 0 : R - col) * n;
+    // column 0 is its own mirror; the others add their own value again (no branch
+    // around the loads, which then stay batched)
+    const int flip = col == 0 ? -1 : 1, at = col == 0 ? n : 0;
     pl.template run<1, false>(
-        buf, [&](int j) { return cscale(row[j], 0.5f * (srow[j] + mrow[j == 0 ? 0 : n - j])); },
+        buf,
+        [&](int j) { return cscale(row[j], 0.5f * (srow[j] + srow[j == 0 ? 0 : at + flip * j])); },
         [&](int j, float2 f) { buf[pl.pad(j)] = f; });  // the last pass has read buf before it writes
     __syncthreads();
     unstage_cols(pl, cols_smem, A + (int64_t)blockIdx.y * plane, lda, j0, wh);
@@ -92,13 +95,13 @@ int launch_cols_power(const FftDesc &d, const float2 *A, int lda, int wh, float2
     });
 }
 
-int launch_cols_inverse(const FftDesc &d, const float2 *B, const float *S, int w, int wh, float2 *A, int lda,
+int launch_cols_inverse(const FftDesc &d, const float2 *B, const float *S, int wh, float2 *A, int lda,
                         int64_t plane, int nb, hipStream_t st) {
     return with_cols_plan(d, [&](auto pl) -> int {
         typedef decltype(pl) Plan;
         const int per = cols_per<Plan>(wh);
         hipLaunchKernelGGL(cols_inverse_kernel<Plan>, dim3(8 * per, nb), dim3(Plan::kThreads), cols_lds(pl), st, pl, B,
-                           S, w, wh, A, lda, plane, per);
+                           S, wh, A, lda, plane, per);
         PRNU_CHECK_LAUNCH();
         return PRNU_OK;
     });

@@ -698,96 +698,55 @@ __global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float
     }
 }
 
-// var = n/(n-1) * sum(x^2) over the row partials, FP64, fixed order.  grid (B)
-__global__ __launch_bounds__(256) void wiener_var_kernel(const double *rowsq_all, int h, int64_t n, double *var_all) {
-    __shared__ double sh[4];
-    const double *rowsq = rowsq_all + (int64_t)blockIdx.x * h;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < h; i += 256) s += rowsq[i];
-    s = block_sum_256(s, sh);
-    if (threadIdx.x == 0) var_all[blockIdx.x] = s * (double)n / (double)(n - 1);
-}
-
-// Variance estimate: min over f in {3,5,7,9} of the zero-padded f x f mean of
-// P (wienerfilter.cu:164-247), then S = var / max(var, varest).
-// A workgroup takes a 64-column x 128-row output tile with its 4-pixel halo
-// in LDS (136 x 72 floats); wave k owns output rows [32 k, 32 k + 32) and a
-// lane one column.  The lane walks its 40 LDS rows once (fully unrolled):
-// per row it forms the horizontal 3/5/7/9 sums around its column (9 LDS
-// reads), and every output row sums the horizontal sums of the rows its box
-// covers, so a row's horizontal sums are formed once for 32 outputs instead
-// of once per 8.  All sums add nonnegative terms directly (no running
+// Variance estimate and scale: S(k) = var / max(var, varest(k)), varest the
+// min over f in {3,5,7,9} of the zero-padded f x f mean of P (wienerfilter.cu:
+// 164-247), var = n/(n-1) * sum(x^2) over the row partials (FP64, fixed order,
+// summed again by every workgroup: h values from L2 against a launch); what
+// the inverse transform needs is S'(k) = (S(k) + S(-k)) / 2.
+// P is symmetric, P(-k) = P(k), and only rows [0, rows/2] (length cols) are
+// held and written: full row r > rows/2 is row rows - r reversed.
+// A workgroup takes a 64-column x 4 V-row output tile with its 4-pixel halo
+// in LDS; wave k owns output rows [V k, V k + V) and a lane one column.  The
+// lane walks its V + 8 LDS rows once (fully unrolled): per row it forms the
+// horizontal 3/5/7/9 sums around its column (9 LDS reads), and every output
+// row sums the horizontal sums of the rows its box covers.  V = 32 forms a
+// row's horizontal sums once for 32 outputs; V = 8 is for planes that have few
+// tiles of 32 (one 512x512 image: 24 workgroups, 18 us).  All sums add nonnegative terms directly (no running
 // differences, which would carry the rounding error of a large bin past its
-// window).  Tiles are numbered image by image, row by row, and dealt to the
-// XCDs in ranges as in fastnoise_kernel.  grid (8 * per)
-// P holds half of the power spectrum, which is symmetric, P(-k) = P(k): rows
-// [0, rows/2] of length cols (full row r > rows/2 is row rows - r reversed:
-// P(r, c) = P(rows - r, (cols - c) % cols)).  S is written on the full rows x
-// cols grid.
-constexpr int kVX = 64, kVY = 128, kVB = 4, kVRows = 32;
-__device__ __forceinline__ float power_full(const float *P, int r, int c, int rows, int cols) {
-    if (r <= rows / 2) return P[(int64_t)r * cols + c];
-    return P[(int64_t)(rows - r) * cols + (c == 0 ? 0 : cols - c)];
-}
+// window).
+// S(-k) differs from S(k) only where a box is cut by the grid's edge: at (r, c)
+// the box of S(k) covers the cells of [0, rows) x [0, cols), that of S(-k) --
+// seen from (r, c) -- the cells of [1, rows] x [1, cols], row `rows` being row
+// 0 and column `cols` column 0 (for c = 0: columns [-4, 0]).  Tiles away from
+// the edges (four in five of 2048x1536) write S(k); the others patch the tile's
+// edge cells to that domain, walk it again and write the mean.  Row 0 stays
+// S(0, c): its reader adds S(0, -c).
+// Tiles are numbered image by image, row by row, and dealt to the XCDs in
+// ranges as in fastnoise_kernel.  grid (8 * per)
+constexpr int kVX = 64, kVB = 4;
 
-__global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, float *S_all, int rows, int cols,
-                                                           const double *var_all, int ntx, int nty, int ntiles) {
-    constexpr int LW = kVX + 2 * kVB, LH = kVY + 2 * kVB;
-    __shared__ __align__(16) float T[LH][LW];
-    const int per = (ntiles + 7) / 8;
-    const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if (t >= ntiles) return;
-    const int b = t / (ntx * nty), rem = t - b * (ntx * nty);
-    const int r0 = (rem / ntx) * kVY, c0 = (rem - (rem / ntx) * ntx) * kVX;
-    const int64_t plane = (int64_t)rows * cols;
-    const float *P = P_all + (int64_t)b * plane;
-    float *S = S_all + (int64_t)b * plane;
-    // thread -> (LDS row, group of 4 columns): 18 groups per row.  A group
-    // inside the grid is 4
-    // consecutive values of one source row -- forward (one 16-byte load when
-    // cols is a multiple of 4: gx0 is) or backward in the mirrored half --
-    // so only groups at the grid's edges take the per-value path.
-    const bool vec4 = (cols & 3) == 0;
-    for (int q = threadIdx.x; q < LH * (LW / 4); q += 256) {
-        const int ly = q / (LW / 4), lx = (q - ly * (LW / 4)) * 4;
-        const int gy = r0 + ly - kVB;
-        const int gx0 = c0 + lx - kVB;
-        const bool row_in = gy >= 0 && gy < rows;
-        float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (vec4 && row_in && gx0 >= 0 && gx0 + 3 < cols) {
-            if (gy <= rows / 2) {
-                val = *reinterpret_cast<const float4 *>(P + (int64_t)gy * cols + gx0);
-            } else {
-                const float *pr = P + (int64_t)(rows - gy) * cols;
-                val.x = pr[gx0 == 0 ? 0 : cols - gx0];
-                val.y = pr[cols - gx0 - 1];
-                val.z = pr[cols - gx0 - 2];
-                val.w = pr[cols - gx0 - 3];
-            }
-        } else if (row_in) {
-            float e[4];
+// min-box variances of the lane's column c of LDS rows [oy0, oy0 + V + 8):
+// put(j, varest) for its V output rows.  mask (MASK): the weight, 0 or 1, of
+// the cell `o` columns away at mask[o + 4].
+template <int V, bool MASK, class Put>
+__device__ __forceinline__ void varest_walk(const float (*T)[kVX + 2 * kVB], int oy0, int c, const float *mask,
+                                            Put put) {
+    // output row j sits at LDS row oy0 + j + 4
+    float h3[V + 8], h5[V + 8], h7[V + 8], h9[V + 8];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int gx = gx0 + k;
-                e[k] = (gx >= 0 && gx < cols) ? power_full(P, gy, gx, rows, cols) : 0.f;
-            }
-            val = make_float4(e[0], e[1], e[2], e[3]);
-        }
-        *reinterpret_cast<float4 *>(&T[ly][lx]) = val;
-    }
-    __syncthreads();
-    const int c = threadIdx.x & 63, oy0 = (threadIdx.x >> 6) * kVRows;
-    const float v = (float)var_all[b];
-    const int gx = c0 + c;
-    // LDS rows oy0 .. oy0 + 39; output row j sits at LDS row oy0 + j + 4
-    float h3[kVRows + 8], h5[kVRows + 8], h7[kVRows + 8], h9[kVRows + 8];
-#pragma unroll
-    for (int i = 0; i < kVRows + 8; ++i) {
+    for (int i = 0; i < V + 8; ++i) {
         const float *row = &T[oy0 + i][c + kVB];
-        h3[i] = row[-1] + row[0] + row[1];
-        h5[i] = h3[i] + row[-2] + row[2];
-        h7[i] = h5[i] + row[-3] + row[3];
-        h9[i] = h7[i] + row[-4] + row[4];
+        if constexpr (MASK) {
+            h3[i] = mask[3] * row[-1] + mask[4] * row[0] + mask[5] * row[1];
+            h5[i] = h3[i] + mask[2] * row[-2] + mask[6] * row[2];
+            h7[i] = h5[i] + mask[1] * row[-3] + mask[7] * row[3];
+            h9[i] = h7[i] + mask[0] * row[-4] + mask[8] * row[4];
+        } else {
+            h3[i] = row[-1] + row[0] + row[1];
+            h5[i] = h3[i] + row[-2] + row[2];
+            h7[i] = h5[i] + row[-3] + row[3];
+            h9[i] = h7[i] + row[-4] + row[4];
+        }
         const int j = i - 8;  // the last row output j needs
         if (j >= 0) {
             // each sum starts from its first term: the same value as 0 + first
@@ -801,27 +760,137 @@ __global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, f
             for (int d = -2; d <= 3; ++d) s7 += h7[j + 4 + d];
 #pragma unroll
             for (int d = -3; d <= 4; ++d) s9 += h9[j + 4 + d];
-            // means by the rounded reciprocals of f^2, the quotient by the
-            // hardware reciprocal (each within an ulp or so)
+            // means by the rounded reciprocals of f^2 (each within an ulp or so)
             float best = s3 * (1.f / 9.f);
             best = fminf(best, s5 * (1.f / 25.f));
             best = fminf(best, s7 * (1.f / 49.f));
             best = fminf(best, s9 * (1.f / 81.f));
-            const int gy = r0 + oy0 + j;
-            if (gy < rows && gx < cols) S[(int64_t)gy * cols + gx] = v * __builtin_amdgcn_rcpf(fmaxf(v, best));
+            put(j, best);
         }
     }
 }
 
-int launch_varest(const float *P, float *S, int rows, int cols, int nb, const double *var, hipStream_t st) {
-    const int ntx = (cols + kVX - 1) / kVX, nty = (rows + kVY - 1) / kVY;
+template <int V>
+__global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, float *S_all, int rows, int cols,
+                                                           const double *rowsq_all, int64_t n, int ntx, int nty,
+                                                           int ntiles) {
+    constexpr int kVY = 4 * V, LW = kVX + 2 * kVB, LH = kVY + 2 * kVB;
+    __shared__ __align__(16) float T[LH][LW];
+    __shared__ double sh[4];
+    const int per = (ntiles + 7) / 8;
+    const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (t >= ntiles) return;
+    const int b = t / (ntx * nty), rem = t - b * (ntx * nty);
+    const int r0 = (rem / ntx) * kVY, c0 = (rem - (rem / ntx) * ntx) * kVX;
+    const float *P = P_all + (int64_t)b * n;
+    float *S = S_all + (int64_t)b * n;
+    // thread -> (LDS row, group of 4 columns): 18 groups per row.  A group
+    // inside the grid is 4
+    // consecutive values of one source row -- forward (one 16-byte load when
+    // cols is a multiple of 4: gx0 is) or backward in the mirrored half --
+    // so only groups at the grid's edges take the per-value path.
+    const bool vec4 = (cols & 3) == 0;
+    const int last = min(rows / 2, r0 + kVY - 1);   // output rows [r0, last]
+    const int need = last - r0 + 1 + 2 * kVB;       // LDS rows they read
+    for (int q = threadIdx.x; q < need * (LW / 4); q += 256) {
+        const int ly = q / (LW / 4), lx = (q - ly * (LW / 4)) * 4;
+        const int gy = r0 + ly - kVB;
+        const int gx0 = c0 + lx - kVB;
+        const bool row_in = gy >= 0 && gy < rows;
+        const float *pr = P + (int64_t)(gy <= rows / 2 ? gy : rows - gy) * cols;
+        const bool fwd = gy <= rows / 2;
+        float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (vec4 && row_in && gx0 >= 0 && gx0 + 3 < cols) {
+            if (fwd) {
+                val = *reinterpret_cast<const float4 *>(pr + gx0);
+            } else {
+                val.x = pr[gx0 == 0 ? 0 : cols - gx0];
+                val.y = pr[cols - gx0 - 1];
+                val.z = pr[cols - gx0 - 2];
+                val.w = pr[cols - gx0 - 3];
+            }
+        } else if (row_in) {
+            float e[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int gx = gx0 + k;
+                e[k] = (gx >= 0 && gx < cols) ? pr[fwd || gx == 0 ? gx : cols - gx] : 0.f;
+            }
+            val = make_float4(e[0], e[1], e[2], e[3]);
+        }
+        *reinterpret_cast<float4 *>(&T[ly][lx]) = val;
+    }
+    double sq = 0.0;
+    for (int i = threadIdx.x; i < cols; i += 256) sq += rowsq_all[(int64_t)b * cols + i];
+    sq = block_sum_256(sq, sh);  // (its barriers order the tile, too)
+    const float v = (float)(sq * (double)n / (double)(n - 1));
+    const int c = threadIdx.x & 63, oy0 = (threadIdx.x >> 6) * V;
+    const int gx = c0 + c;
+    const bool idle = r0 + oy0 > last;  // a wave past the last row
+    auto scale = [&](float est) { return v * __builtin_amdgcn_rcpf(fmaxf(v, est)); };  // within an ulp or so
+    const bool edge = r0 == 0 || c0 == 0 || c0 + kVX + kVB > cols || last + kVB >= rows;
+    if (!edge) {
+        if (idle) return;
+        varest_walk<V, false>(T, oy0, c, nullptr, [&](int j, float est) {
+            const int gy = r0 + oy0 + j;
+            if (gy <= last) S[(int64_t)gy * cols + gx] = scale(est);
+        });
+        return;
+    }
+    float s[V];
+    if (!idle) varest_walk<V, false>(T, oy0, c, nullptr, [&](int j, float est) { s[j] = scale(est); });
+    __syncthreads();
+    // the tile of S(-k): cell (y, x) of [1, rows] x [1, cols], and for column 0
+    // of [1, rows] x (-cols, 0]
+    auto cell = [&](int y, int x) {
+        if (y < 1 || y > rows || x > cols || cols + x < 0) return 0.f;
+        if (x < 0) x += cols;
+        if (x == cols) x = 0;
+        if (y == rows) y = 0;
+        return y <= rows / 2 ? P[(int64_t)y * cols + x] : P[(int64_t)(rows - y) * cols + (x == 0 ? 0 : cols - x)];
+    };
+    if (last + kVB >= rows || cols <= kVB) {  // a few rows or columns: every cell
+        for (int q = threadIdx.x; q < need * LW; q += 256)
+            T[q / LW][q % LW] = cell(r0 + q / LW - kVB, c0 + q % LW - kVB);
+    } else {  // differs in rows <= 0, in columns < 0 and in column `cols`
+        if (r0 == 0)
+            for (int q = threadIdx.x; q < (kVB + 1) * LW; q += 256) T[q / LW][q % LW] = 0.f;
+        __syncthreads();
+        const int lx = cols - c0 + kVB;
+        for (int q = threadIdx.x; q < need * (kVB + 1); q += 256) {
+            const int ly = q / (kVB + 1), k = q % (kVB + 1);
+            if (k < kVB && c0 == 0) T[ly][k] = cell(r0 + ly - kVB, k - kVB);
+            if (k == kVB && lx < LW) T[ly][lx] = cell(r0 + ly - kVB, cols);
+        }
+    }
+    __syncthreads();
+    if (idle) return;
+    float mask[9];
+#pragma unroll
+    for (int o = -4; o <= 4; ++o) mask[o + 4] = (gx == 0 ? (o <= 0 && gx + o > -cols) : gx + o >= 1) ? 1.f : 0.f;
+    varest_walk<V, true>(T, oy0, c, mask, [&](int j, float est) {
+        const int gy = r0 + oy0 + j;
+        if (gy <= last && gx < cols) S[(int64_t)gy * cols + gx] = gy == 0 ? s[j] : 0.5f * (s[j] + scale(est));
+    });
+}
+
+template <int V>
+int launch_varest_rows(const float *P, float *S, int rows, int cols, int nb, const double *rowsq, hipStream_t st) {
+    const int ntx = (cols + kVX - 1) / kVX, nty = (rows / 2 + 4 * V) / (4 * V);
     const int64_t ntiles = (int64_t)ntx * nty * nb;
     PRNU_REQUIRE(ntiles < (int64_t(1) << 30), "wiener: %lld variance tiles", (long long)ntiles);
     const int per = (int)((ntiles + 7) / 8);
-    hipLaunchKernelGGL(varest_scale_kernel, dim3((unsigned)(8 * per)), dim3(256), 0, st, P, S, rows, cols, var, ntx,
-                       nty, (int)ntiles);
+    hipLaunchKernelGGL(varest_scale_kernel<V>, dim3((unsigned)(8 * per)), dim3(256), 0, st, P, S, rows, cols, rowsq,
+                       (int64_t)rows * cols, ntx, nty, (int)ntiles);
     PRNU_CHECK_LAUNCH();
     return PRNU_OK;
+}
+
+// Two workgroups per CU at V = 32 fill the chip; below that shorter tiles do.
+int launch_varest(const float *P, float *S, int rows, int cols, int nb, const double *rowsq, hipStream_t st) {
+    const int64_t tiles = (int64_t)((cols + kVX - 1) / kVX) * ((rows / 2 + 128) / 128) * nb;
+    return tiles >= 512 ? launch_varest_rows<32>(P, S, rows, cols, nb, rowsq, st)
+                        : launch_varest_rows<8>(P, S, rows, cols, nb, rowsq, st);
 }
 
 // Rows 2r and 2r+1 from their half spectra in A (h x (w/2+1)): one inverse
@@ -890,7 +959,7 @@ struct ExtractWs {
     int64_t n;              // plane stride (elements) of A, P, S
     float2 *A, *B;          // complex planes of the Wiener filter (B transposed)
     float *P, *S;           // power spectrum / scale (S also holds the FastNoise output)
-    double *rowsq, *var, *colpart, *rowpart, *colmean, *rowmean, *g;
+    double *rowsq, *colpart, *rowpart, *colmean, *rowmean, *g;
     float *cz, *rz;         // FP32 zero-mean column terms (2w) and row means (2h) per image
     int64_t cp_stride, rp_stride;
     int tiles_x, tiles_y;
@@ -905,8 +974,8 @@ int zm_tiles_y_max(int h, int w) { return std::max((h + kZmTileRows - 1) / kZmTi
 size_t per_image_bytes(int h, int w) {
     const int64_t n = (int64_t)h * w;
     const int tx = zm_tiles_x_max(w), ty = zm_tiles_y_max(h, w);
-    return 24 * (size_t)n + 8 * (size_t)(h + 1 + 2 * w * ty + 2 * h * tx + 2 * w + 2 * h + 4) +
-           4 * (size_t)(2 * w + 2 * h) + 13 * 256;
+    return 24 * (size_t)n + 8 * (size_t)(h + 2 * w * ty + 2 * h * tx + 2 * w + 2 * h + 4) +
+           4 * (size_t)(2 * w + 2 * h) + 12 * 256;
 }
 
 int get_ws(Context *c, int nb, ExtractWs &e) {
@@ -922,8 +991,7 @@ int get_ws(Context *c, int nb, ExtractWs &e) {
     const size_t sz[] = {align256(sizeof(float2) * n * nb),
                          align256(sizeof(float2) * n * nb),
                          align256(sizeof(float) * n * nb),    align256(sizeof(float) * n * nb),
-                         align256(sizeof(double) * h * nb),   align256(sizeof(double) * nb),
-                         align256(sizeof(double) * e.cp_stride * nb), align256(sizeof(double) * e.rp_stride * nb),
+                         align256(sizeof(double) * h * nb),   align256(sizeof(double) * e.cp_stride * nb), align256(sizeof(double) * e.rp_stride * nb),
                          align256(sizeof(double) * 2 * w * nb), align256(sizeof(double) * 2 * h * nb),
                          align256(sizeof(double) * 4 * nb),   align256(sizeof(float) * 2 * w * nb),
                          align256(sizeof(float) * 2 * h * nb)};
@@ -932,10 +1000,10 @@ int get_ws(Context *c, int nb, ExtractWs &e) {
     PRNU_TRY(c->ws_filter.ensure(total));
     char *p = static_cast<char *>(c->ws_filter.ptr);
     void **slots[] = {(void **)&e.A,       (void **)&e.B,       (void **)&e.P,       (void **)&e.S,
-                      (void **)&e.rowsq,   (void **)&e.var,     (void **)&e.colpart, (void **)&e.rowpart,
+                      (void **)&e.rowsq,   (void **)&e.colpart, (void **)&e.rowpart,
                       (void **)&e.colmean, (void **)&e.rowmean, (void **)&e.g,       (void **)&e.cz,
                       (void **)&e.rz};
-    for (int k = 0; k < 13; ++k) {
+    for (int k = 0; k < 12; ++k) {
         *slots[k] = p;
         p += sz[k];
     }
@@ -1038,8 +1106,8 @@ int launch_rows_c2r(const FftDesc &dw, const float2 *A, int64_t plane, int h, in
 
 // Wiener filter of nb images (img, img_stride floats apart) into out, on
 // half spectra: row FFTs two rows at a time, column FFTs (+ |F|^2) over the
-// w/2+1 columns, the variance stencil on the full grid (mirrored reads of
-// the half power spectrum), the symmetrized scale + inverse column FFTs,
+// w/2+1 columns, the variance stencil (the symmetrized scale of half the
+// grid), scale + inverse column FFTs,
 // real inverse row FFTs two rows at a time.
 int launch_wiener(Context *c, ExtractWs &e, int nb, const float *img, int64_t img_stride, float *out,
                   int64_t out_stride, bool zm, hipStream_t st) {
@@ -1065,12 +1133,10 @@ int launch_wiener(Context *c, ExtractWs &e, int nb, const float *img, int64_t im
         PRNU_CHECK_LAUNCH();
         return PRNU_OK;
     }));
-    hipLaunchKernelGGL(wiener_var_kernel, dim3(nb), dim3(256), 0, st, e.rowsq, h, n, e.var);
-    PRNU_CHECK_LAUNCH();
     // B = A^T (wh x h); the zero-padded box-min stencil is transpose invariant
     PRNU_TRY(launch_cols_power(dh, e.A, lda, wh, e.B, e.P, n, nb, st));
-    PRNU_TRY(launch_varest(e.P, e.S, w, h, nb, e.var, st));
-    PRNU_TRY(launch_cols_inverse(dh, e.B, e.S, w, wh, e.A, lda, n, nb, st));
+    PRNU_TRY(launch_varest(e.P, e.S, w, h, nb, e.rowsq, st));
+    PRNU_TRY(launch_cols_inverse(dh, e.B, e.S, wh, e.A, lda, n, nb, st));
     return launch_rows_c2r(dw, e.A, n, h, nb, out, out_stride, 1.0f / (float)((double)w * h), lda, st);
 }
 
