@@ -770,6 +770,8 @@ __device__ __forceinline__ void varest_walk(const float (*T)[kVX + 2 * kVB], int
     }
 }
 
+// (32 planes of 2048x1536: 211 us over the whole plane, 158 us so; 4 of
+// 4000x3000 106 -> 83 us; one 512x512 14 -> 8.7 us with V = 8, 18 us with 32.)
 template <int V>
 __global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, float *S_all, int rows, int cols,
                                                            const double *rowsq_all, int64_t n, int ntx, int nty,

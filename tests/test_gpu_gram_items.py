@@ -69,3 +69,33 @@ def test_split_item_keeps_the_slabs(slab_blocks):
         pl.close()
     store.close()
     gram.close()
+
+
+@pytest.mark.parametrize("fmt", ["split_bf16", "fp32", "fp16", "fp8"])
+@pytest.mark.parametrize("count,n,first,offset", [(1, 6, 0, 0), (9, 1023, 2, 0), (8, 1024, 0, 0), (17, 1029, 3, 1),
+                                                  (5, 5000, 1, 3)])
+def test_put_edges(fmt, count, n, first, offset):
+    """Inserts around the packing's 8 patterns and 1024 values, with pattern
+    rows off 16-byte alignment: the stored statistics (FP64 sums of FP32
+    products: 1e-10), slots around the range untouched, and the same blocks as
+    one pattern put at a time (bytes equal)."""
+    g = torch.Generator(device="cuda").manual_seed(n + count)
+    rows = [torch.randn(n + offset, generator=g, device="cuda")[offset:] for _ in range(count)]
+    stores = [csi.PatternStore(n, first + count + 2, fmt) for _ in range(2)]
+    stores[0].put(rows, first_slot=first)
+    for i, r in enumerate(rows):
+        stores[1].put([r], first_slot=first + i)
+    images = []
+    for s in stores:
+        img = torch.empty(s.image_bytes(first + count + 2), dtype=torch.uint8)
+        s.save(0, first + count + 2, img)
+        images.append(img.numpy())
+    blocks = len(images[0]) - (first + count + 2) * 24   # the slots past and before `first` hold no statistics yet
+    assert np.array_equal(images[0][:blocks], images[1][:blocks])
+    for s in stores:
+        got = s.stats(count, first)
+        for i, r in enumerate(rows):
+            sx, sxx = O.pattern_sums(r.cpu().numpy())
+            assert got[0][i] == pytest.approx(sx, rel=1e-9, abs=1e-9) and got[1][i] == pytest.approx(sxx, rel=1e-10)
+            assert got[2][i] == r.abs().max().item()
+        s.close()
