@@ -187,3 +187,25 @@ def test_decoder_pool_matches_single_decoder():
         got.append(out.cpu().numpy())
     pool.close()
     assert len(got) == 4 and all(np.array_equal(g, w) for g, w in zip(got, want))
+
+
+@pytest.mark.parametrize("sub", [0, 2])
+@pytest.mark.parametrize("kw", [{}, {"restart_marker_rows": 1}])
+def test_chunk_and_wave_edges(sub, kw):
+    """Scans of 1 to some 140 chunks of 128 bytes, so their ends fall on both
+    sides of a chunk's and of a wave's (64 chunks) border: bit for bit."""
+    rng = np.random.default_rng(5 + sub)
+    sizes, files, lengths = [], [], set()
+    for k in range(40):
+        h, w = 8 + 4 * k, 16 + 5 * k
+        img = np.clip(128 + rng.normal(0, 3 + k, (h, w, 3)), 0, 255).astype(np.uint8)
+        files.append(encode(img, quality=75 + k // 2, subsampling=sub, **kw))
+        sizes.append((h, w))
+        lengths.add(len(files[-1]) // 8192)
+    assert len(lengths) >= 2
+    dec = jpeg.JpegDecoder()
+    got, st = decode_mixed(dec, files, sizes)
+    assert st == [0] * len(files)
+    for f, g, s in zip(files, got, sizes):
+        assert np.array_equal(g, pil_rgb(f)), s
+    dec.close()
