@@ -24,32 +24,36 @@ static bool fft_factor(int n, int *radix, int *passes) {
     static const int kRadices[] = {16, 8, 4, 2, 20, 12, 10, 6, 15, 9, 5, 3};
     std::vector<int> best, cur;
     int best_sum = 0;
-    auto search = [&](auto &self, int left, int from, int sum) -> void {
-        if (left == 1) {
-            if (best.empty() || cur.size() < best.size() || (cur.size() == best.size() && sum < best_sum)) {
+    auto search = [&](auto &self, int left, int from, int sum, int depth) -> void {
+        if (depth == 0) {
+            if (left == 1 && (best.empty() || sum < best_sum)) {
                 best = cur;
                 best_sum = sum;
             }
             return;
         }
-        if (!best.empty() && cur.size() >= best.size()) return;
+        int most = 1;  // what depth passes can reach
+        for (int k = 0; k < depth; ++k) most *= 20;
+        if (left > most) return;
         for (int i = from; i < (int)(sizeof(kRadices) / sizeof(int)); ++i) {
             if (left % kRadices[i]) continue;
             cur.push_back(kRadices[i]);
-            self(self, left / kRadices[i], i, sum + kRadices[i]);
+            self(self, left / kRadices[i], i, sum + kRadices[i], depth - 1);
             cur.pop_back();
         }
     };
-    search(search, n, 0, 0);
-    if (best.empty() || best.size() > (size_t)kFftMaxPasses) return false;
+    for (int depth = 1; depth <= std::min(kFftMaxPasses, 6) && best.empty(); ++depth) search(search, n, 0, 0, depth);
+    if (best.empty()) return false;
     *passes = (int)best.size();
     std::copy(best.begin(), best.end(), radix);
     return true;
 }
 
 // Radices 8, 4, 2, then 3 and 5 alone (a power-of-two part 8^k * 2 becomes
-// 8^(k-1) * 4 * 4): the plan of PCE's row pass, whose rounding the scores keep
-// (the peak is one value of the plane, its error is not averaged).
+// 8^(k-1) * 4 * 4): PCE's plan.  A score's error is the bias of the plane's
+// energy, which its roundings do not average out: 4 spectra of 500x960 were
+// 1.2e-7 off so, 2.0e-7 with the composite radices, 3 of 3375x96 2.1e-8 and
+// 5.3e-8.
 static void fft_factor_basic(int n, int *radix, int *passes) {
     int p = 0, e2 = 0;
     for (; n % 2 == 0; n /= 2) ++e2;

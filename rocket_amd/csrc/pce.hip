@@ -8,8 +8,9 @@
 //   1. pce_rows_*        build rows u and h - u of Z and run their inverse row
 //                        FFTs (length w) in LDS;
 //   2. pce_cols_kernel   strips of adjacent columns of the row-pass output
-//                        through LDS (cols_device.hpp): inverse FFT (length h)
-//                        of each column, whose last pass hands every output to
+//                        through LDS (cols_device.hpp) at 1024 and 1536 rows,
+//                        pce_cols_row_kernel after a transpose otherwise:
+//                        inverse FFT (length h) of each column, whose last pass hands every output to
 //                        the per-column sums: the max |Re c| with its index
 //                        and sum (Re c)^2 in FP64 for each pair of the couple
 //                        (the correlation planes themselves are never
@@ -161,13 +162,110 @@ __device__ __forceinline__ void herm_pair(const float2 *X, const float2 *Y, int 
     hm = make_float2(0.5f * (c2.x + m2.x), 0.5f * (c2.y - m2.y));
 }
 
+// ------------------------------------- transforms of a run-time length
+// The rows and columns of the lengths without a plan of their own: a 256-thread
+// workgroup each, radices 8, 4, 2, 3, 5 (fft_desc_basic), one template
+// instance per pass.  A score divides the square of one value by an energy
+// whose bias the roundings do not average out, so the plans of the extraction
+// chain (composite radices, one loop over all passes) are not taken here: 4
+// spectra of 500x960 came 2.0e-7 off with them, 1.2e-7 so; 3 of 3375x96 5.3e-8
+// and 2.1e-8.  MAXN: the per-thread butterfly arrays are sized for rows up to
+// kFftSmallN, kFftMidN, kFftMaxN.
+constexpr int kFftSmallN = 2048, kFftMidN = 4096;
+
+__device__ __forceinline__ int pass_mod(int j, int Ns) { return (Ns & (Ns - 1)) == 0 ? (j & (Ns - 1)) : j % Ns; }
+
+template <int R, int DIR, bool FIRST, bool LAST, int MAXN, class Get, class Put>
+__device__ __forceinline__ void fft_pass_io(float2 *buf, int n, int Ns, const float2 *tw, Get &get, Put &put) {
+    constexpr int kMaxB = (MAXN / R + kFftThreads - 1) / kFftThreads;
+    const int nb = n / R;
+    const int twstep = n / (Ns * R);
+    const int tid = threadIdx.x;
+    float2 v[kMaxB][R];
+#pragma unroll
+    for (int b = 0; b < kMaxB; ++b) {
+        const int j = tid + b * kFftThreads;
+        if (j < nb) {
+            if constexpr (FIRST) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) v[b][r] = get(j + r * nb);
+            } else {
+                const int k = pass_mod(j, Ns);
+                v[b][0] = buf[j];
+#pragma unroll
+                for (int r = 1; r < R; ++r) v[b][r] = cmul(buf[j + r * nb], twiddle<DIR>(tw, r * k * twstep));
+            }
+        }
+    }
+    if constexpr (!FIRST) __syncthreads();  // every read of buf precedes the writes below
+#pragma unroll
+    for (int b = 0; b < kMaxB; ++b) {
+        const int j = tid + b * kFftThreads;
+        if (j < nb) {
+            dft<R, DIR>(v[b]);
+            const int k = FIRST ? 0 : pass_mod(j, Ns);
+            const int base = (j - k) * R + k;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                if constexpr (LAST)
+                    put(base + q * Ns, v[b][q]);
+                else
+                    buf[base + q * Ns] = v[b][q];
+            }
+        }
+    }
+    __syncthreads();
+}
+
+template <int DIR, bool FIRST, bool LAST, int MAXN, class Get, class Put>
+__device__ __forceinline__ void fft_pass_io_r(int R, float2 *buf, int n, int Ns, const float2 *tw, Get &get,
+                                              Put &put) {
+    if (R == 8)
+        fft_pass_io<8, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
+    else if (R == 4)
+        fft_pass_io<4, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
+    else if (R == 2)
+        fft_pass_io<2, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
+    else if (R == 3)
+        fft_pass_io<3, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
+    else
+        fft_pass_io<5, DIR, FIRST, LAST, MAXN>(buf, n, Ns, tw, get, put);
+}
+
+// Length-d.n DFT of values given by get(i) (each read once) to put(i, X[i])
+// (each written once), through LDS buf (d.n values) for the passes between;
+// ends with a barrier, so the caller may reuse buf.
+template <int DIR, int MAXN, class Get, class Put>
+__device__ inline void fft_row(float2 *buf, const FftDesc &d, Get get, Put put) {
+    // the hot lengths with compile-time strides
+    if constexpr (MAXN >= 2048) {
+        if (d.n == 2048) return fft_row_c<DIR, 2048>(buf, d.tw, get, put);
+        if (d.n == 1536) return fft_row_c<DIR, 1536>(buf, d.tw, get, put);
+    }
+    if constexpr (MAXN >= 1024) {
+        if (d.n == 1024) return fft_row_c<DIR, 1024>(buf, d.tw, get, put);
+    }
+    const int P = d.passes;
+    if (P == 1) {
+        fft_pass_io_r<DIR, true, true, MAXN>(d.radix[0], buf, d.n, 1, d.tw, get, put);
+        return;
+    }
+    fft_pass_io_r<DIR, true, false, MAXN>(d.radix[0], buf, d.n, 1, d.tw, get, put);
+    int Ns = d.radix[0];
+    for (int p = 1; p < P - 1; ++p) {
+        fft_pass_io_r<DIR, false, false, MAXN>(d.radix[p], buf, d.n, Ns, d.tw, get, put);
+        Ns *= d.radix[p];
+    }
+    fft_pass_io_r<DIR, false, true, MAXN>(d.radix[P - 1], buf, d.n, Ns, d.tw, get, put);
+}
+
 // Row i of Z = H_a + i H_b for couple blockIdx.y (pairs 2q, 2q+1 of the
 // batch; the second may be absent), inverse row FFT: the first pass reads
 // the Hermitian parts straight from the half spectra, the last pass writes
 // the row of A.  grid (16 ceil((h/2 + 1) / 8), couples), LDS w complex.
-template <int VARIANT, class R>
-__global__ __launch_bounds__(R::T) void pce_rows2_kernel(R pl, int h, int nb, PceBatch bt, float2 *__restrict__ Aall,
-                                                         int64_t pstride) {
+template <int VARIANT, int MAXN>
+__global__ __launch_bounds__(kFftThreads) void pce_rows2_kernel(FftDesc d, int h, int nb, PceBatch bt,
+                                                                float2 *__restrict__ Aall, int64_t pstride) {
     extern __shared__ float2 buf[];
     // Row i reads spectrum rows i and (h - i) mod h (the mirrored half of the
     // cross spectrum), and so does row (h - i) mod h: workgroups x and x + 8
@@ -182,14 +280,14 @@ __global__ __launch_bounds__(R::T) void pce_rows2_kernel(R pl, int h, int nb, Pc
     const int i = side ? (h - u) % h : u;
     if (side && i == u) return;
     const int q = blockIdx.y;
-    const int w = pl.n();
+    const int w = d.n;
     const float2 *Xa, *Ya, *Xb = nullptr, *Yb = nullptr;
     pce_operands(bt, 2 * q, Xa, Ya);
     const bool two = 2 * q + 1 < nb;
     if (two) pce_operands(bt, 2 * q + 1, Xb, Yb);
     float2 *A = Aall + (int64_t)q * pstride + (int64_t)i * w;
-    pl.template run<1>(
-        buf,
+    fft_row<1, MAXN>(
+        buf, d,
         [&](int j) {
             const float2 ha = herm_at<VARIANT>(Xa, Ya, h, w, i, j);
             if (!two) return ha;
@@ -206,13 +304,13 @@ __global__ __launch_bounds__(R::T) void pce_rows2_kernel(R pl, int h, int nb, Pc
 // in both variants), so its transform input is
 // Z(-u, j) = conj(H_a(u, -j)) + i conj(H_b(u, -j)).  That halves the
 // spectrum reads of pce_rows2_kernel, whose two workgroups per pair each
-// form their own row's Hermitian parts.  grid (h/2 + 1, couples), LDS 2w
-// complex and the transform buffer (H_a, H_b of row u).
-template <int VARIANT, class R>
-__global__ __launch_bounds__(R::T) void pce_rows_mirror_kernel(R pl, int h, int nb, PceBatch bt,
-                                                               float2 *__restrict__ Aall, int64_t pstride) {
+// form their own row's Hermitian parts.  grid (h/2 + 1, couples), LDS 3w
+// complex (H_a, H_b of row u, the transform buffer).
+template <int VARIANT, int MAXN>
+__global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d, int h, int nb, PceBatch bt,
+                                                                      float2 *__restrict__ Aall, int64_t pstride) {
     extern __shared__ float2 smem[];
-    const int w = pl.n();
+    const int w = d.n;
     float2 *ha = smem, *hb = smem + w, *buf = smem + 2 * w;
     const int u = blockIdx.x;
     if (u > h / 2) return;
@@ -222,7 +320,7 @@ __global__ __launch_bounds__(R::T) void pce_rows_mirror_kernel(R pl, int h, int 
     pce_operands(bt, 2 * q, Xa, Ya);
     const bool two = 2 * q + 1 < nb;
     if (two) pce_operands(bt, 2 * q + 1, Xb, Yb);
-    for (int j = threadIdx.x; j <= w / 2; j += R::T) {  // each spectrum value read once
+    for (int j = threadIdx.x; j <= w / 2; j += kFftThreads) {  // each spectrum value read once
         float2 a, am, b = make_float2(0.f, 0.f), bm = make_float2(0.f, 0.f);
         herm_pair<VARIANT>(Xa, Ya, w, u, um, j, a, am);
         if (two) herm_pair<VARIANT>(Xb, Yb, w, u, um, j, b, bm);
@@ -235,22 +333,84 @@ __global__ __launch_bounds__(R::T) void pce_rows_mirror_kernel(R pl, int h, int 
     }
     __syncthreads();
     float2 *A = Aall + (int64_t)q * pstride;
-    pl.template run<1>(
-        buf,
+    fft_row<1, MAXN>(
+        buf, d,
         [&](int j) {
             const float2 a = ha[j], b = hb[j];
             return make_float2(a.x - b.y, a.y + b.x);
         },
         [&](int j, float2 f) { A[(int64_t)u * w + j] = f; });
     if (um == u) return;
-    pl.template run<1>(
-        buf,
+    fft_row<1, MAXN>(
+        buf, d,
         [&](int j) {
             const int mj = j == 0 ? 0 : w - j;
             const float2 a = ha[mj], b = hb[mj];
             return make_float2(a.x + b.y, b.x - a.y);
         },
         [&](int j, float2 f) { A[(int64_t)um * w + j] = f; });
+}
+
+// Column j of couple blockIdx.y from the transposed row-pass output
+// (B[j*h + i] = A[i][j]): inverse FFT of length h; every output value goes
+// straight into this thread's sums of Re (pair 2q) and Im (pair 2q + 1) --
+// FP64 energy and the max |value| with its linear index i*w + j, smallest
+// index on ties -- which a fixed-order block reduction turns into the
+// column's partials.  grid (w, couples), LDS h complex.
+template <int MAXN>
+__global__ __launch_bounds__(kFftThreads) void pce_cols_row_kernel(FftDesc d, int w, int nb, const float2 *__restrict__ Ball,
+                                                               int64_t pstride, PeakPart *__restrict__ partall) {
+    extern __shared__ float2 buf[];
+    __shared__ double sh_e[2][4];
+    __shared__ float sh_v[2][4];
+    __shared__ int sh_i[2][4];
+    const int h = d.n, q = blockIdx.y, j = blockIdx.x;
+    const float2 *col = Ball + (int64_t)q * pstride + (int64_t)j * h;
+    double e0 = 0.0, e1 = 0.0;
+    float b0 = -1.0f, b1 = -1.0f;
+    int i0 = 0x7fffffff, i1 = 0x7fffffff;
+    fft_row<1, MAXN>(
+        buf, d, [&](int i) { return col[i]; },
+        [&](int i, float2 z) {
+            const int idx = i * w + j;
+            e0 += (double)z.x * (double)z.x;
+            e1 += (double)z.y * (double)z.y;
+            argmax_merge(b0, i0, fabsf(z.x), idx);
+            argmax_merge(b1, i1, fabsf(z.y), idx);
+        });
+    const int halves = 2 * q + 1 < nb ? 2 : 1;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    e0 = wave_sum_d(e0);
+    e1 = wave_sum_d(e1);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        float v2 = __shfl_xor(b0, off, 64);
+        int k2 = __shfl_xor(i0, off, 64);
+        argmax_merge(b0, i0, v2, k2);
+        v2 = __shfl_xor(b1, off, 64);
+        k2 = __shfl_xor(i1, off, 64);
+        argmax_merge(b1, i1, v2, k2);
+    }
+    if (lane == 0) {
+        sh_e[0][wave] = e0;
+        sh_e[1][wave] = e1;
+        sh_v[0][wave] = b0;
+        sh_v[1][wave] = b1;
+        sh_i[0][wave] = i0;
+        sh_i[1][wave] = i1;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < halves) {  // fixed-order merge of the 4 waves
+        PeakPart p;
+        p.energy = (sh_e[t][0] + sh_e[t][1]) + (sh_e[t][2] + sh_e[t][3]);
+        float best = sh_v[t][0];
+        int bi = sh_i[t][0];
+        for (int k = 1; k < 4; ++k) argmax_merge(best, bi, sh_v[t][k], sh_i[t][k]);
+        p.absmax = best;
+        p.index = bi;
+        partall[(int64_t)(2 * q + t) * w + j] = p;
+    }
 }
 
 // pce_rows_mirror_kernel for w = W = 1024 with one wave per row and W = 2048
@@ -330,7 +490,9 @@ __global__ __launch_bounds__(2 * mirror_row_threads<W>()) void pce_rows_mirror_w
 // straight into its thread's sums of Re (pair 2q) and Im (pair 2q + 1) -- FP64
 // energy and the max |value| with its linear index i*w + j, smallest index on
 // ties -- which a fixed-order reduction over the column's waves turns into the
-// column's partials.  grid (8 per, couples).
+// column's partials.  grid (8 per, couples).  (66 pairs of 2048x1536: 1310 us
+// with 301 us of transposes and 373 us of pce_cols_row_kernel and the rows one
+// by one, 1006 us with these strips and the rows in mirror pairs.)
 template <class P>
 __global__ __launch_bounds__(P::kThreads) void pce_cols_kernel(P pl, int w, int nb, const float2 *__restrict__ Aall,
                                                                int64_t pstride, PeakPart *__restrict__ partall,
@@ -354,14 +516,7 @@ __global__ __launch_bounds__(P::kThreads) void pce_cols_kernel(P pl, int w, int 
         argmax_merge(b0, i0, fabsf(z.x), idx);
         argmax_merge(b1, i1, fabsf(z.y), idx);
     };
-    if constexpr (P::kConst) {
-        pl.template run<1, true>(buf, [&](int i) { return buf[pl.pad(i)]; }, add);
-    } else {  // the sums inside every radix's last pass would spill: through LDS once more
-        pl.template run<1, true>(
-            buf, [&](int i) { return buf[pl.pad(i)]; }, [&](int i, float2 z) { buf[pl.pad(i)] = z; });
-        for (int i = t; i < pl.n(); i += P::T) add(i, buf[pl.pad(i)]);
-        if constexpr (kWaves > 1) __syncthreads();
-    }
+    pl.template run<1, true>(buf, [&](int i) { return buf[pl.pad(i)]; }, add);
     e0 = wave_sum_d(e0);
     e1 = wave_sum_d(e1);
 #pragma unroll
@@ -577,32 +732,76 @@ __global__ __launch_bounds__(64) void pce_score_kernel(const double *__restrict_
     outall[base + p] = pce;
 }
 
+// out[b][c][r] = in[b][r][c], planes `stride` values apart.
+constexpr int kTT = 32;
+
+__global__ __launch_bounds__(256) void transpose_kernel(const float2 *__restrict__ in, float2 *__restrict__ out,
+                                                        int rows, int cols, int64_t stride) {
+    __shared__ float2 tile[kTT][kTT + 1];
+    const int64_t off = (int64_t)blockIdx.z * stride;
+    const int c0 = blockIdx.x * kTT, r0 = blockIdx.y * kTT;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
+#pragma unroll
+    for (int i = 0; i < kTT; i += 8) {
+        const int r = r0 + ty + i, c = c0 + tx;
+        if (r < rows && c < cols) tile[ty + i][tx] = in[off + (int64_t)r * cols + c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTT; i += 8) {
+        const int c = c0 + ty + i, r = r0 + tx;
+        if (r < rows && c < cols) out[off + (int64_t)c * rows + r] = tile[tx][ty + i];
+    }
+}
+
+template <int V, int MAXN>
+void launch_pce_rows_rt(const FftDesc &dw, dim3 mgrid, dim3 rgrid, int h, int nb, const PceBatch &bt, float2 *A,
+                        int64_t pstride, hipStream_t st) {
+    if (dw.n <= 1024)  // both rows of a mirror pair in one workgroup (24 KiB of LDS)
+        hipLaunchKernelGGL((pce_rows_mirror_kernel<V, MAXN>), mgrid, dim3(kFftThreads),
+                           3 * sizeof(float2) * (size_t)dw.n, st, dw, h, nb, bt, A, pstride);
+    else
+        hipLaunchKernelGGL((pce_rows2_kernel<V, MAXN>), rgrid, dim3(kFftThreads), sizeof(float2) * (size_t)dw.n, st, dw,
+                           h, nb, bt, A, pstride);
+}
+
 template <int V>
 int launch_pce_rows(const FftDesc &dw, dim3 mgrid, dim3 rgrid, int h, int nb, const PceBatch &bt, float2 *A,
                     int64_t pstride, hipStream_t st) {
-    if (dw.n == 1024) {
+    if (dw.n == 1024)
         hipLaunchKernelGGL((pce_rows_mirror_wave_kernel<V, 1024>), mgrid, dim3(128), 0, st, dw.tw, h, nb, bt, A,
                            pstride);
-    } else if (dw.n == 2048) {
+    else if (dw.n == 2048)
         hipLaunchKernelGGL((pce_rows_mirror_wave_kernel<V, 2048>), mgrid, dim3(512), 0, st, dw.tw, h, nb, bt, A,
                            pstride);
-    } else if (dw.n == 1536) {
-        const RowC<1536> pl{dw.tw};
-        hipLaunchKernelGGL((pce_rows_mirror_kernel<V, RowC<1536>>), mgrid, dim3(pl.T),
-                           2 * sizeof(float2) * dw.n + pl.smem(), st, pl, h, nb, bt, A, pstride);
-    } else if (dw.n < 2048) {
-        const RowRt<256> pl{dw};
-        hipLaunchKernelGGL((pce_rows_mirror_kernel<V, RowRt<256>>), mgrid, dim3(pl.T),
-                           2 * sizeof(float2) * dw.n + pl.smem(), st, pl, h, nb, bt, A, pstride);
-    } else if (dw.n <= 4096) {
-        const RowRt<512> pl{dw};
-        hipLaunchKernelGGL((pce_rows2_kernel<V, RowRt<512>>), rgrid, dim3(pl.T), pl.smem(), st, pl, h, nb, bt, A,
-                           pstride);
-    } else {
-        const RowRt<1024> pl{dw};
-        hipLaunchKernelGGL((pce_rows2_kernel<V, RowRt<1024>>), rgrid, dim3(pl.T), pl.smem(), st, pl, h, nb, bt, A,
-                           pstride);
-    }
+    else if (dw.n <= kFftSmallN)
+        launch_pce_rows_rt<V, kFftSmallN>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st);
+    else if (dw.n <= kFftMidN)
+        launch_pce_rows_rt<V, kFftMidN>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st);
+    else
+        launch_pce_rows_rt<V, kFftMaxN>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st);
+    PRNU_CHECK_LAUNCH();
+    return PRNU_OK;
+}
+
+template <class Plan>
+int launch_pce_cols(const Plan &pl, int w, int nb, int couples, const float2 *A, int64_t pstride, PeakPart *part,
+                    hipStream_t st) {
+    const int per = cols_per<Plan>(w);
+    hipLaunchKernelGGL(pce_cols_kernel<Plan>, dim3(8 * per, couples), dim3(Plan::kThreads), cols_lds(pl), st, pl, w, nb,
+                       A, pstride, part, per);
+    PRNU_CHECK_LAUNCH();
+    return PRNU_OK;
+}
+
+template <int MAXN>
+int launch_pce_cols_rt(const FftDesc &dh, int w, int nb, int couples, const float2 *A, float2 *B, int64_t pstride,
+                       PeakPart *part, hipStream_t st) {
+    hipLaunchKernelGGL(transpose_kernel, dim3((w + kTT - 1) / kTT, (dh.n + kTT - 1) / kTT, couples), dim3(256), 0, st,
+                       A, B, dh.n, w, pstride);
+    PRNU_CHECK_LAUNCH();
+    hipLaunchKernelGGL((pce_cols_row_kernel<MAXN>), dim3(w, couples), dim3(kFftThreads), sizeof(float2) * (size_t)dh.n,
+                       st, dh, w, nb, B, pstride, part);
     PRNU_CHECK_LAUNCH();
     return PRNU_OK;
 }
@@ -615,28 +814,31 @@ int pce_batch(Context *c, int variant, const PceBatch &bt, int nb, double *out, 
     const size_t pbytes = ((sizeof(PeakPart) * w) + 255) & ~size_t(255);
     const int64_t pstride = (int64_t)(plane / sizeof(float2));
     const size_t wbytes = ((sizeof(double) * kWinSlots * nb) + 255) & ~size_t(255);
-    PRNU_TRY(c->ws_pce.ensure(plane * couples + pbytes * nb + wbytes));
+    const bool strips = h == 1024 || h == 1536;  // columns read from the rows' own layout
+    const size_t planes = plane * couples * (strips ? 1 : 2);
+    PRNU_TRY(c->ws_pce.ensure(planes + pbytes * nb + wbytes));
     char *base = static_cast<char *>(c->ws_pce.ptr);
-    float2 *A = reinterpret_cast<float2 *>(base);  // row-pass output, h x w per couple
-    PeakPart *part = reinterpret_cast<PeakPart *>(base + plane * couples);
-    double *wbuf = reinterpret_cast<double *>(base + plane * couples + pbytes * nb);
+    float2 *A = reinterpret_cast<float2 *>(base);                                        // row-pass output, h x w per couple
+    float2 *B = strips ? nullptr : reinterpret_cast<float2 *>(base + plane * couples);  // its transpose, w x h
+    PeakPart *part = reinterpret_cast<PeakPart *>(base + planes);
+    double *wbuf = reinterpret_cast<double *>(base + planes + pbytes * nb);
     const FftDesc &dw = fft_desc_basic(c->fft_w);
-    const FftDesc &dh = fft_desc(c->fft_h);
+    const FftDesc &dh = fft_desc_basic(c->fft_h);
     const dim3 rgrid((unsigned)((h / 2 + 1 + 7) / 8 * 16), couples);  // mirror pairs of rows (pce_rows2_kernel)
-    // rows up to 2048: both rows of a mirror pair in one workgroup (at most 50
-    // KiB of LDS, three workgroups per CU)
     const dim3 mgrid((unsigned)(h / 2 + 1), couples);
     PRNU_TRY(variant == PRNU_PCE_REFERENCE
                  ? launch_pce_rows<PRNU_PCE_REFERENCE>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st)
                  : launch_pce_rows<PRNU_PCE_TEXTBOOK>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st));
-    PRNU_TRY(with_cols_plan(dh, [&](auto pl) -> int {
-        typedef decltype(pl) Plan;
-        const int per = cols_per<Plan>(w);
-        hipLaunchKernelGGL(pce_cols_kernel<Plan>, dim3(8 * per, couples), dim3(Plan::kThreads), cols_lds(pl), st, pl, w,
-                           nb, A, pstride, part, per);
-        PRNU_CHECK_LAUNCH();
-        return PRNU_OK;
-    }));
+    if (h == 1024)
+        PRNU_TRY(launch_pce_cols(ColsC<1024>{dh.tw}, w, nb, couples, A, pstride, part, st));
+    else if (h == 1536)
+        PRNU_TRY(launch_pce_cols(ColsC<1536>{dh.tw}, w, nb, couples, A, pstride, part, st));
+    else if (h <= kFftSmallN)
+        PRNU_TRY(launch_pce_cols_rt<kFftSmallN>(dh, w, nb, couples, A, B, pstride, part, st));
+    else if (h <= kFftMidN)
+        PRNU_TRY(launch_pce_cols_rt<kFftMidN>(dh, w, nb, couples, A, B, pstride, part, st));
+    else
+        PRNU_TRY(launch_pce_cols_rt<kFftMaxN>(dh, w, nb, couples, A, B, pstride, part, st));
     // window rows (and, for the reference variant, the last element's value)
     const dim3 wgrid_ref(nb, kSquare + 1), wgrid_txt(nb, kSquare), sgrid((nb + 63) / 64);
     hipLaunchKernelGGL(pce_peak_kernel, dim3(nb), dim3(256), 0, st, part, h, w, wbuf);
