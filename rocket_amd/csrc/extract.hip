@@ -609,8 +609,8 @@ __global__ __launch_bounds__(256) void zm_apply_kernel(float *img_all, int64_t i
 // transform z = a + i b of length w: A_k = (Z_k + conj Z_{w-k}) / 2 and
 // B_k = (Z_k - conj Z_{w-k}) / 2i.
 
-// Rows 2r and 2r+1 of image b: (optional zero-mean) -> sums of squares
-// (FP64) -> forward FFT (w) -> half spectra into A (h x (w/2+1)).
+// Rows 2r and 2r+1 of image b: (optional zero-mean) -> forward FFT (w) -> half
+// spectra into A (h x (w/2+1)); each row's sum of squares (FP64).
 // grid (ceil(h/2), B).
 // Zero-mean, odd widths (cz and rz non-null): x - cz[row parity][j] -
 // rz[j & 1][row] in FP32, the column terms cz = colmean - g and row means rz
@@ -620,11 +620,14 @@ __global__ __launch_bounds__(256) void zm_apply_kernel(float *img_all, int64_t i
 // What the row means and g would still take away is one constant on the
 // row's even columns and one on its odd columns, which lie in bins 0 and w/2
 // alone; the zero-mean row has no even-column sum and no odd-column sum, so
-// both bins are zero: they are written as zeros, and the row's sum of squares
-// loses Se^2 / (w/2) + So^2 / (w/2), Se and So the row's even- and odd-column
-// sums from the same two bins.  No row sums are taken before the transform
-// (32 frames of 2048x1536: 304 -> 275 us, two loads and two subtractions less
-// per value pair).
+// both bins are zero and are written as zeros.  The row's sum of squares is
+// that of the bins left (Parseval, 2/w times the half spectrum's powers): a sum
+// of squares taken before the transform would have to lose those of the row
+// means again, and where a frame's structure is horizontal they are nearly all
+// of it, so that the difference is rounding of either sign (2000x1500, two-row
+// bars and one 8x8 patch: the pattern 6.7e-4 off; 2.5e-7 so).  No row sums are
+// taken before the transform (32 frames of 2048x1536: 299 -> 265 us, two loads
+// and two subtractions less per value pair).
 template <class R, bool ZM_EVEN>
 __global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float *img_all, int64_t img_stride, int h,
                                                                float2 *A_all, int64_t plane, double *rowsq_all,
@@ -656,8 +659,10 @@ __global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float
                 va = (va - cz0[j]) - (odd ? ra1 : ra0);
                 vb = two ? (vb - cz1[j]) - (odd ? rb1 : rb0) : 0.f;
             }
-            sq0 += (double)va * (double)va;
-            sq1 += (double)vb * (double)vb;
+            if (!ZM_EVEN) {
+                sq0 += (double)va * (double)va;
+                sq1 += (double)vb * (double)vb;
+            }
             return make_float2(va, vb);
         };
     auto put = [&](int j, float2 f) { buf[j] = f; };  // the last pass has read buf before it writes
@@ -668,6 +673,10 @@ __global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float
         float2 fa = make_float2(0.5f * (zk.x + zm_.x), 0.5f * (zk.y - zm_.y));
         float2 fb = make_float2(0.5f * (zk.y + zm_.y), -0.5f * (zk.x - zm_.x));
         if (ZM_EVEN && (k == 0 || 2 * k == w)) fa = fb = make_float2(0.f, 0.f);
+        if (ZM_EVEN) {
+            sq0 += (double)fa.x * (double)fa.x + (double)fa.y * (double)fa.y;
+            sq1 += (double)fb.x * (double)fb.x + (double)fb.y * (double)fb.y;
+        }
         a0[k] = fa;
         if (two) a0[lda + k] = fb;
     }
@@ -687,11 +696,8 @@ __global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float
             s1 += (sh[1][k] + sh[1][k + 1]) + (sh[1][k + 2] + sh[1][k + 3]);
         }
         if (ZM_EVEN) {
-            // Z_0 = Se + So, Z_{w/2} = Se - So (row i0 the real, i1 the imaginary parts):
-            // Se^2 + So^2 = (Z_0^2 + Z_{w/2}^2) / 2
-            const float2 z0 = buf[0], zh = buf[w / 2];
-            s0 -= ((double)z0.x * z0.x + (double)zh.x * zh.x) / (double)w;
-            s1 -= ((double)z0.y * z0.y + (double)zh.y * zh.y) / (double)w;
+            s0 *= 2.0 / (double)w;
+            s1 *= 2.0 / (double)w;
         }
         rowsq_all[(int64_t)b * h + i0] = s0;
         if (two) rowsq_all[(int64_t)b * h + i1] = s1;

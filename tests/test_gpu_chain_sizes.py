@@ -46,6 +46,43 @@ def test_chain_forms(h, w, fmt, rng):
     assert np.abs(got - want).max() <= 2e-5 * max(np.abs(want).max(), 1e-30)
 
 
+def striped(h, w, kind, patch, seed):
+    """A frame whose rows are constant, with one textured patch."""
+    r = np.random.default_rng(seed)
+    y = np.arange(h)
+    row = {"sine": 128 + 100 * np.sin(2 * np.pi * y / 37.3), "bars": np.where(y // 2 % 2, 230, 20),
+           "noise": r.integers(0, 256, h)}[kind]
+    img = np.repeat(np.round(row)[:, None], w, axis=1).astype(np.uint8)
+    img[h // 3:h // 3 + patch, w // 4:w // 4 + patch] = r.integers(0, 256, (patch, patch))
+    return img
+
+
+@pytest.mark.parametrize("h,w,kind,patch", [(1500, 2000, "bars", 8), (1500, 2000, "noise", 8), (1500, 2000, "sine", 64),
+                                            (1000, 1500, "bars", 8), (1080, 1920, "bars", 8), (240, 1000, "bars", 8),
+                                            (240, 1800, "noise", 8), (1536, 2048, "noise", 8), (1536, 2048, "bars", 64),
+                                            (1024, 1024, "noise", 16), (75, 500, "noise", 4)])
+def test_striped_frames(h, w, kind, patch):
+    """Frames whose row means carry nearly all of the energy before the
+    zero-mean, which the Wiener variance must not see."""
+    img = striped(h, w, kind, patch, h + w)
+    want = O.prnu_pattern(img)
+    got = chain(img, _lib.INPUT_GRAY8).reshape(h, w)
+    assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("h,w", [(240, 1000), (1000, 1500), (96, 60)])
+def test_stripes_alone(h, w):
+    """Row-constant frames: the exact pattern is zero and what is left is the
+    rounding of a transform of values up to 1, 2^-24 per value and level (13
+    levels at most), times a scale of at most 1.  (Zero exactly, the scale is
+    0 / 0: NaN.)"""
+    for seed in range(6):
+        for kind in ("noise", "sine", "bars"):
+            img = striped(h, w, kind, 0, seed)
+            got = chain(img, _lib.INPUT_GRAY8)
+            assert np.isnan(got).all() or np.abs(got).max() <= 4 * 13 * 2.0 ** -24
+
+
 # heights and widths of every plan of the column strips (64 threads per column
 # below 1024 rows, 128 up to 2048, 256 up to 4096, 512 above) and of the rows,
 # with an odd number of columns, fewer columns than a strip, and one radix alone
