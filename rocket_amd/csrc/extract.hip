@@ -732,10 +732,11 @@ __global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float
 constexpr int kVX = 64, kVB = 4;
 
 // min-box variances of the lane's column c of LDS rows [oy0, oy0 + V + 8):
-// put(j, varest) for its V output rows.  mask (MASK): the weight, 0 or 1, of
-// the cell `o` columns away at mask[o + 4].
+// put(j, varest) for its V output rows.  in[o + 4] (MASK): whether the cell `o`
+// columns away belongs to the box.  A cell that does not is left out, whatever
+// it holds (a power past FP32 is infinite, and 0 times that no number).
 template <int V, bool MASK, class Put>
-__device__ __forceinline__ void varest_walk(const float (*T)[kVX + 2 * kVB], int oy0, int c, const float *mask,
+__device__ __forceinline__ void varest_walk(const float (*T)[kVX + 2 * kVB], int oy0, int c, const bool *in,
                                             Put put) {
     // output row j sits at LDS row oy0 + j + 4
     float h3[V + 8], h5[V + 8], h7[V + 8], h9[V + 8];
@@ -743,10 +744,16 @@ __device__ __forceinline__ void varest_walk(const float (*T)[kVX + 2 * kVB], int
     for (int i = 0; i < V + 8; ++i) {
         const float *row = &T[oy0 + i][c + kVB];
         if constexpr (MASK) {
-            h3[i] = mask[3] * row[-1] + mask[4] * row[0] + mask[5] * row[1];
-            h5[i] = h3[i] + mask[2] * row[-2] + mask[6] * row[2];
-            h7[i] = h5[i] + mask[1] * row[-3] + mask[7] * row[3];
-            h9[i] = h7[i] + mask[0] * row[-4] + mask[8] * row[4];
+            float e[9];
+#pragma unroll
+            for (int o = -4; o <= 4; ++o) {
+                const float p = row[o];
+                e[o + 4] = in[o + 4] ? p : 0.f;
+            }
+            h3[i] = e[3] + e[4] + e[5];
+            h5[i] = h3[i] + e[2] + e[6];
+            h7[i] = h5[i] + e[1] + e[7];
+            h9[i] = h7[i] + e[0] + e[8];
         } else {
             h3[i] = row[-1] + row[0] + row[1];
             h5[i] = h3[i] + row[-2] + row[2];
@@ -873,10 +880,10 @@ __global__ __launch_bounds__(256) void varest_scale_kernel(const float *P_all, f
     }
     __syncthreads();
     if (idle) return;
-    float mask[9];
+    bool in[9];
 #pragma unroll
-    for (int o = -4; o <= 4; ++o) mask[o + 4] = (gx == 0 ? (o <= 0 && gx + o > -cols) : gx + o >= 1) ? 1.f : 0.f;
-    varest_walk<V, true>(T, oy0, c, mask, [&](int j, float est) {
+    for (int o = -4; o <= 4; ++o) in[o + 4] = gx == 0 ? (o <= 0 && gx + o > -cols) : gx + o >= 1;
+    varest_walk<V, true>(T, oy0, c, in, [&](int j, float est) {
         const int gy = r0 + oy0 + j;
         if (gy <= last && gx < cols) S[(int64_t)gy * cols + gx] = gy == 0 ? s[j] : 0.5f * (s[j] + scale(est));
     });

@@ -83,6 +83,28 @@ def test_stripes_alone(h, w):
             assert np.isnan(got).all() or np.abs(got).max() <= 4 * 13 * 2.0 ** -24
 
 
+def test_wiener_infinite_power_beside_a_box():
+    """Two waves, the first of a power past FP32.  The box of the second holds
+    the first's bin on one side (variance infinite, scale 0) and on the mirrored
+    side, cut by the spectrum's edge, does not (variance P / 81): the first
+    vanishes, the second keeps half of that side's scale.  Tolerance 1e-3 of
+    what is left: the transforms' rounding, 2^-24 of the first wave per bin,
+    is some 1e-4 of it."""
+    h, w, n = 48, 64, 48 * 64
+    y, x = np.mgrid[0:h, 0:w]
+    a, b = 1.3e16, 1.0e16
+    wave = np.cos(2 * np.pi * (21 * x / w + y / h))
+    img = (a * np.cos(2 * np.pi * 20 * x / w) + b * wave).astype(np.float32)
+    assert (n * a / 2) ** 2 > float(np.finfo(np.float32).max) > (n * b / 2) ** 2
+    var = np.sum(img.astype(np.float64) ** 2) * n / (n - 1)
+    want = 0.5 * var / ((n * b / 2) ** 2 / 81) * b * wave
+    f = csi.PRNUFilter(h, w)
+    t = torch.from_numpy(img.ravel()).cuda()
+    f.get_wiener_filter().apply_gpu(t)
+    f.cleanup()
+    assert np.abs(t.cpu().numpy().reshape(h, w) - want).max() <= 1e-3 * np.abs(want).max()
+
+
 # heights and widths of every plan of the column strips (64 threads per column
 # below 1024 rows, 128 up to 2048, 256 up to 4096, 512 above) and of the rows,
 # with an odd number of columns, fewer columns than a strip, and one radix alone
