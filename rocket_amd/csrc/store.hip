@@ -266,16 +266,6 @@ struct StoreGramArgs {
 __device__ __forceinline__ int s_off(int row, int chunk) { return row * kBlkBytes + ((chunk ^ (row & 7)) << 4); }
 
 constexpr int kBufS = kRowsS * kBlkBytes;  // 64 KiB per LDS stage
-// FP16 items work in half blocks (32 values, 64-byte rows) through a ring of
-// five 32 KiB stages, four of them on their way (gram_item_fp16).
-constexpr int kRing16 = 5;
-constexpr int kHalfRow = kBlkBytes / 2;
-constexpr int kBuf16 = kRowsS * kHalfRow;
-template <int FMT, int VAR>
-constexpr int item_lds() {
-    return FMT == PRNU_PREC_FP16 && VAR != 1 ? kRing16 * kBuf16 : 2 * kBufS;
-}
-
 // A wave's FP32 partial block to `out` (row stride 256), without the 16 x 16
 // sub-blocks outside [0, rows) x [0, cols) of it or (tri) wholly below the
 // triangle's diagonal: the reduction does not read them.
@@ -305,102 +295,6 @@ __device__ __forceinline__ void lds_fill16(const uint8_t *base, int bytes, uint8
 #endif
 }
 
-// gram_item for FP16 blocks with direct-to-LDS loads.  An FP16 stage is one
-// product per fragment pair, a third of split-BF16's, so with one 64 KiB stage
-// on its way while the other is multiplied the item waits for memory: 3 us a
-// stage where the fills come from HBM, 0.9 us of it MFMA.  Half blocks make
-// five stages of the CU's 160 KiB of LDS, four in flight: twice the bytes
-// (500, 300 and 120 patterns of 1, 3.1 and 12 M values in one plan: 2.0 ms
-// with the 64 KiB pair, 1.72 ms with the ring; the 120 alone 5.3 TB/s of its
-// blocks).
-// A stage is one K = 32 MFMA per fragment pair; rows are 64 bytes, their four
-// 16-byte chunks XOR-swizzled by (row >> 1) & 3 (conflict-free reads of 16
-// rows).  A wave waits for its own loads of the stage (vmcnt, 4 loads each)
-// and then for the other waves; the same barrier tells it that every wave is
-// done with the stage before, whose buffer the next fill takes.  The sums of
-// an element run over K in the same order as gram_item's: the same bits.
-template <bool SPLIT, bool PRIO>
-__device__ __forceinline__ void gram_item_fp16(const uint8_t *__restrict__ blocks, int64_t cap_bytes, int first,
-                                               int count, int first_b, int count_b, const ItemWaves &w,
-                                               int64_t b_begin, int64_t b_end, int64_t kcb, float *__restrict__ out,
-                                               int rows, int cols, bool tri, uint8_t *lds, int tid) {
-    const bool half = w.nq <= 2;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // load `it` of a stage fills LDS rows 128 it + 16 wave + [0, 16), lane l at
-    // byte 16 l: row l >> 2, slot l & 3, which holds chunk (l & 3) ^ ((row >> 1) & 3)
-    const int lr = lane >> 2, chunk = (lane & 3) ^ ((lr >> 1) & 3);
-    uint32_t voff[4];
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int loc = w.q[it] + 16 * wave + lr;
-        const int slot = it < 2 ? first + min(loc, count - 1) : first_b + min(loc, count_b - 1);
-        voff[it] = (uint32_t)slot * kBlkBytes + (uint32_t)(chunk << 4);
-    }
-    // half blocks of the item and of this wave's own slab
-    const int nst = 2 * (int)(SPLIT ? min(kcb, b_end - b_begin) : b_end - b_begin);
-    const int own = out == nullptr ? 0 : SPLIT ? 2 * (int)min(kcb, b_end - b_begin - w.kw * kcb) : nst;
-    auto issue = [&](int q, uint8_t *buf) {
-        const int64_t b = b_begin + (q >> 1);
-#pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            if (SPLIT || it < 2 || !half) {
-                const int64_t col = SPLIT ? min(b + w.kq[it] * kcb, b_end - 1) : b;
-                lds_fill16(blocks + col * cap_bytes, (int)cap_bytes, buf + (128 * it + 16 * wave) * kHalfRow,
-                           voff[it] + (q & 1) * kHalfRow);
-            }
-        }
-    };
-    floatx4 acc[8][4];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-    for (int d = 0; d < kRing16 - 1; ++d)
-        if (d < nst) issue(d, lds + d * kBuf16);
-    const int frow = lane & 15, ch = lane >> 4;
-    const int roff = frow * kHalfRow + ((ch ^ ((frow >> 1) & 3)) << 4);
-    const int aoff = w.a_off * kHalfRow + roff, boff = w.b_off * kHalfRow + roff;
-    int at = 0, to = kRing16 - 1;  // ring slots of stage q and of stage q + 4
-    for (int q = 0; q < nst; ++q) {
-        // stages asked for after q: wait until only their loads are outstanding
-        // (4 a stage, 2 where the item has two quarters).  s_waitcnt
-        // immediates: vmcnt 3:0, expcnt 6:4 (7: no wait), lgkmcnt 11:8 (0)
-        const int ahead = min(nst - 1 - q, kRing16 - 2);
-        static_assert(kRing16 == 5, "the waits below count three stages ahead");
-        const int left = (!SPLIT && half ? 2 : 4) * ahead;
-        if (left == 12) __builtin_amdgcn_s_waitcnt(0x007c);
-        else if (left == 8) __builtin_amdgcn_s_waitcnt(0x0078);
-        else if (left == 6) __builtin_amdgcn_s_waitcnt(0x0076);
-        else if (left == 4) __builtin_amdgcn_s_waitcnt(0x0074);
-        else if (left == 2) __builtin_amdgcn_s_waitcnt(0x0072);
-        else __builtin_amdgcn_s_waitcnt(0x0070);
-        asm volatile("s_barrier" ::: "memory");
-        if (q + kRing16 - 1 < nst) issue(q + kRing16 - 1, lds + to * kBuf16);
-        if (q < own) {
-            const uint8_t *buf = lds + at * kBuf16;
-            if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
-            halfx8 b0[4];
-#pragma unroll
-            for (int cb = 0; cb < 4; ++cb) b0[cb] = *reinterpret_cast<const halfx8 *>(buf + boff + cb * 16 * kHalfRow);
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb) {
-                const halfx8 a0 = *reinterpret_cast<const halfx8 *>(buf + aoff + rb * 16 * kHalfRow);
-#pragma unroll
-                for (int cb = 0; cb < 4; ++cb)
-                    acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b0[cb], acc[rb][cb], 0, 0, 0);
-            }
-            if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
-        }
-        at = at + 1 == kRing16 ? 0 : at + 1;
-        to = to + 1 == kRing16 ? 0 : to + 1;
-    }
-    __syncthreads();  // a caller may start the next item on the same LDS
-    if (own > 0) write_partial(acc, w, out, rows, cols, tri, lane);
-}
-
 // One work item over the K blocks [b_begin, b_end): LDS rows
 // [128 k, 128 k + 128) hold the patterns w.q[k] + [0, 128) of the slots
 // [first, first+count) for k = 0, 1 and of [first_b, first_b+count_b) for
@@ -412,7 +306,10 @@ __device__ __forceinline__ void gram_item_fp16(const uint8_t *__restrict__ block
 // 2 = direct-to-LDS loads and raised wave priority over the MFMA block.
 // SPLIT (direct loads): an item of w.ks slabs of kcb blocks from b_begin on,
 // cut at nkb = b_end; quarter k is read at slab w.kq[k], a wave stops where
-// its own slab (w.kw) ends.
+// its own slab (w.kw) ends.  (Tried for FP16, whose stage is one product per
+// fragment pair: half blocks through a ring of five 32 KiB stages, four in
+// flight.  120 patterns of 12 M values, all of them split items: 545 us, 498
+// with this pair of 64 KiB stages; 300 of 3.1 M 716 and 705.)
 template <int FMT, int VAR, bool SPLIT>
 __device__ __forceinline__ void gram_item(const uint8_t *__restrict__ blocks, int64_t cap_bytes, int first, int count,
                                           int first_b, int count_b, const ItemWaves &w, int64_t b_begin,
@@ -681,7 +578,6 @@ template <int FMT, int VAR>
 __device__ __forceinline__ void run_item(const uint8_t *blocks, int64_t cap_bytes, int first, int count, int first_b,
                                          int count_b, int ntb, int ks, int S, int64_t nkb, int64_t kcb,
                                          float *partials, int u, int s, uint8_t *lds, int tid = threadIdx.x) {
-    constexpr bool kRing = FMT == PRNU_PREC_FP16 && VAR != 1;
     // wave-uniform: keep it in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     ItemWaves w = ntb > 0 ? rect_waves(u, ntb, wave) : item_waves(u, count, wave, ks);
@@ -702,12 +598,8 @@ __device__ __forceinline__ void run_item(const uint8_t *blocks, int64_t cap_byte
     if (w.ks > 1) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) w.kq[k] = __builtin_amdgcn_readfirstlane(w.kq[k]);
-        if constexpr (kRing)
-            gram_item_fp16<true, VAR == 2>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, nkb, kcb,
-                                           out, rows, cols, true, lds, tid);
-        else
-            gram_item<FMT, VAR == 1 ? 0 : VAR, true>(blocks, cap_bytes, first, count, first_b, count_b, w,
-                                                     b_begin, nkb, kcb, out, rows, cols, true, lds, tid);
+        gram_item<FMT, VAR == 1 ? 0 : VAR, true>(blocks, cap_bytes, first, count, first_b, count_b, w, b_begin, nkb,
+                                                 kcb, out, rows, cols, true, lds, tid);
         return;
     }
     const int64_t b_end = min(nkb, b_begin + kcb);
@@ -950,7 +842,7 @@ __global__ __launch_bounds__(kThr4, 1) void store_gram4_kernel(StoreGramArgs a) 
 // a slab run on one XCD (workgroup ids are dealt to the 8 XCDs round-robin).
 template <int FMT, int VAR>
 __global__ __launch_bounds__(kThrS, 1) void store_gram_kernel(StoreGramArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[item_lds<FMT, VAR>()];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBufS];
     int u, s;
     if (!ItemIndex(a.T, a.ks, a.S).at(blockIdx.x, a.xcd_remap, u, s)) return;
     run_item<FMT, VAR>(a.blocks, a.cap_bytes, a.first, a.count, a.first, a.count, 0, a.ks, a.S, a.nkb, a.kcb,
@@ -977,7 +869,7 @@ struct GroupDev {
 template <int FMT, int VAR>
 __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_kernel(const GroupDev *__restrict__ groups,
                                                                     int ngroups) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[item_lds<FMT, VAR>()];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBufS];
     const int64_t v = blockIdx.x;
     int lo = 0, hi = ngroups - 1;  // last group with v_begin <= v
     while (lo < hi) {
@@ -1016,7 +908,7 @@ template <int FMT>
 __global__ __launch_bounds__(kThrS, 1) void store_gram_groups_persistent_kernel(const GroupDev *__restrict__ groups,
                                                                                int ngroups, int64_t v_total,
                                                                                int *__restrict__ queue) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[item_lds<FMT, 0>()];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kBufS];
     int *taken = reinterpret_cast<int *>(lds);
     const int x = blockIdx.x & 7;
     for (;;) {

@@ -72,6 +72,39 @@ def test_split_item_keeps_the_slabs(slab_blocks):
 
 
 @pytest.mark.parametrize("fmt", ["split_bf16", "fp32", "fp16", "fp8"])
+@pytest.mark.parametrize("count", [120, 300])
+@pytest.mark.parametrize("blocks,per_slab", [(2001, 7), (1201, 4), (900, 3)])
+def test_split_items(fmt, count, blocks, per_slab):
+    """Split items of several stages with short last slabs and groups: near
+    FP64, and the same bits by every way of loading, as a plan's set and from a
+    persistent launch."""
+    values = {"split_bf16": 32, "fp32": 32, "fp16": 64, "fp8": 128}[fmt]
+    n = (values * blocks - 5) // 3 * 3
+    p = patterns(count, n // 3, 3, 4, seed=blocks + count, gain=0.3)
+    want = O.ncc_matrix(p.cpu().numpy())
+    gram = csi.GramNCC(n // 3, 3)
+    store = csi.PatternStore(n, count + 2, fmt)
+    store.put(p, first_slot=2)
+    slabs = -(-blocks // per_slab)
+    assert slabs > 256  # more items than CUs: the last one takes several slabs
+    got = []
+    for variant in (0, 1, 2):
+        cfg = (ctypes.c_int32 * 3)(slabs, 1, variant)
+        _lib.call("prnu_gram_set_config", gram._ctx.handle, _lib.PRECISIONS[fmt], cfg)
+        got.append(store.gram(gram, count, 2).cpu().numpy())
+    plan = csi.GramPlan(gram, [(store, 2, count)], slab_values=values * per_slab)
+    for persistent in (False, True):
+        plan.persistent = persistent
+        got.append(plan.run()[0].cpu().numpy())
+    plan.close()
+    store.close()
+    gram.close()
+    assert np.abs(got[0] - want).max() <= tolerance(fmt, n)
+    for g in got[1:]:
+        assert np.array_equal(g, got[0])
+
+
+@pytest.mark.parametrize("fmt", ["split_bf16", "fp32", "fp16", "fp8"])
 @pytest.mark.parametrize("count,n,first,offset", [(1, 6, 0, 0), (9, 1023, 2, 0), (8, 1024, 0, 0), (17, 1029, 3, 1),
                                                   (5, 5000, 1, 3)])
 def test_put_edges(fmt, count, n, first, offset):
