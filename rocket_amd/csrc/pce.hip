@@ -235,8 +235,12 @@ __device__ __forceinline__ void fft_pass_io_r(int R, float2 *buf, int n, int Ns,
 // Length-d.n DFT of values given by get(i) (each read once) to put(i, X[i])
 // (each written once), through LDS buf (d.n values) for the passes between;
 // ends with a barrier, so the caller may reuse buf.
+// Always inlined: as a function of its own (rows of 8192 values with the
+// reference's Hermitian parts, 98,000 lines of assembly) it is longer than a
+// branch reaches, and the long branches that the compiler then makes overwrite
+// s[30:31], the return address.
 template <int DIR, int MAXN, class Get, class Put>
-__device__ inline void fft_row(float2 *buf, const FftDesc &d, Get get, Put put) {
+__device__ __forceinline__ void fft_row(float2 *buf, const FftDesc &d, Get get, Put put) {
     // the hot lengths with compile-time strides
     if constexpr (MAXN >= 2048) {
         if (d.n == 2048) return fft_row_c<DIR, 2048>(buf, d.tw, get, put);

@@ -128,7 +128,7 @@ def test_wiener_and_spectrum_plans(h, w, rng):
     f.cleanup()
 
 
-@pytest.mark.parametrize("h,w", PLANS)
+@pytest.mark.parametrize("h,w", PLANS + [(12, 7500), (7500, 12)])
 @pytest.mark.parametrize("variant", [_lib.PCE_REFERENCE, _lib.PCE_TEXTBOOK])
 def test_pce_plans(variant, h, w, rng):
     """Relative PCE error <= 1e-4, the bound of every other size."""
