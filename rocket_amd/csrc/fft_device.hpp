@@ -369,12 +369,12 @@ __device__ __forceinline__ void fft_rt(float2 *buf, const FftDesc &d, int lane, 
     }
 }
 
-// One pass of a row whose length is known at compile time.  The first pass
-// (FIRST, Ns = 1, no twiddles) takes its inputs from get(i) instead of LDS and
-// the last (LAST, Ns * R = n) hands its outputs to put(i, v).
 // LDS bytes of a run-time-plan row of n values.
 inline size_t fft_row_smem(int n) { return sizeof(float2) * (size_t)fft_pad_lds(n); }
 
+// One pass of a row whose length is known at compile time.  The first pass
+// (FIRST, Ns = 1, no twiddles) takes its inputs from get(i) instead of LDS and
+// the last (LAST, Ns * R = n) hands its outputs to put(i, v).
 // The length N and the pass's Ns are compile-time constants: strides, twiddle
 // steps and the butterfly index's modulus fold into immediates.  (A pad slot
 // per 8 values measured slower here: the padded addresses cost registers.)
@@ -498,7 +498,6 @@ struct FftWavePlan<2048> {  // radix 16, 16, 8 on two waves
 };
 template <int N>
 constexpr int fft_wave_lds() { return N + (N >> FftWavePlan<N>::kPadShift); }
-constexpr int fft_wave_lds(int n) { return n + n / 16; }  // the 1024-point plan's
 template <int SH = 4>
 __device__ __forceinline__ int fft_wave_pad(int p) { return p + (p >> SH); }
 
@@ -570,7 +569,7 @@ __device__ __forceinline__ void fft_wave_pass(float2 *buf, const float2 *tw, Get
 }
 
 // 1024 points as radix 16, 16, 4 (16 values per lane); get(i) and put(i, X)
-// as fft_rt's.  buf: fft_wave_lds(1024) values.
+// as fft_rt's.  buf: fft_wave_lds<1024>() values.
 template <int DIR, bool SYNC_FIRST = false, bool WSYNC = false, class Get, class Put>
 __device__ __forceinline__ void fft_wave_1024(float2 *buf, const float2 *tw, Get get, Put put) {
     fft_wave_pass<16, DIR, true, false, 1024, 1, SYNC_FIRST, 4, 64, WSYNC>(buf, tw, get, put);

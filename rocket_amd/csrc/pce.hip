@@ -163,7 +163,8 @@ __device__ __forceinline__ void herm_pair(const float2 *X, const float2 *Y, int 
 }
 
 // ------------------------------------- transforms of a run-time length
-// The rows and columns of the lengths without a plan of their own: a 256-thread
+// The rows and columns that pce_rows_mirror_wave_kernel (1024 and 2048 columns)
+// and pce_cols_kernel (1024 and 1536 rows) do not take: a 256-thread
 // workgroup each, radices 8, 4, 2, 3, 5 (fft_desc_basic), one template
 // instance per pass.  A score divides the square of one value by an energy
 // whose bias the roundings do not average out, so the plans of the extraction
@@ -241,13 +242,10 @@ __device__ __forceinline__ void fft_pass_io_r(int R, float2 *buf, int n, int Ns,
 // s[30:31], the return address.
 template <int DIR, int MAXN, class Get, class Put>
 __device__ __forceinline__ void fft_row(float2 *buf, const FftDesc &d, Get get, Put put) {
-    // the hot lengths with compile-time strides
-    if constexpr (MAXN >= 2048) {
+    // with compile-time strides: columns of 2048, rows of 1536 values
+    if constexpr (MAXN == kFftSmallN) {
         if (d.n == 2048) return fft_row_c<DIR, 2048>(buf, d.tw, get, put);
         if (d.n == 1536) return fft_row_c<DIR, 1536>(buf, d.tw, get, put);
-    }
-    if constexpr (MAXN >= 1024) {
-        if (d.n == 1024) return fft_row_c<DIR, 1024>(buf, d.tw, get, put);
     }
     const int P = d.passes;
     if (P == 1) {
@@ -310,7 +308,7 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows2_kernel(FftDesc d, int h
 // spectrum reads of pce_rows2_kernel, whose two workgroups per pair each
 // form their own row's Hermitian parts.  grid (h/2 + 1, couples), LDS 3w
 // complex (H_a, H_b of row u, the transform buffer).
-template <int VARIANT, int MAXN>
+template <int VARIANT>
 __global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d, int h, int nb, PceBatch bt,
                                                                       float2 *__restrict__ Aall, int64_t pstride) {
     extern __shared__ float2 smem[];
@@ -337,7 +335,7 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d,
     }
     __syncthreads();
     float2 *A = Aall + (int64_t)q * pstride;
-    fft_row<1, MAXN>(
+    fft_row<1, kFftSmallN>(
         buf, d,
         [&](int j) {
             const float2 a = ha[j], b = hb[j];
@@ -345,7 +343,7 @@ __global__ __launch_bounds__(kFftThreads) void pce_rows_mirror_kernel(FftDesc d,
         },
         [&](int j, float2 f) { A[(int64_t)u * w + j] = f; });
     if (um == u) return;
-    fft_row<1, MAXN>(
+    fft_row<1, kFftSmallN>(
         buf, d,
         [&](int j) {
             const int mj = j == 0 ? 0 : w - j;
@@ -421,11 +419,12 @@ __global__ __launch_bounds__(kFftThreads) void pce_cols_row_kernel(FftDesc d, in
 // with four: all waves form H_a, H_b of row u into LDS together, then the first
 // half transforms row u and the second row -u at the same time (the passes of
 // fft_wave_1024 / fft_block_2048_r8; two waves per row at 2048, radix 16, 16,
-// 8, round a little less well: 1.3e-7 against 1.1e-7 of the score), their transform buffers laid over H_a, H_b
-// once the first pass has read them.  When u is its own mirror, the second
-// half transforms and stores nothing of its own (it still takes part in every
-// barrier).  At 2048 columns each row by its own workgroup, reading its
-// Hermitian parts for itself, measured 597 us per 66 pairs of 2048x1536.
+// 8, round a little less well: 1.3e-7 against 1.1e-7 of the score), their
+// transform buffers laid over H_a, H_b once the first pass has read them.  When
+// u is its own mirror, the second half transforms and stores nothing of its own
+// (it still takes part in every barrier).  At 2048 columns each row by its own workgroup, reading its
+// Hermitian parts for itself, measured 577 us per 66 pairs of 2048x1536, in
+// mirror pairs 457 us.
 // grid (h/2 + 1, couples), 2 T threads.
 template <int W>
 constexpr int mirror_row_threads() { return W == 1024 ? 64 : 256; }
@@ -493,7 +492,7 @@ __global__ __launch_bounds__(2 * mirror_row_threads<W>()) void pce_rows_mirror_w
 // strips (cols_device.hpp): inverse FFT of length h; every output value goes
 // straight into its thread's sums of Re (pair 2q) and Im (pair 2q + 1) -- FP64
 // energy and the max |value| with its linear index i*w + j, smallest index on
-// ties -- which a fixed-order reduction over the column's waves turns into the
+// ties -- which a fixed-order reduction over the column's wave turns into the
 // column's partials.  grid (8 per, couples).  (66 pairs of 2048x1536: 1310 us
 // with 301 us of transposes and 373 us of pce_cols_row_kernel and the rows one
 // by one, 1006 us with these strips and the rows in mirror pairs.)
@@ -506,13 +505,12 @@ __global__ __launch_bounds__(P::kThreads) void pce_cols_kernel(P pl, int w, int 
     if (strip >= (w + P::COLS - 1) / P::COLS) return;
     const int q = blockIdx.y, j0 = strip * P::COLS;
     stage_cols(pl, Aall + (int64_t)q * pstride, w, j0, w, pce_smem);
-    const int c = (int)threadIdx.x / P::T, j = j0 + c;
+    static_assert(P::T == 64, "pce_cols_kernel: one wave per column");
+    const int c = (int)threadIdx.x / P::T, t = (int)threadIdx.x & (P::T - 1), j = j0 + c;
     float2 *buf = pce_smem + c * pl.stride();
     double e0 = 0.0, e1 = 0.0;
     float b0 = -1.0f, b1 = -1.0f;
     int i0 = 0x7fffffff, i1 = 0x7fffffff;
-    constexpr int kWaves = P::T / 64;  // of a column
-    const int t = (int)threadIdx.x & (P::T - 1);
     auto add = [&](int i, float2 z) {
         const int idx = i * w + j;
         e0 += (double)z.x * (double)z.x;
@@ -533,24 +531,7 @@ __global__ __launch_bounds__(P::kThreads) void pce_cols_kernel(P pl, int w, int 
         argmax_merge(b1, i1, v2, k2);
     }
     const int halves = 2 * q + 1 < nb ? 2 : 1;
-    if constexpr (kWaves > 1) {  // every wave has read its column
-        PeakPart *sh = reinterpret_cast<PeakPart *>(buf);
-        if ((t & 63) < 2) {
-            PeakPart &p = sh[2 * (t >> 6) + (t & 63)];
-            p.energy = (t & 63) == 0 ? e0 : e1;
-            p.absmax = (t & 63) == 0 ? b0 : b1;
-            p.index = (t & 63) == 0 ? i0 : i1;
-        }
-        __syncthreads();
-        if (t < halves && j < w) {
-            PeakPart p = sh[t];
-            for (int k = 1; k < kWaves; ++k) {
-                p.energy += sh[2 * k + t].energy;
-                argmax_merge(p.absmax, p.index, sh[2 * k + t].absmax, sh[2 * k + t].index);
-            }
-            partall[(int64_t)(2 * q + t) * w + j] = p;
-        }
-    } else if (t < halves && j < w) {
+    if (t < halves && j < w) {
         PeakPart p;
         p.energy = t == 0 ? e0 : e1;
         p.absmax = t == 0 ? b0 : b1;
@@ -759,16 +740,15 @@ __global__ __launch_bounds__(256) void transpose_kernel(const float2 *__restrict
 }
 
 template <int V, int MAXN>
-void launch_pce_rows_rt(const FftDesc &dw, dim3 mgrid, dim3 rgrid, int h, int nb, const PceBatch &bt, float2 *A,
-                        int64_t pstride, hipStream_t st) {
-    if (dw.n <= 1024)  // both rows of a mirror pair in one workgroup (24 KiB of LDS)
-        hipLaunchKernelGGL((pce_rows_mirror_kernel<V, MAXN>), mgrid, dim3(kFftThreads),
-                           3 * sizeof(float2) * (size_t)dw.n, st, dw, h, nb, bt, A, pstride);
-    else
-        hipLaunchKernelGGL((pce_rows2_kernel<V, MAXN>), rgrid, dim3(kFftThreads), sizeof(float2) * (size_t)dw.n, st, dw,
-                           h, nb, bt, A, pstride);
+void launch_pce_rows2(const FftDesc &dw, dim3 rgrid, int h, int nb, const PceBatch &bt, float2 *A, int64_t pstride,
+                      hipStream_t st) {
+    hipLaunchKernelGGL((pce_rows2_kernel<V, MAXN>), rgrid, dim3(kFftThreads), sizeof(float2) * (size_t)dw.n, st, dw, h,
+                       nb, bt, A, pstride);
 }
 
+// Mirror pairs of rows up to 1024 values (24 KiB of LDS) and at 2048, where the
+// pair kernel has a plan (66 pairs of 2048x1536: 577 us row by row, 457 so);
+// between and above them row by row: the pair form has not been measured there.
 template <int V>
 int launch_pce_rows(const FftDesc &dw, dim3 mgrid, dim3 rgrid, int h, int nb, const PceBatch &bt, float2 *A,
                     int64_t pstride, hipStream_t st) {
@@ -778,12 +758,15 @@ int launch_pce_rows(const FftDesc &dw, dim3 mgrid, dim3 rgrid, int h, int nb, co
     else if (dw.n == 2048)
         hipLaunchKernelGGL((pce_rows_mirror_wave_kernel<V, 2048>), mgrid, dim3(512), 0, st, dw.tw, h, nb, bt, A,
                            pstride);
+    else if (dw.n < 1024)
+        hipLaunchKernelGGL(pce_rows_mirror_kernel<V>, mgrid, dim3(kFftThreads), 3 * sizeof(float2) * (size_t)dw.n, st,
+                           dw, h, nb, bt, A, pstride);
     else if (dw.n <= kFftSmallN)
-        launch_pce_rows_rt<V, kFftSmallN>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st);
+        launch_pce_rows2<V, kFftSmallN>(dw, rgrid, h, nb, bt, A, pstride, st);
     else if (dw.n <= kFftMidN)
-        launch_pce_rows_rt<V, kFftMidN>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st);
+        launch_pce_rows2<V, kFftMidN>(dw, rgrid, h, nb, bt, A, pstride, st);
     else
-        launch_pce_rows_rt<V, kFftMaxN>(dw, mgrid, rgrid, h, nb, bt, A, pstride, st);
+        launch_pce_rows2<V, kFftMaxN>(dw, rgrid, h, nb, bt, A, pstride, st);
     PRNU_CHECK_LAUNCH();
     return PRNU_OK;
 }
@@ -818,7 +801,10 @@ int pce_batch(Context *c, int variant, const PceBatch &bt, int nb, double *out, 
     const size_t pbytes = ((sizeof(PeakPart) * w) + 255) & ~size_t(255);
     const int64_t pstride = (int64_t)(plane / sizeof(float2));
     const size_t wbytes = ((sizeof(double) * kWinSlots * nb) + 255) & ~size_t(255);
-    const bool strips = h == 1024 || h == 1536;  // columns read from the rows' own layout
+    // columns read from the rows' own layout, where cols_device.hpp has a plan of
+    // PCE's radices; other heights (2048 among them, which has none) through a
+    // transpose
+    const bool strips = h == 1024 || h == 1536;
     const size_t planes = plane * couples * (strips ? 1 : 2);
     PRNU_TRY(c->ws_pce.ensure(planes + pbytes * nb + wbytes));
     char *base = static_cast<char *>(c->ws_pce.ptr);
