@@ -128,12 +128,34 @@ def test_wiener_and_spectrum_plans(h, w, rng):
     f.cleanup()
 
 
-@pytest.mark.parametrize("h,w", PLANS + [(12, 7500), (7500, 12)])
+@pytest.mark.parametrize("h,w", [(24, 512), (25, 500), (500, 540)])
+def test_batch_equals_single_across_the_stencil(h, w, rng):
+    """24 frames fill the chip with the variance stencil's long tiles, one frame
+    takes the short ones: the same bits."""
+    count = max(24, -(-512 // (-(-h // 64) * ((w // 2 + 128) // 128))))
+    imgs = torch.from_numpy(rng.integers(0, 256, size=(count, h * w), dtype=np.uint8)).cuda()
+    f = csi.PRNUFilter(h, w)
+    out, one = torch.empty((count, h * w), device="cuda"), torch.empty(h * w, device="cuda")
+    f.apply_gpu_batch(imgs, out, _lib.INPUT_GRAY8)
+    for i in (0, count // 2, count - 1):
+        f.apply_gpu(imgs[i], one, _lib.INPUT_GRAY8)
+        assert torch.equal(out[i], one)
+    f.cleanup()
+
+
+# PCE's forms: rows of 1024 and 2048 values in mirror pairs, shorter ones too,
+# longer ones and 1536 one by one; columns of 1024 and 1536 by strips (16-byte
+# and, for odd widths, 8-byte staging, a last strip of few columns), the others
+# through a transpose in three size classes; even and odd numbers of rows
+PCE_PLANS = [(16, 20), (600, 45), (1200, 18), (2000, 27), (1536, 15), (1024, 30), (20, 1800), (12, 2500), (12, 2048),
+             (15, 2048), (15, 1024), (96, 1024), (1536, 64), (1536, 2048), (1024, 45), (16, 1536), (12, 7500),
+             (2048, 24), (2250, 18), (4374, 12), (7500, 12), (8100, 12), (2048, 1536)]
+
+
+@pytest.mark.parametrize("h,w", PCE_PLANS)
 @pytest.mark.parametrize("variant", [_lib.PCE_REFERENCE, _lib.PCE_TEXTBOOK])
 def test_pce_plans(variant, h, w, rng):
     """Relative PCE error <= 1e-4, the bound of every other size."""
-    if h * w <= 121 or min(h, w) < 11:
-        pytest.skip("the window covers the plane or wraps onto itself")
     k = rng.normal(size=(h, w))
     pats = [(0.5 * k + rng.normal(size=(h, w))).astype(np.float32) for _ in range(3)]
     spec = [np.ascontiguousarray(O.spectrum(p).astype(np.complex64)) for p in pats]
