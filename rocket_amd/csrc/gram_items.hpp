@@ -13,7 +13,7 @@ namespace prnu {
 constexpr int kGramTile = 256;  // patterns per side of a partial tile
 
 // Linear index over the upper triangle (row-major, I <= J) -> (I, J).
-__device__ inline int2 tri_tile(int t, int nt) {
+__host__ __device__ inline int2 tri_tile(int t, int nt) {
     int I = 0;
     while (t >= nt - I) {
         t -= nt - I;
@@ -67,15 +67,15 @@ struct ItemWaves {
 };
 
 // First pattern of LDS row `row` (a multiple of 64); no indexed private array.
-__device__ __forceinline__ int row_pattern(const ItemWaves &w, int row) {
+__host__ __device__ __forceinline__ int row_pattern(const ItemWaves &w, int row) {
     const int k = row >> 7;
     const int q0 = w.q[0], q1 = w.q[1], q2 = w.q[2], q3 = w.q[3];
     return (k < 2 ? (k == 0 ? q0 : q1) : (k == 2 ? q2 : q3)) + (row & 127);
 }
 
-__device__ __forceinline__ int tri_index(int I, int J, int nt) { return I * nt - I * (I - 1) / 2 + (J - I); }
+__host__ __device__ __forceinline__ int tri_index(int I, int J, int nt) { return I * nt - I * (I - 1) / 2 + (J - I); }
 
-__device__ __forceinline__ void item_tiles(ItemWaves &r, int x, int y) {
+__host__ __device__ __forceinline__ void item_tiles(ItemWaves &r, int x, int y) {
     r.q[0] = x * kGramTile;
     r.q[1] = x * kGramTile + 128;
     r.q[2] = y * kGramTile;
@@ -94,7 +94,7 @@ __host__ __device__ inline int slab_split(int count) {
 // Item u of a slab of the triangle of `count` patterns, the last one taking ks
 // slabs (1 or slab_split(count)) (nt = ceil(count /
 // 256) partial tiles), for wave `wave`.
-__device__ __forceinline__ ItemWaves item_waves(int u, int count, int wave, int ks) {
+__host__ __device__ __forceinline__ ItemWaves item_waves(int u, int count, int wave, int ks) {
     ItemWaves r;
     r.ks = 1;
     r.kq[0] = r.kq[1] = r.kq[2] = r.kq[3] = r.kw = 0;
@@ -214,7 +214,7 @@ struct ItemIndex {
 };
 
 // A rectangle of nt x ntb tiles: item u = tile (u / ntb, u % ntb).
-__device__ __forceinline__ ItemWaves rect_waves(int u, int ntb, int wave) {
+__host__ __device__ __forceinline__ ItemWaves rect_waves(int u, int ntb, int wave) {
     ItemWaves r;
     r.ks = 1;
     r.kq[0] = r.kq[1] = r.kq[2] = r.kq[3] = r.kw = 0;

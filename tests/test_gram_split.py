@@ -1,59 +1,70 @@
-"""Host check of the slab-split work items (no GPU): a mirror of ItemIndex and
-slab_split (rocket_amd/csrc/gram_items.hpp) must give every (item, slab) of
-the triangle exactly once, the split item's slabs in groups of ks, and deal
-both kinds of items evenly over the 8 XCDs (id mod 8)."""
+"""Host check of the Gram's work items (no GPU): rocket_amd/csrc/gram_items.hpp
+itself, compiled for the host (gram_items_driver.cpp), must multiply every
+128 x 64 block that meets the upper triangle exactly once per slab, from rows
+that the item loads at that slab, into that block's place of its partial tile;
+a split item must take its slabs in groups of ks; and both kinds of items must
+be dealt evenly over the 8 XCDs (id mod 8)."""
+import pathlib
+import shutil
+import subprocess
+
+import numpy as np
 import pytest
 
-
-def items_per_slab(count):
-    Q, m = (count + 127) >> 7, (count + 127) >> 8
-    return m * (m - 1) // 2 + (m + (m + 4) // 4 if Q % 2 else (6 * m + 7) // 8)
+HERE = pathlib.Path(__file__).parent
 
 
-def slab_split(count):
-    Q = (count + 127) >> 7
-    if Q % 2 == 0:
-        return 1
-    return {1: 4, 2: 2}.get(((Q >> 1) + 1) & 3, 1)
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    if not shutil.which("g++") or not pathlib.Path("/opt/rocm/include/hip/hip_runtime.h").exists():
+        pytest.skip("needs g++ and the HIP headers")
+    exe = tmp_path_factory.mktemp("gram") / "gram_items_driver"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    str(HERE / "gram_items_driver.cpp"), "-o", str(exe)], check=True)
 
-
-def ids(T, ks, S, remap):
-    Tn, groups = T - (ks > 1), -(-S // ks) if ks > 1 else 0
-    up = lambda v: -(-v // 8) * 8 if remap else v   # noqa: E731
-    return Tn * up(S) + up(groups)
-
-
-def at(i, T, ks, S, remap):
-    Tn = T - (ks > 1)
-    S8 = -(-S // 8) * 8 if remap else S
-    if i >= Tn * S8:
-        return Tn, (i - Tn * S8) * ks
-    return ((i >> 3) % Tn, (i >> 3) // Tn * 8 + (i & 7)) if remap else (i % Tn, i // Tn)
+    def run(count, ks, S, remap):
+        out = subprocess.run([str(exe), str(count), str(ks), str(S), str(int(remap))], check=True,
+                             capture_output=True, text=True).stdout.splitlines()
+        return [int(v) for v in out[0].split()], np.array([[int(v) for v in ln.split()] for ln in out[1:]])
+    return run
 
 
 @pytest.mark.parametrize("remap", [True, False])
 @pytest.mark.parametrize("S", [1, 3, 8, 37, 64])
 @pytest.mark.parametrize("count", [1, 120, 128, 129, 300, 384, 600, 800, 1100, 1400])
-def test_every_item_and_slab_once(count, S, remap):
-    T, ks = items_per_slab(count), slab_split(count)
-    seen, xcds = {}, [0] * 8
-    for i in range(ids(T, ks, S, remap)):
-        u, s = at(i, T, ks, S, remap)
-        if s >= S:
-            continue
-        split = ks > 1 and u == T - 1
-        xcds[i & 7] += 1
-        for k in range(ks if split else 1):
-            if s + k < S:
-                seen[u, s + k] = seen.get((u, s + k), 0) + 1
-    assert seen == {(u, s): 1 for u in range(T) for s in range(S)}
-    if remap:
-        assert max(xcds) - min(xcds) <= T
+def test_every_block_and_slab_once(driver, count, S, remap):
+    T, split, _ = driver(count, 1, 1, False)[0]
+    for ks in {1, split}:
+        _, rows = driver(count, ks, S, remap)
+        ident, u, first, wave, a, b, kqa, kqb, kw, tile, off = rows.T
+        assert (first + 0 < S).all() and (kqa == kw).all() and (kqb == kw).all()
+        assert (kw[(u < T - 1) | (ks == 1)] == 0).all()        # only the last item takes several slabs
+        assert (first[(u == T - 1) & (ks > 1)] % ks == 0).all() and kw.max() < ks
+        # the block's place in its partial tile (the triangle's tiles, row by row)
+        nt = (count + 255) // 256
+        ti, tj = a // 256, b // 256
+        assert (tile == ti * nt - ti * (ti - 1) // 2 + (tj - ti)).all()
+        assert (off == (a % 256) * 256 + b % 256).all()
+        # every block that meets the triangle of the patterns, once per slab
+        slab = first + kw
+        here = slab < S                                        # past the last slab: not written
+        got = sorted(zip(slab[here], a[here], b[here]))
+        assert len(set(got)) == len(got)
+        need = {(s, i, j) for s in range(S) for i in range(0, count, 128) for j in range(0, count, 64)
+                if j + 63 >= i and (i // 128) <= (j // 128)}
+        assert need <= set(got)
+        assert all(i // 128 <= j // 128 for _, i, j in got)
+        if remap:
+            per_xcd = np.bincount(np.unique(ident[u < T - (ks > 1)]) & 7, minlength=8)
+            assert per_xcd.max() - per_xcd.min() <= T
+            per_xcd = np.bincount(np.unique(ident[(u == T - 1) & (ks > 1)]) & 7, minlength=8)
+            assert per_xcd.max() - per_xcd.min() <= 1
 
 
 @pytest.mark.parametrize("count,ks", [(1, 4), (128, 4), (129, 1), (300, 2), (600, 1), (800, 1), (1100, 4), (1300, 2)])
-def test_split_fills_the_last_item(count, ks):
-    assert slab_split(count) == ks
-    m = (count + 127) >> 8
-    if ks > 1:  # the one-quarter units of the last item, times ks, are the item's four
-        assert ((m + 1) % 4) * ks == 4
+def test_split_fills_the_last_item(driver, count, ks):
+    (T, split, _), rows = driver(count, ks, 4, False)
+    assert split == ks
+    last = rows[rows[:, 1] == T - 1]
+    if ks > 1:  # its eight waves all work in a full group of slabs
+        assert set(last[last[:, 2] == 0][:, 3]) == set(range(8))
