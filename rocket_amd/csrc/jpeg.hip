@@ -859,13 +859,13 @@ bool build_huff(const RawHuff &r, HuffTab &t) {
 }
 
 // Two-level decoding table of one Huffman table, appended to `out` (uint16
-// entries): kLook2 first-level entries indexed by the next 9 bits, then the
-// second-level subtables.  An entry is (length << 8) | symbol for a code of
-// at most 9 bits (first level) or of any length (second level), 0 for no
-// code, or, in the first level, 0x8000 | (nb << 12) | off for the 9-bit
-// prefix of longer codes: their entry is at second-level index off + the nb
-// bits after the prefix (nb = longest such code - 9).  off == 0xFFF: the
-// subtable did not fit in `budget` entries; decoded by the canonical walk.
+// entries): 512 first-level entries indexed by the next 9 bits, then the
+// second-level subtables.  An entry is sym_entry's for a code of at most 9 bits
+// (first level) or of any length (second level), bad_entry's for no code, or, in
+// the first level, 0x8000 | (nb << 12) | off for the 9-bit prefix of longer
+// codes: their entry is at second-level index off + the nb bits after the
+// prefix (nb = longest such code - 9).  off == 0xFFF: the subtable did not fit
+// in `budget` entries; decoded by the canonical walk.
 // The table has passed build_huff (no over-subscribed length).
 void build_lut2(const RawHuff &r, bool dc, std::vector<uint16_t> &out, int budget) {
     std::vector<uint16_t> L(512, (uint16_t)bad_entry(dc)), sub;
@@ -878,7 +878,7 @@ void build_lut2(const RawHuff &r, bool dc, std::vector<uint16_t> &out, int budge
     for (int l = 1; l <= 16; ++l) {
         for (int i = 0; i < r.counts[l - 1]; ++i, ++code, ++k) {
             if (l <= 9) {
-                for (int j = 0; j < (1 << (9 - l)); ++j) 
+                for (int j = 0; j < (1 << (9 - l)); ++j)
                     L[(code << (9 - l)) + j] = (uint16_t)sym_entry(l, r.vals[k], dc);
             } else {
                 const int p = code >> (l - 9);
@@ -903,7 +903,7 @@ void build_lut2(const RawHuff &r, bool dc, std::vector<uint16_t> &out, int budge
         if ((L[p] & 0xFFF) == 0xFFF) continue;
         const int nb = (L[p] >> 12) & 7, off = L[p] & 0xFFF, extra = c.l - 9;
         const int rest = c.code & ((1 << extra) - 1), span = 1 << (nb - extra);
-        for (int j = 0; j < span; ++j) 
+        for (int j = 0; j < span; ++j)
             sub[off + (rest << (nb - extra)) + j] = (uint16_t)sym_entry(c.l, c.sym, dc);
     }
     out.insert(out.end(), L.begin(), L.end());
