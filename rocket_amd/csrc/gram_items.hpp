@@ -195,6 +195,8 @@ struct ItemIndex {
         return Tn * S8 + (remap ? (groups() + 7) / 8 * 8 : groups());
     }
     __host__ __device__ int64_t items() const { return (int64_t)Tn * S + groups(); }
+    // items of the XCD that gets the most (ids mod 8 = 0)
+    __host__ __device__ int64_t xcd_items() const { return (int64_t)Tn * ((S + 7) / 8) + (groups() + 7) / 8; }
     // id -> item u and its first slab s; false: padding
     __host__ __device__ bool at(int64_t id, bool remap, int &u, int &s) const {
         const int64_t S8 = remap ? (S + 7) / 8 * 8 : S, normal = Tn * S8;
@@ -230,10 +232,10 @@ __host__ __device__ __forceinline__ ItemWaves rect_waves(int u, int ntb, int wav
 
 
 // Blocks of K per slab, at most `longest` (0: no limit), and per set g the
-// slabs splits[g] (in: slab_split, out: that or 1) its last item takes:
-// store.hip.
-int64_t choose_slab(const int *items, int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
-                    size_t max_bytes, int64_t longest);
+// slabs splits[g] (in: slab_split, out: that or 1) its last item takes, for
+// products of format `precision`: store.hip.
+int64_t choose_slab(const int *items, int *splits, const int *tiles, const int64_t *nkb, int ngroups, int precision,
+                    int cus, size_t max_bytes, int64_t longest);
 int device_cus(int device);
 // FP64 sum of the S partials of every element and the NCC epilogue: store.hip.
 int launch_tri_reduce(const float *partials, int S, int nt, int count, const double *sum, const double *sumsq,

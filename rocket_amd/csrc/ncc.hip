@@ -736,12 +736,12 @@ GramPlan plan_gram(const Context *c, int count, int precision) {
         int64_t S = std::min<int64_t>(c->gram_cfg[precision].slabs, stages);
         S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * p.tiles)));
         p.kchunk = ((stages + S - 1) / S) * kKT;
-        if (p.T * S <= device_cus(c->device)) p.ks = 1;  // (choose_slab)
+        if (p.T * ((S + 7) / 8) * 8 <= device_cus(c->device)) p.ks = 1;  // (choose_slab)
     } else {
         int64_t S = std::max<int64_t>(1, (256 * 5 + p.tiles - 1) / p.tiles);
         S = std::min<int64_t>(S, std::max<int64_t>(1, stages / 16));
         S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * p.tiles)));
-        p.kchunk = kKT * choose_slab(&p.T, &p.ks, &p.tiles, &stages, 1, device_cus(c->device), size_t(2) << 30,
+        p.kchunk = kKT * choose_slab(&p.T, &p.ks, &p.tiles, &stages, 1, precision, device_cus(c->device), size_t(2) << 30,
                                      (stages + S - 1) / S);
     }
     p.S = (K + p.kchunk - 1) / p.kchunk;

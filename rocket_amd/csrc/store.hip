@@ -1064,55 +1064,86 @@ int device_cus(int device) {
     return cus;
 }
 
-// Blocks per slab for groups of (items per slab, K blocks): all work items
-// cost about kcb block-stages and one CU runs one item at a time, so the
-// launch takes about ceil(items / cus) * kcb stages, plus a per-slab cost
-// (the partial tile each item writes and the reduction reads, ~2 stages).
-// splits[g]: the slabs the last item of group g takes at once (slab_split).
-// Searches kcb and returns the cheapest whose partial tiles fit `max_bytes`.
-// `longest` (if > 0) bounds the slab: an FP32 accumulator's rounding error
-// grows with it.
-static int64_t choose_kcb(const int *items, const int *splits, const int *tiles, const int64_t *nkb, int ngroups,
-                          int cus, size_t max_bytes, int64_t longest, double *best_cost) {
-    int64_t max_nkb = 1;
-    for (int g = 0; g < ngroups; ++g) max_nkb = std::max(max_nkb, nkb[g]);
-    double best = 1e300;
-    if (longest > 0) max_nkb = std::min(max_nkb, longest);
-    int64_t best_kcb = max_nkb;
-    for (int64_t kcb = std::min<int64_t>(16, max_nkb); kcb <= max_nkb; kcb += (kcb < 256 ? 8 : kcb < 2048 ? 32 : 256)) {
-        double total = 0.0, part = 0.0;
-        for (int g = 0; g < ngroups; ++g) {
-            const int64_t S = (nkb[g] + kcb - 1) / kcb;
-            total += (double)ItemIndex(items[g], splits[g], (int)std::min<int64_t>(S, 1 << 30)).items();
-            part += (double)tiles[g] * S * kTileS * kTileS * sizeof(float);
-        }
+namespace {
+
+// Shortest slab worth its own partial tile, and the steps of the search above it.
+constexpr int64_t kKcbMin = 16;
+int64_t kcb_step(int64_t kcb) { return kcb < 256 ? 8 : kcb < 2048 ? 32 : 256; }
+
+// The kcb (blocks per slab) of least cost(kcb) whose partial tiles fit
+// `max_bytes`, at most `longest` (if > 0); `most` if none fits.
+template <class Cost>
+int64_t search_kcb(const int *tiles, const int64_t *nkb, int ngroups, size_t max_bytes, int64_t longest, Cost cost,
+                   double *best_cost) {
+    int64_t most = 1;
+    for (int g = 0; g < ngroups; ++g) most = std::max(most, nkb[g]);
+    if (longest > 0) most = std::min(most, longest);
+    int64_t best_kcb = most;
+    *best_cost = 1e300;
+    for (int64_t kcb = std::min(kKcbMin, most); kcb <= most; kcb += kcb_step(kcb)) {
+        double part = 0.0;
+        for (int g = 0; g < ngroups; ++g)
+            part += (double)tiles[g] * ((nkb[g] + kcb - 1) / kcb) * kTileS * kTileS * sizeof(float);
         if (part > (double)max_bytes) continue;
-        const double rounds = std::ceil(total / cus);
-        const double cost = rounds * (double)(kcb + 2);
-        if (cost < best * (1.0 - 1e-9)) {
-            best = cost;
+        const double c = cost(kcb);
+        if (c < *best_cost * (1.0 - 1e-9)) {
+            *best_cost = c;
             best_kcb = kcb;
         }
     }
-    *best_cost = best;
     return best_kcb;
 }
 
-// The slab of a set of triangles and rectangles: the cheapest with every item
-// taking one slab at a time, or a shorter one whose split items cost less (not
-// longer: items of several slabs are there to shorten the launch, not at the
-// price of the sums' precision).  A set that does not fill the CUs keeps one
-// slab per item: its launch is one item's length either way, and an item of
-// four slabs loads four times the rows (3 patterns of 162x72: 81 us a call,
-// 92 with split items).
-int64_t choose_slab(const int *items, int *splits, const int *tiles, const int64_t *nkb, int ngroups, int cus,
-                    size_t max_bytes, int64_t longest) {
+}  // namespace
+
+// The slab of a set of triangles and rectangles.  All work items cost about kcb
+// block-stages and one CU runs one item at a time, so a launch takes its rounds
+// of items times kcb, plus a cost per slab (the partial tile each item writes
+// and the reduction reads).
+// First the cheapest with every item taking one slab: rounds of the whole chip,
+// 2 stages a slab.  Then a shorter one whose split items cost less (not longer:
+// an FP32 accumulator's rounding error grows with the slab).  That comparison
+// counts the items of the busiest XCD, ids going to the XCDs round-robin: 510
+// items in two rounds of 256 CUs were three, 65 of them on the first XCD (380
+// patterns of 2 M values, FP32 3860 us whole, 4395 so; 3025 in rounds that
+// fit).  And it counts 24 stages a slab, 2 for FP32 products: beside the partial
+// tile, a split item reads its quarters from HBM again where the others share
+// an XCD's L2, which shows where a stage is one product (380 of 786,432, FP16:
+// 206 us whole, 288 in 512 slabs of 24 blocks, 192 in 154 of 80).
+// A set that does not fill the CUs keeps one slab per item: its launch is one
+// item's length either way, and an item of four slabs loads four times the rows
+// (3 patterns of 162x72: 81 us a call, 92 with split items).
+int64_t choose_slab(const int *items, int *splits, const int *tiles, const int64_t *nkb, int ngroups, int precision,
+                    int cus, size_t max_bytes, int64_t longest) {
     const std::vector<int> one(ngroups, 1);
-    double cost_one = 0.0, cost = 0.0;
-    const int64_t kcb_one = choose_kcb(items, one.data(), tiles, nkb, ngroups, cus, max_bytes, longest, &cost_one);
-    const int64_t kcb = choose_kcb(items, splits, tiles, nkb, ngroups, cus, max_bytes, kcb_one, &cost);
-    if (cost < cost_one) return kcb;
-    std::copy(one.begin(), one.end(), splits);
+    auto index = [&](const int *ks, int g, int64_t kcb) {
+        return ItemIndex(items[g], ks[g], (int)std::min<int64_t>((nkb[g] + kcb - 1) / kcb, 1 << 30));
+    };
+    auto chip_cost = [&](int64_t kcb) {
+        double total = 0.0;
+        for (int g = 0; g < ngroups; ++g) total += (double)index(one.data(), g, kcb).items();
+        return std::ceil(total / cus) * (double)(kcb + 2);
+    };
+    auto xcd_load = [&](const int *ks, int64_t kcb) {
+        double load = 0.0;
+        for (int g = 0; g < ngroups; ++g) load += (double)index(ks, g, kcb).xcd_items();
+        return load;
+    };
+    const double xcd_cus = std::max(1.0, cus / 8.0), per_slab = precision == PRNU_PREC_FP32 ? 2.0 : 24.0;
+    auto xcd_cost = [&](const int *ks, int64_t kcb) {
+        return std::ceil(xcd_load(ks, kcb) / xcd_cus) * ((double)kcb + per_slab);
+    };
+    double cost = 0.0;
+    const int64_t kcb_one = search_kcb(tiles, nkb, ngroups, max_bytes, longest, chip_cost, &cost);
+    if (std::any_of(splits, splits + ngroups, [](int k) { return k > 1; })) {
+        const int64_t kcb = search_kcb(tiles, nkb, ngroups, max_bytes, kcb_one,
+                                       [&](int64_t k) { return xcd_cost(splits, k); }, &cost);
+        if (cost < xcd_cost(one.data(), kcb_one)) {
+            if (xcd_load(one.data(), kcb) <= xcd_cus) std::copy(one.begin(), one.end(), splits);
+            return kcb;
+        }
+        std::copy(one.begin(), one.end(), splits);
+    }
     return kcb_one;
 }
 
@@ -1233,10 +1264,10 @@ int store_gram_ncc(Context *c, Store *s, int first, int count, double *d_ncc, hi
         int64_t S = std::min<int64_t>(cfg.slabs, s->nkb);
         S = std::min<int64_t>(S, std::max<int64_t>(1, (int64_t(2) << 30) / (tile_bytes * tiles)));
         a.kcb = (s->nkb + S - 1) / S;
-        if (a.T * S <= device_cus(c->device)) a.ks = 1;  // (choose_slab)
+        if (a.T * ((S + 7) / 8) * 8 <= device_cus(c->device)) a.ks = 1;  // (choose_slab)
     } else {
         const int64_t nkb = s->nkb;
-        a.kcb = choose_slab(&a.T, &a.ks, &tiles, &nkb, 1, device_cus(c->device), size_t(2) << 30, 0);
+        a.kcb = choose_slab(&a.T, &a.ks, &tiles, &nkb, 1, s->format, device_cus(c->device), size_t(2) << 30, 0);
     }
     a.S = (int)((s->nkb + a.kcb - 1) / a.kcb);
     a.xcd_remap = cfg.xcd_remap;
@@ -1340,7 +1371,7 @@ int plan_layout(GramPlan *p, int64_t kcb) {
     int64_t v = 0, items = 0, part = 0, whole = 0;
     for (const PlanBlock &g : p->groups) {
         const int64_t k = std::min<int64_t>(kcb, g.store->nkb);
-        whole += g.items() * ((g.store->nkb + k - 1) / k);
+        whole += g.items() * (((g.store->nkb + k - 1) / k + 7) / 8 * 8);
     }
     const bool split = p->split && whole > p->cus;  // (choose_slab)
     for (size_t i = 0; i < p->groups.size(); ++i) {
@@ -1394,7 +1425,7 @@ int plan_layout(GramPlan *p, int64_t kcb) {
     return PRNU_OK;
 }
 
-// Default slab: the cheapest by the rounds model of choose_kcb.
+// Default slab: choose_slab's.
 int64_t plan_default_kcb(GramPlan *p) {
     std::vector<int> items, splits, tiles;
     std::vector<int64_t> nkb;
@@ -1404,8 +1435,8 @@ int64_t plan_default_kcb(GramPlan *p) {
         tiles.push_back(g.tiles());
         nkb.push_back(g.store->nkb);
     }
-    const int64_t kcb = choose_slab(items.data(), splits.data(), tiles.data(), nkb.data(), (int)items.size(), p->cus,
-                                    kPlanPartialCap, 0);
+    const int64_t kcb = choose_slab(items.data(), splits.data(), tiles.data(), nkb.data(), (int)items.size(),
+                                    p->format, p->cus, kPlanPartialCap, 0);
     p->split = std::any_of(splits.begin(), splits.end(), [](int k) { return k > 1; });
     return kcb;
 }

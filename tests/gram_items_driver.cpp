@@ -2,7 +2,8 @@
 // (rocket_amd/csrc/gram_items.hpp, compiled for the host), one line per id and
 // working wave: item, first slab, wave, first A and B pattern, the slabs of
 // the LDS quarters that hold them, the wave's slab, partial tile, offset in it.
-// Arguments: count ks S remap.  First line: items per slab, slab_split, ids.
+// Arguments: count ks S remap.  First line: items per slab, slab_split,
+// ids, items of the busiest XCD.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -17,7 +18,7 @@ int main(int argc, char **argv) {
     using namespace prnu;
     const int T = tri_items_per_slab(count);
     const ItemIndex index(T, ks, S);
-    std::printf("%d %d %lld\n", T, slab_split(count), (long long)index.ids(remap));
+    std::printf("%d %d %lld %lld\n", T, slab_split(count), (long long)index.ids(remap), (long long)index.xcd_items());
     for (int64_t id = 0; id < index.ids(remap); ++id) {
         int u, s;
         if (!index.at(id, remap, u, s)) continue;

@@ -132,3 +132,38 @@ def test_put_edges(fmt, count, n, first, offset):
             assert got[0][i] == pytest.approx(sx, rel=1e-9, abs=1e-9) and got[1][i] == pytest.approx(sxx, rel=1e-10)
             assert got[2][i] == r.abs().max().item()
         s.close()
+
+
+def busiest_xcd(T, ks, S):
+    """Items of the XCD with the most, ids dealt to 8 in turn (the split item's after the others')."""
+    whole, groups = (T - 1, -(-S // ks)) if ks > 1 else (T, 0)
+    return whole * -(-S // 8) + -(-groups // 8)
+
+
+@pytest.mark.parametrize("fmt,n", [("fp16", 786432), ("fp16", 2000000), ("split_bf16", 262144), ("fp8", 3145728),
+                                   ("fp32", 2000000)])
+@pytest.mark.parametrize("count,T,ks", [(300, 2, 2), (380, 2, 2), (120, 1, 4), (500, 3, 1)])
+def test_split_items_shorten_the_launch(fmt, n, count, T, ks):
+    """The slab of a plan: rounds of the busiest XCD's 32 CUs times the slab and
+    the cost of one (24 stages, 2 for FP32) are not above those of the slab that
+    items of one slab at a time would get."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    values = {"split_bf16": 32, "fp32": 32, "fp16": 64, "fp8": 128}[fmt]
+    blocks, extra = -(-n // values), 2 if fmt == "fp32" else 24
+    gram = csi.GramNCC(n // 2, 2)
+    store = csi.PatternStore(n, count, fmt)
+    plan = csi.GramPlan(gram, [(store, 0, count)])
+    info = plan.info()
+    plan.close()
+    store.close()
+    gram.close()
+    kcb = info["slab_values"] // values
+    S = -(-blocks // kcb)
+    split = info["work_items"] < T * S
+    assert info["work_items"] == (T * S if not split else (T - 1) * S + -(-S // ks))
+    steps = [16 + 8 * i for i in range(30)] + [256 + 32 * i for i in range(56)] + [2048 + 256 * i for i in range(600)]
+    one = min((k for k in steps if k <= blocks), key=lambda k: (-(-(T * -(-blocks // k)) // 256) * (k + 2), k))
+    cost = lambda T, ks, k: -(-busiest_xcd(T, ks, -(-blocks // k)) // 32) * (k + extra)  # noqa: E731
+    assert kcb <= one and cost(T, ks if split else 1, kcb) <= cost(T, 1, one)
+    if ks == 1:
+        assert kcb == one

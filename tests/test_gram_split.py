@@ -33,9 +33,9 @@ def driver(tmp_path_factory):
 @pytest.mark.parametrize("S", [1, 3, 8, 37, 64])
 @pytest.mark.parametrize("count", [1, 120, 128, 129, 300, 384, 600, 800, 1100, 1400])
 def test_every_block_and_slab_once(driver, count, S, remap):
-    T, split, _ = driver(count, 1, 1, False)[0]
+    T, split = driver(count, 1, 1, False)[0][:2]
     for ks in {1, split}:
-        _, rows = driver(count, ks, S, remap)
+        (_, _, _, xcd_items), rows = driver(count, ks, S, remap)
         ident, u, first, wave, a, b, kqa, kqb, kw, tile, off = rows.T
         assert (first + 0 < S).all() and (kqa == kw).all() and (kqb == kw).all()
         assert (kw[(u < T - 1) | (ks == 1)] == 0).all()        # only the last item takes several slabs
@@ -55,6 +55,7 @@ def test_every_block_and_slab_once(driver, count, S, remap):
         assert need <= set(got)
         assert all(i // 128 <= j // 128 for _, i, j in got)
         if remap:
+            assert np.bincount(np.unique(ident) & 7, minlength=8).max() == xcd_items
             per_xcd = np.bincount(np.unique(ident[u < T - (ks > 1)]) & 7, minlength=8)
             assert per_xcd.max() - per_xcd.min() <= T
             per_xcd = np.bincount(np.unique(ident[(u == T - 1) & (ks > 1)]) & 7, minlength=8)
@@ -63,7 +64,7 @@ def test_every_block_and_slab_once(driver, count, S, remap):
 
 @pytest.mark.parametrize("count,ks", [(1, 4), (128, 4), (129, 1), (300, 2), (600, 1), (800, 1), (1100, 4), (1300, 2)])
 def test_split_fills_the_last_item(driver, count, ks):
-    (T, split, _), rows = driver(count, ks, 4, False)
+    (T, split, _, _), rows = driver(count, ks, 4, False)
     assert split == ks
     last = rows[rows[:, 1] == T - 1]
     if ks > 1:  # its eight waves all work in a full group of slabs
