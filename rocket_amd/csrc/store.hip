@@ -80,28 +80,36 @@ struct StatPartS {
 // max|x| / 448, FP16 the power of two 2^(e - 15), max|x| < 2^e (the exponent
 // is clamped from below so that the multiplier of a tiny pattern stays a
 // finite float).
-// grid (ceil(n_padded / 1024), ceil(count / 8)), 256 threads.
+// ONE: eight consecutive pieces of 1024 values of one pattern instead, for
+// calls of few patterns, where most of a workgroup's slots would stand empty
+// (split-BF16, one pattern of 12 M values a call: 132 us with them, 70 so; four
+// of 3.1 M 69 and 62, five 70 and 71).  Same partials, same bytes.
+// grid (nchunk, ceil(count / 8)), ONE (ceil(nchunk / 8), count), 256 threads;
+// nchunk = ceil(n_padded / 1024).
 constexpr int kPutVals = 1024, kPutSlots = 8;
 
-template <int FMT>
+template <int FMT, bool ONE>
 __global__ __launch_bounds__(256) void store_put_kernel(const float *const *ptrs, int count, int64_t n, int64_t nkb,
-                                                        uint8_t *blocks, int cap_pad, int first, StatPartS *part,
-                                                        const float *absmax, float *scale) {
+                                                        uint8_t *blocks, int cap_pad, int first, int nchunk,
+                                                        StatPartS *part, const float *absmax, float *scale) {
     constexpr bool kStats = FMT == PRNU_PREC_SPLIT_BF16 || FMT == PRNU_PREC_FP32;
     constexpr int kVals = FMT == PRNU_PREC_FP8 ? kBlk8 : FMT == PRNU_PREC_FP16 ? kBlk16 : kBlk;
-    constexpr int kBlocks = kPutVals / kVals;                  // of the workgroup
+    constexpr int kBlocks = kPutVals / kVals;                  // of a piece
     constexpr int kRow = kPutSlots * kBlkBytes + 64;           // LDS bytes per block (+64: banks)
     __shared__ __attribute__((aligned(16))) uint8_t lds[kBlocks * kRow];
     __shared__ StatPartS wave_part[4][kPutSlots];
     const int t = threadIdx.x, lane = t & 63;
-    const int p0 = blockIdx.y * kPutSlots;
-    const int64_t k0 = (int64_t)blockIdx.x * kPutVals + 4 * t;
+    // entry p of the workgroup: its pattern, its piece, whether there is one
+    auto pattern = [&](int p) { return ONE ? (int)blockIdx.y : (int)blockIdx.y * kPutSlots + p; };
+    auto piece = [&](int p) { return ONE ? (int)blockIdx.x * kPutSlots + p : (int)blockIdx.x; };
+    auto there = [&](int p) { return ONE ? piece(p) < nchunk : pattern(p) < count; };
     float4 v[kPutSlots];
 #pragma unroll
     for (int p = 0; p < kPutSlots; ++p) {
         v[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (p0 + p < count) {
-            const float *x = ptrs[p0 + p];
+        if (there(p)) {
+            const float *x = ptrs[pattern(p)];
+            const int64_t k0 = (int64_t)piece(p) * kPutVals + 4 * t;
             if (k0 + 4 <= n && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
                 v[p] = *reinterpret_cast<const float4 *>(x + k0);
             } else {
@@ -133,15 +141,15 @@ __global__ __launch_bounds__(256) void store_put_kernel(const float *const *ptrs
         } else if constexpr (FMT == PRNU_PREC_FP32) {
             *reinterpret_cast<float4 *>(to + 4 * at) = v[p];
         } else if constexpr (FMT == PRNU_PREC_FP8) {
-            const float a = p0 + p < count ? absmax[first + p0 + p] : 0.f;
+            const float a = there(p) ? absmax[first + pattern(p)] : 0.f;
             const float inv = a > 0.f ? kE4M3Max / a : 1.0f;
             int w = 0;
             w = __builtin_amdgcn_cvt_pk_fp8_f32(e[0] * inv, e[1] * inv, w, false);
             w = __builtin_amdgcn_cvt_pk_fp8_f32(e[2] * inv, e[3] * inv, w, true);
             *reinterpret_cast<int *>(to + at) = w;
-            if (blockIdx.x == 0 && t == 0 && p0 + p < count) scale[first + p0 + p] = a > 0.f ? a / kE4M3Max : 1.0f;
+            if (piece(p) == 0 && t == 0 && there(p)) scale[first + pattern(p)] = a > 0.f ? a / kE4M3Max : 1.0f;
         } else {
-            const float a = p0 + p < count ? absmax[first + p0 + p] : 0.f;
+            const float a = there(p) ? absmax[first + pattern(p)] : 0.f;
             int ex = 0;
             (void)frexpf(a, &ex);  // a = m * 2^ex, m in [0.5, 1): a < 2^ex
             ex = a > 0.f ? max(-100, ex) : 15;
@@ -151,7 +159,7 @@ __global__ __launch_bounds__(256) void store_put_kernel(const float *const *ptrs
             for (int q = 0; q < 4; ++q) h[q] = __builtin_bit_cast(uint16_t, (_Float16)(e[q] * mult));
             *reinterpret_cast<uint2 *>(to + 2 * at) =
                 make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
-            if (blockIdx.x == 0 && t == 0 && p0 + p < count) scale[first + p0 + p] = ldexpf(1.0f, ex - 15);
+            if (piece(p) == 0 && t == 0 && there(p)) scale[first + pattern(p)] = ldexpf(1.0f, ex - 15);
         }
         if constexpr (kStats) {
             s[p] = 0.0;
@@ -166,9 +174,20 @@ __global__ __launch_bounds__(256) void store_put_kernel(const float *const *ptrs
             }
         }
     }
-    if constexpr (kStats) {
-        // 8 patterns x 64 lanes: three exchange steps leave each lane the sums of
-        // 8 lanes for one pattern (lane & 7, bits in exchange order), three more
+    __syncthreads();
+    // 64 threads per block: 8 entries x 8 chunks of 16 bytes
+    const int p = lane >> 3;
+#pragma unroll
+    for (int k = t >> 6; k < kBlocks; k += 4) {
+        const int64_t blk = (int64_t)piece(p) * kBlocks + k;
+        if (blk < nkb && there(p))
+            *reinterpret_cast<uint4 *>(blocks + ((size_t)blk * cap_pad + first + pattern(p)) * kBlkBytes +
+                                       (lane & 7) * 16) =
+                *reinterpret_cast<const uint4 *>(lds + k * kRow + lane * 16);
+    }
+    if constexpr (kStats) {  // while the stores leave
+        // 8 entries x 64 lanes: three exchange steps leave each lane the sums of
+        // 8 lanes for one entry (lane & 7, bits in exchange order), three more
         // the wave's
 #pragma unroll
         for (int half = kPutSlots / 2, off = 1; half > 0; half >>= 1, off <<= 1) {
@@ -192,25 +211,15 @@ __global__ __launch_bounds__(256) void store_put_kernel(const float *const *ptrs
             const int p = ((lane & 1) << 2) | (lane & 2) | ((lane >> 2) & 1);
             wave_part[t >> 6][p] = StatPartS{s[0], ss[0], am[0], 0.f};
         }
-    }
-    __syncthreads();
-    if (kStats && t < kPutSlots && p0 + t < count) {
-        StatPartS o;
-        o.s = (wave_part[0][t].s + wave_part[1][t].s) + (wave_part[2][t].s + wave_part[3][t].s);
-        o.ss = (wave_part[0][t].ss + wave_part[1][t].ss) + (wave_part[2][t].ss + wave_part[3][t].ss);
-        o.am = fmaxf(fmaxf(wave_part[0][t].am, wave_part[1][t].am), fmaxf(wave_part[2][t].am, wave_part[3][t].am));
-        o.pad = 0.f;
-        part[(int64_t)(p0 + t) * gridDim.x + blockIdx.x] = o;
-    }
-    // 64 threads per block: 8 slots x 8 chunks of 16 bytes
-    const int slot = lane >> 3;
-#pragma unroll
-    for (int k = t >> 6; k < kBlocks; k += 4) {
-        const int64_t blk = (int64_t)blockIdx.x * kBlocks + k;
-        if (blk < nkb && p0 + slot < count)
-            *reinterpret_cast<uint4 *>(blocks + ((size_t)blk * cap_pad + first + p0 + slot) * kBlkBytes +
-                                       (lane & 7) * 16) =
-                *reinterpret_cast<const uint4 *>(lds + k * kRow + lane * 16);
+        __syncthreads();
+        if (t < kPutSlots && there(t)) {
+            StatPartS o;
+            o.s = (wave_part[0][t].s + wave_part[1][t].s) + (wave_part[2][t].s + wave_part[3][t].s);
+            o.ss = (wave_part[0][t].ss + wave_part[1][t].ss) + (wave_part[2][t].ss + wave_part[3][t].ss);
+            o.am = fmaxf(fmaxf(wave_part[0][t].am, wave_part[1][t].am), fmaxf(wave_part[2][t].am, wave_part[3][t].am));
+            o.pad = 0.f;
+            part[(int64_t)pattern(t) * nchunk + piece(t)] = o;
+        }
     }
 }
 
@@ -1206,38 +1215,45 @@ void store_destroy(Store *s) {
     delete s;
 }
 
+// Calls of fewer patterns take the kernel's ONE form (figures there).
+constexpr int kPutOneBelow = 5;
+
+template <int FMT>
+int launch_put(Store *s, const float *const *d_ptrs, int count, int first, int nchunk, StatPartS *part,
+               hipStream_t st) {
+    const unsigned pieces = (unsigned)((nchunk + kPutSlots - 1) / kPutSlots);
+    if (count < kPutOneBelow)
+        hipLaunchKernelGGL((store_put_kernel<FMT, true>), dim3(pieces, (unsigned)count), dim3(256), 0, st, d_ptrs,
+                           count, s->n, s->nkb, s->blocks, s->cap_pad, first, nchunk, part, s->absmax, s->scale);
+    else
+        hipLaunchKernelGGL((store_put_kernel<FMT, false>),
+                           dim3((unsigned)nchunk, (unsigned)((count + kPutSlots - 1) / kPutSlots)), dim3(256), 0, st,
+                           d_ptrs, count, s->n, s->nkb, s->blocks, s->cap_pad, first, nchunk, part, s->absmax,
+                           s->scale);
+    PRNU_CHECK_LAUNCH();
+    return PRNU_OK;
+}
+
 int store_put(Store *s, const float *const *d_ptrs, int count, int first, hipStream_t st) {
     PRNU_REQUIRE(count >= 1 && first >= 0 && first + count <= s->capacity,
                  "store_put: slots [%d, %d) outside the capacity %d", first, first + count, s->capacity);
     PRNU_REQUIRE((count + 7) / 8 <= 65535, "store_put: at most 524280 patterns per call");
-    const dim3 grid((unsigned)((s->nkb * block_values(s->format) + kPutVals - 1) / kPutVals),
-                    (unsigned)((count + kPutSlots - 1) / kPutSlots));
+    const int nchunk = (int)((s->nkb * block_values(s->format) + kPutVals - 1) / kPutVals);
     if (s->format == PRNU_PREC_FP8 || s->format == PRNU_PREC_FP16) {
         // statistics (and max|x|, which sets the scale) first, then quantise
         PRNU_REQUIRE(count <= 65535, "store_put: at most 65535 %s patterns per call",
                      s->format == PRNU_PREC_FP8 ? "FP8" : "FP16");
         PRNU_TRY(launch_pattern_stats(d_ptrs, count, s->n, s->sum + first, s->sumsq + first, s->absmax + first,
                                       s->ws_part, st));
-        if (s->format == PRNU_PREC_FP8)
-            hipLaunchKernelGGL(store_put_kernel<PRNU_PREC_FP8>, grid, dim3(256), 0, st, d_ptrs, count, s->n, s->nkb,
-                               s->blocks, s->cap_pad, first, nullptr, s->absmax, s->scale);
-        else
-            hipLaunchKernelGGL(store_put_kernel<PRNU_PREC_FP16>, grid, dim3(256), 0, st, d_ptrs, count, s->n, s->nkb,
-                               s->blocks, s->cap_pad, first, nullptr, s->absmax, s->scale);
-        PRNU_CHECK_LAUNCH();
-        return PRNU_OK;
+        return s->format == PRNU_PREC_FP8 ? launch_put<PRNU_PREC_FP8>(s, d_ptrs, count, first, nchunk, nullptr, st)
+                                          : launch_put<PRNU_PREC_FP16>(s, d_ptrs, count, first, nchunk, nullptr, st);
     }
-    const unsigned gx = grid.x;
-    PRNU_TRY(s->ws_part.ensure(sizeof(StatPartS) * (size_t)gx * count));
+    PRNU_TRY(s->ws_part.ensure(sizeof(StatPartS) * (size_t)nchunk * count));
     StatPartS *part = static_cast<StatPartS *>(s->ws_part.ptr);
-    if (s->format == PRNU_PREC_SPLIT_BF16)
-        hipLaunchKernelGGL(store_put_kernel<PRNU_PREC_SPLIT_BF16>, grid, dim3(256), 0, st, d_ptrs, count, s->n,
-                           s->nkb, s->blocks, s->cap_pad, first, part, nullptr, nullptr);
-    else
-        hipLaunchKernelGGL(store_put_kernel<PRNU_PREC_FP32>, grid, dim3(256), 0, st, d_ptrs, count, s->n, s->nkb,
-                           s->blocks, s->cap_pad, first, part, nullptr, nullptr);
-    PRNU_CHECK_LAUNCH();
-    hipLaunchKernelGGL(store_stats_final_kernel, dim3(count), dim3(256), 0, st, part, (int)gx, count, first, s->sum,
+    PRNU_TRY(s->format == PRNU_PREC_SPLIT_BF16
+                 ? launch_put<PRNU_PREC_SPLIT_BF16>(s, d_ptrs, count, first, nchunk, part, st)
+                 : launch_put<PRNU_PREC_FP32>(s, d_ptrs, count, first, nchunk, part, st));
+    hipLaunchKernelGGL(store_stats_final_kernel, dim3(count), dim3(256), 0, st, part, nchunk, count, first, s->sum,
                        s->sumsq, s->absmax);
     PRNU_CHECK_LAUNCH();
     return PRNU_OK;

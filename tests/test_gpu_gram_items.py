@@ -106,12 +106,13 @@ def test_split_items(fmt, count, blocks, per_slab):
 
 @pytest.mark.parametrize("fmt", ["split_bf16", "fp32", "fp16", "fp8"])
 @pytest.mark.parametrize("count,n,first,offset", [(1, 6, 0, 0), (9, 1023, 2, 0), (8, 1024, 0, 0), (17, 1029, 3, 1),
-                                                  (5, 5000, 1, 3)])
+                                                  (5, 5000, 1, 3), (4, 8193, 0, 1), (6, 20000, 2, 0)])
 def test_put_edges(fmt, count, n, first, offset):
     """Inserts around the packing's 8 patterns and 1024 values, with pattern
     rows off 16-byte alignment: the stored statistics (FP64 sums of FP32
-    products: 1e-10), slots around the range untouched, and the same blocks as
-    one pattern put at a time (bytes equal)."""
+    products: 1e-10), slots around the range untouched, and the same blocks and
+    statistics as one pattern put at a time (bytes equal; up to four patterns a
+    call take eight pieces of one pattern to a workgroup)."""
     g = torch.Generator(device="cuda").manual_seed(n + count)
     rows = [torch.randn(n + offset, generator=g, device="cuda")[offset:] for _ in range(count)]
     stores = [csi.PatternStore(n, first + count + 2, fmt) for _ in range(2)]
@@ -125,6 +126,7 @@ def test_put_edges(fmt, count, n, first, offset):
         images.append(img.numpy())
     blocks = len(images[0]) - (first + count + 2) * 24   # the slots past and before `first` hold no statistics yet
     assert np.array_equal(images[0][:blocks], images[1][:blocks])
+    assert all(np.array_equal(a, b) for a, b in zip(*(s.stats(count, first) for s in stores)))
     for s in stores:
         got = s.stats(count, first)
         for i, r in enumerate(rows):
