@@ -1365,18 +1365,20 @@ int decode_batch(JpegDecoder *dec, const uint8_t *const *files, const int64_t *s
         PRNU_CHECK_HIP(hipMemsetAsync(d_coef, 0, (size_t)coef_blocks * 128, st));
         PRNU_CHECK_HIP(hipMemsetAsync(d_changed, 0, sizeof(int) * ((size_t)max_chunks + 2), st));
         const dim3 gch((unsigned)((nchunk + kLanes - 1) / kLanes));
-        // linking rounds until one changes nothing; after round r the first
-        // r + 1 chunks of every segment are exact, so rounds 0..max_chunks
-        // always suffice.  The host looks at the flag once per group of
-        // rounds; a round after the fixed point returns at once.
+        // linking rounds until one changes nothing; round r takes the exact
+        // entry of a segment's chunk r, so max_chunks rounds always suffice.
+        // The host looks at the flag once per group of rounds, and not after
+        // the last (files of one chunk a segment wait for nothing here); a
+        // round after the fixed point returns at once.
         constexpr int kRoundsPerCheck = 4;
-        for (int r = 0; r <= max_chunks;) {
-            const int r_end = std::min(max_chunks + 1, r + kRoundsPerCheck);
+        for (int r = 0; r < max_chunks;) {
+            const int r_end = std::min(max_chunks, r + kRoundsPerCheck);
             for (; r < r_end; ++r) {
                 hipLaunchKernelGGL(jpeg_chunk_round_kernel, gch, dim3(kLanes), 0, st, d_seg, d_cseg, nchunk, d_tab,
                                    d_lut, d_data, r, d_entry, d_exit[(r + 1) & 1], d_exit[r & 1], d_changed);
                 PRNU_CHECK_LAUNCH();
             }
+            if (r == max_chunks) break;
             int changed = 0;
             PRNU_CHECK_HIP(hipMemcpyAsync(&changed, d_changed + (r - 1), sizeof(int), hipMemcpyDeviceToHost, st));
             PRNU_CHECK_HIP(hipStreamSynchronize(st));
