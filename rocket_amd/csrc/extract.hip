@@ -692,8 +692,13 @@ __global__ __launch_bounds__(R::T) void wiener_rows_fwd_kernel(R pl, const float
         double s0 = 0.0, s1 = 0.0;
 #pragma unroll
         for (int k = 0; k < NW; k += 4) {
-            s0 += (sh[0][k] + sh[0][k + 1]) + (sh[0][k + 2] + sh[0][k + 3]);
-            s1 += (sh[1][k] + sh[1][k + 1]) + (sh[1][k + 2] + sh[1][k + 3]);
+            if constexpr (NW < 4) {
+                s0 = NW == 1 ? sh[0][0] : sh[0][0] + sh[0][NW - 1];
+                s1 = NW == 1 ? sh[1][0] : sh[1][0] + sh[1][NW - 1];
+            } else {
+                s0 += (sh[0][k] + sh[0][k + 1]) + (sh[0][k + 2] + sh[0][k + 3]);
+                s1 += (sh[1][k] + sh[1][k + 1]) + (sh[1][k + 2] + sh[1][k + 3]);
+            }
         }
         if (ZM_EVEN) {
             s0 *= 2.0 / (double)w;
