@@ -11,9 +11,9 @@
 // Why strips: a column pass over a transposed plane needs two transposes
 // around it (16 bytes per value read and written twice more; four frames of
 // 4000x3000: 160 us), and a column read straight from the plane takes 64 lines
-// per load.  The 160 KiB of LDS hold 8 columns of up to 2048 values, 4 of up
-// to 4096 or 2 of up to 8192, at 16 values per thread (ColsRt); the hot lengths
-// 1024 and 1536 have compile-time plans on one wave per column (ColsC).
+// per load.  A strip is 8 columns of up to 1023 values or 2 of up to 8192 (136
+// KiB of LDS), at 16 values per thread (ColsRt); the hot lengths 1024 and 1536
+// have compile-time plans on one wave per column, 8 columns a strip (ColsC).
 #pragma once
 
 #include "fft_device.hpp"
@@ -56,17 +56,23 @@ size_t cols_lds(const P &pl) {
     return sizeof(float2) * (size_t)P::COLS * pl.stride();
 }
 
-// Calls f(plan) with the plan of columns of d.n values.  (At 1536 rows the
-// run-time plan on two waves per column measured 333 and 356 us for the
-// chain's two passes over 32 frames of 2048x1536, the compile-time plan 263 and
-// 291; strips of 4 columns, two workgroups per CU, 277 and 328.)
+// Calls f(plan) with the plan of columns of d.n values.
+// Strips of 2 columns where a column takes two waves or more: up to four
+// workgroups a CU, which stage and transform in turn, and enough of them for a
+// narrow frame (wide strips of 8 columns up to 2048 values and 4 up to 4096
+// against these, the chain: one frame of 100x2000 102 -> 86 us, 4 of 4000x3000
+// 895 -> 842, 32 of 2000x1500 1623 -> 1528; 8 of 4096x4096 2316 -> 2355).  One
+// wave a column: 8 columns (8 frames of 1000x2000 267 us, 289 by 2).  (At 1536
+// rows the run-time plan on two waves per column, strips of 8, measured 333 and
+// 356 us for the chain's two passes over 32 frames of 2048x1536, the
+// compile-time plan 263 and 291, by 4 columns 277 and 328.)
 template <class F>
 auto with_cols_plan(const FftDesc &d, F f) {
     if (d.n == 1024) return f(ColsC<1024>{d.tw});
     if (d.n == 1536) return f(ColsC<1536>{d.tw});
     if (d.n < 1024) return f(ColsRt<64, 8>{d});
-    if (d.n <= 2048) return f(ColsRt<128, 8>{d});
-    if (d.n <= 4096) return f(ColsRt<256, 4>{d});
+    if (d.n <= 2048) return f(ColsRt<128, 2>{d});
+    if (d.n <= 4096) return f(ColsRt<256, 2>{d});
     return f(ColsRt<512, 2>{d});
 }
 
